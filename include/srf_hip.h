@@ -175,9 +175,9 @@ int srf_image_from_kernel_layout(const float *src_kernel, float *dst_xyz, int32_
  * during create / rebuild only, which synchronise `stream`.  An event list may
  * bin into at most 2^31 - 1 segments, and a plan's grid may have at most 32767
  * cells along x and along y (SRF_ERR_UNSUPPORTED beyond: split the list into
- * several plans, as OSEM subsets are).  The memory comes from a stream-ordered pool per
- * device that keeps up to 16 GiB of freed plan memory for the next plans
- * (hipMalloc where a device has no pools; srf_plan_pool_trim releases it);
+ * several plans, as OSEM subsets are).  The memory comes from a pool per
+ * device that keeps up to 16 GiB of freed plan memory for the next plans, in
+ * order between streams by events (srf_plan_pool_trim releases it);
  * srf_plan_destroy first waits for the device, as hipFree does. */
 typedef struct srf_plan srf_plan;
 
@@ -221,7 +221,7 @@ int srf_plan_rebuild(srf_plan *plan, const float *lors, int64_t n, int64_t lor_s
                      const srf_plan_opts_t *opts, void *stream);
 int srf_plan_destroy(srf_plan *plan);
 /* Returns the current device's pooled plan memory above keep_bytes to the
- * system (hipMemPoolTrimTo after draining the device), so that other HIP users
+ * system (hipFree after draining the device), so that other HIP users
  * of the process (torch's caching allocator) can have it; 0 releases all
  * memory no live plan holds.  No reference counterpart (the plan pool is this
  * library's). */

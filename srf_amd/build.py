@@ -20,7 +20,8 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libsrf_hip.so")
 
-SOURCES = ["srf_project.hip", "srf_elementwise.hip", "srf_tiled.hip", "srf_sss.hip", "srf_cnn.hip", "srf_geometry.hip"]
+SOURCES = ["srf_project.hip", "srf_elementwise.hip", "srf_tiled.hip", "srf_sss.hip", "srf_cnn.hip", "srf_geometry.hip",
+           "srf_pool.hip"]
 
 
 def hipcc():

@@ -19,6 +19,13 @@ inline int launch_status()
 // captured into a HIP graph and replayed.
 int fill_f32(float *dst, float v, int64_t n, hipStream_t s);
 
+// Device memory for plans and scratch (srf_pool.hip).  pool_get: at least `bytes`
+// on the current device, for use in stream order on s (nullptr: none left).
+// pool_put: given back once the work queued on s so far is done (idle: nothing
+// uses it any more).  Not for a stream that is being captured.
+void *pool_get(size_t bytes, hipStream_t s);
+void pool_put(void *p, hipStream_t s, bool idle = false);
+
 struct LaunchGeom;
 // Validates a grid (and TOF parameters) and derives the per-launch constants.
 int make_geom(const srf_grid_t &g, const srf_tof_t *tof, LaunchGeom &G);

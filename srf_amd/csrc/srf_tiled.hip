@@ -1380,7 +1380,6 @@ template <class T>
 struct DevBuf {
     T *p = nullptr;
     size_t cap = 0;
-    bool pooled = false;   // from the plan pool (else hipMalloc)
 };
 
 struct srf_plan {
@@ -1392,10 +1391,12 @@ struct srf_plan {
     bool valid;   // the last build succeeded: item and tile tables match G / T
     DevBuf<SegRec> recs;
     DevBuf<int> rec_ev;
-    DevBuf<Item> items;
-    DevBuf<int> tile_items;
-    DevBuf<int> order;      // projector's launch order of the items: estimated work, largest first
-    DevBuf<int> order_bp;   // backprojector's: 8 bands of tile layers, one per XCD
+    // the item tables, one upload: pointers into `tables`
+    DevBuf<char> tables;
+    Item *items;
+    int *tile_items;
+    int *order;      // projector's launch order of the items: estimated work, largest first
+    int *order_bp;   // backprojector's: 8 bands of tile layers, one per XCD
     // one-shot timing events around the next tiled kernel (srf_plan_time_next)
     hipEvent_t ev_before = nullptr, ev_after = nullptr;
     DevBuf<int> ev_off;
@@ -1429,52 +1430,14 @@ int dmalloc(T **p, size_t count, size_t &total)
     return SRF_OK;
 }
 
-// Plan memory comes from one stream-ordered pool per device that keeps up to
-// POOL_KEEP bytes of freed memory for reuse.  Many plans built and destroyed
-// in a row (one per OSEM subset of many scans, or chunk after chunk) then
-// reuse pool memory instead of calling hipMalloc / hipFree, which map and
-// unmap memory and wait for the device each time.
-constexpr uint64_t POOL_KEEP = 16ull << 30;
-constexpr int POOL_DEVICES = 64;
-std::mutex pool_mu;
-hipMemPool_t pools[POOL_DEVICES];
-bool pool_failed[POOL_DEVICES];
-
-hipMemPool_t plan_pool()
-{
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= POOL_DEVICES) return nullptr;
-    std::lock_guard<std::mutex> lock(pool_mu);
-    if (!pools[dev] && !pool_failed[dev]) {
-        hipMemPoolProps props = {};
-        props.allocType = hipMemAllocationTypePinned;
-        props.handleTypes = hipMemHandleTypeNone;
-        props.location.type = hipMemLocationTypeDevice;
-        props.location.id = dev;
-        hipMemPool_t pool = nullptr;
-        if (hipMemPoolCreate(&pool, &props) != hipSuccess) {
-            (void)hipGetLastError();
-            pool_failed[dev] = true;
-            return nullptr;
-        }
-        uint64_t keep = POOL_KEEP;
-        (void)hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep);
-        pools[dev] = pool;
-    }
-    return pools[dev];
-}
-
-// Freed in stream order on s: work already queued on s may still read it.
+// Given back to the pool (srf_pool.hip): `idle` once nothing uses the buffer any
+// more, else in stream order on s.
 template <class T>
-void dfree(DevBuf<T> &b, hipStream_t s)
+void dfree(DevBuf<T> &b, hipStream_t s, bool idle = false)
 {
-    if (b.p) {
-        if (b.pooled) (void)hipFreeAsync(b.p, s);
-        else (void)hipFree(b.p);
-    }
+    pool_put(b.p, s, idle);
     b.p = nullptr;
     b.cap = 0;
-    b.pooled = false;
 }
 
 // At least `count` elements (1 if count is 0), reallocated only to grow.  A
@@ -1491,35 +1454,29 @@ int ensure(DevBuf<T> &b, size_t count, hipStream_t s)
         // read it, so drain the device before it goes back to the pool
         count += count / 4;
         (void)hipDeviceSynchronize();
-        dfree(b, s);
+        dfree(b, s, true);
     }
-    // a device without memory pools falls back to hipMalloc
-    hipMemPool_t pool = plan_pool();
-    const hipError_t e = pool ? hipMallocFromPoolAsync((void **)&b.p, count * sizeof(T), pool, s)
-                              : hipMalloc((void **)&b.p, count * sizeof(T));
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        b.p = nullptr;
-        return SRF_ERR_LAUNCH;
-    }
+    b.p = static_cast<T *>(pool_get(count * sizeof(T), s));
+    if (!b.p) return SRF_ERR_LAUNCH;
     b.cap = count;
-    b.pooled = pool != nullptr;
     return SRF_OK;
 }
 
-void free_scratch(srf_plan *P, hipStream_t s)
+// (after the stream has been synchronised)
+void free_scratch(srf_plan *P)
 {
-    dfree(P->ev_cnt, s);
-    dfree(P->key_count, s);
-    dfree(P->scan_tmp, s);
-    dfree(P->sort_tmp, s);
-    dfree(P->sk, s);
-    dfree(P->sk2, s);
-    dfree(P->idx, s);
-    dfree(P->idx2, s);
-    dfree(P->wpair, s);
-    dfree(P->recs2, s);
-    dfree(P->slot_ev, s);
+    const hipStream_t s = nullptr;
+    dfree(P->ev_cnt, s, true);
+    dfree(P->key_count, s, true);
+    dfree(P->scan_tmp, s, true);
+    dfree(P->sort_tmp, s, true);
+    dfree(P->sk, s, true);
+    dfree(P->sk2, s, true);
+    dfree(P->idx, s, true);
+    dfree(P->idx2, s, true);
+    dfree(P->wpair, s, true);
+    dfree(P->recs2, s, true);
+    dfree(P->slot_ev, s, true);
 }
 
 // Destroy: the plan may have been used on any stream, so the device is
@@ -1529,25 +1486,20 @@ void plan_free(srf_plan *P)
     if (!P) return;
     (void)hipDeviceSynchronize();
     const hipStream_t s = nullptr;
-    dfree(P->recs, s);
-    dfree(P->rec_ev, s);
-    dfree(P->items, s);
-    dfree(P->tile_items, s);
-    dfree(P->order, s);
-    dfree(P->order_bp, s);
-    dfree(P->ev_off, s);
-    dfree(P->ev_flag, s);
-    dfree(P->partial, s);
-    dfree(P->tile_buf, s);
-    free_scratch(P, s);
+    dfree(P->recs, s, true);
+    dfree(P->rec_ev, s, true);
+    dfree(P->tables, s, true);
+    dfree(P->ev_off, s, true);
+    dfree(P->ev_flag, s, true);
+    dfree(P->partial, s, true);
+    dfree(P->tile_buf, s, true);
+    free_scratch(P);
     delete P;
 }
 
 size_t plan_bytes(const srf_plan *P)
 {
-    return P->recs.cap * sizeof(SegRec) + P->rec_ev.cap * sizeof(int) + P->items.cap * sizeof(Item) +
-           P->tile_items.cap * sizeof(int) + P->order.cap * sizeof(int) +
-           P->order_bp.cap * sizeof(int) + P->ev_off.cap * sizeof(int) +
+    return P->recs.cap * sizeof(SegRec) + P->rec_ev.cap * sizeof(int) + P->tables.cap + P->ev_off.cap * sizeof(int) +
            P->ev_flag.cap + P->partial.cap * sizeof(float) + P->tile_buf.cap * sizeof(float);
 }
 
@@ -1638,8 +1590,7 @@ int plan_build(srf_plan *P, const float *lors, int64_t n, int64_t lor_stride, co
     PB_TRY(ensure(P->key_count, (size_t)T.nkeys, s));
     hipLaunchKernelGGL(k_fill_u32, dim3((T.nkeys + 255) / 256), dim3(256), 0, s, P->key_count.p, 0u,
                        (int64_t)T.nkeys);
-    hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((n + 1 + 255) / 256)), dim3(256), 0, s,
-                       (unsigned *)P->ev_cnt.p, 0u, n + 1);
+    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(256), 0, s, (unsigned *)P->ev_cnt.p + n, 0u, (int64_t)1);
     const unsigned nb = (unsigned)((n + BIN_THREADS - 1) / BIN_THREADS);
     const size_t shm = (size_t)T.nkeys * sizeof(unsigned);
     if (n > 0) {
@@ -1657,52 +1608,19 @@ int plan_build(srf_plan *P, const float *lors, int64_t n, int64_t lor_stride, co
     PB_TRY(ensure(P->scan_tmp, tmp_bytes, s));
     PB_HIP(hipcub::DeviceScan::ExclusiveSum(P->scan_tmp.p, tmp_bytes, P->ev_cnt.p, P->ev_off.p, (int)(n + 1), s));
     std::vector<unsigned> kc((size_t)T.nkeys);
-    int total = 0;
     PB_HIP(hipMemcpyAsync(kc.data(), P->key_count.p, kc.size() * sizeof(unsigned), hipMemcpyDeviceToHost, s));
-    PB_HIP(hipMemcpyAsync(&total, P->ev_off.p + n, sizeof(int), hipMemcpyDeviceToHost, s));
     PB_HIP(hipStreamSynchronize(s));
     // segment slots are 32-bit: a list with more than 2^31 - 1 segments (the
     // 32-bit prefix sum above would have wrapped) is refused
     uint64_t kc_sum = 0;
     for (unsigned c : kc) kc_sum += c;
     if (kc_sum > (uint64_t)INT_MAX) return SRF_ERR_UNSUPPORTED;
-    const int64_t nseg = total;
-    // work items from the key counts (keys are tile-major, so a tile's items are contiguous)
-    std::vector<Item> items;
-    std::vector<int> order, order_bp;
-    std::vector<int> tile_items((size_t)T.ntiles + 1, 0);
-    unsigned acc = 0;
-    for (int k = 0; k < T.nkeys; ++k) {
-        const int tile = k / NCLASS;
-        if (k % NCLASS == 0) tile_items[tile] = (int)items.size();
-        for (unsigned st = 0; st < kc[k]; st += item_max) {
-            items.push_back(Item{(int)(acc + st), (int)std::min<unsigned>(item_max, kc[k] - st), tile, k % NCLASS,
-                                 0.0f, 0.0f, {0.0f, 0.0f}});
-        }
-        acc += kc[k];
-    }
-    tile_items[T.ntiles] = (int)items.size();
-    if ((int64_t)acc != nseg) return SRF_ERR_LAUNCH;
-    const int nitems = (int)items.size();
+    const int64_t nseg = (int64_t)kc_sum;
     PB_TRY(ensure(P->recs, (size_t)nseg, s));
     PB_TRY(ensure(P->rec_ev, (size_t)nseg, s));
     PB_TRY(ensure(P->partial, (size_t)nseg, s));
-    PB_TRY(ensure(P->items, items.size(), s));
-    PB_TRY(ensure(P->tile_items, tile_items.size(), s));
-    PB_TRY(ensure(P->order, items.size(), s));
-    PB_TRY(ensure(P->order_bp, items.size(), s));
-    PB_TRY(ensure(P->tile_buf, (size_t)std::max(1, nitems) * TVOX, s));
-    if (!items.empty())
-        PB_HIP(hipMemcpyAsync(P->items.p, items.data(), items.size() * sizeof(Item), hipMemcpyHostToDevice, s));
-    PB_HIP(hipMemcpyAsync(P->tile_items.p, tile_items.data(), tile_items.size() * sizeof(int),
-                           hipMemcpyHostToDevice, s));
-    order = launch_order_largest_first(items);
-    order_bp = launch_order_by_xcd(items);
-    if (!order.empty()) {
-        PB_HIP(hipMemcpyAsync(P->order.p, order.data(), order.size() * sizeof(int), hipMemcpyHostToDevice, s));
-        PB_HIP(hipMemcpyAsync(P->order_bp.p, order_bp.data(), order_bp.size() * sizeof(int),
-                               hipMemcpyHostToDevice, s));
-    }
+    // the records are built and sorted on the device while the host lays out the
+    // work items below (the items come from the key counts alone)
     if (n > 0) {
         PB_TRY(ensure(P->sk, (size_t)nseg, s));
         PB_TRY(ensure(P->sk2, (size_t)nseg, s));
@@ -1743,10 +1661,44 @@ int plan_build(srf_plan *P, const float *lors, int64_t n, int64_t lor_stride, co
             std::swap(P->recs, P->recs2);
         }
     }
-    if (nitems > 0)
-        hipLaunchKernelGGL(k_item_wmax, dim3((unsigned)nitems), dim3(256), 0, s, P->wpair.p, P->items.p);
-    PB_HIP(hipGetLastError());
-    PB_HIP(hipStreamSynchronize(s));
+    // work items from the key counts (keys are tile-major, so a tile's items are contiguous)
+    std::vector<Item> items;
+    std::vector<int> tile_items((size_t)T.ntiles + 1, 0);
+    unsigned acc = 0;
+    for (int k = 0; k < T.nkeys; ++k) {
+        const int tile = k / NCLASS;
+        if (k % NCLASS == 0) tile_items[tile] = (int)items.size();
+        for (unsigned st = 0; st < kc[k]; st += item_max) {
+            items.push_back(Item{(int)(acc + st), (int)std::min<unsigned>(item_max, kc[k] - st), tile, k % NCLASS,
+                                 0.0f, 0.0f, {0.0f, 0.0f}});
+        }
+        acc += kc[k];
+    }
+    tile_items[T.ntiles] = (int)items.size();
+    const int nitems = (int)items.size();
+    PB_TRY(ensure(P->tile_buf, (size_t)std::max(1, nitems) * TVOX, s));
+    {
+        const std::vector<int> order = launch_order_largest_first(items), order_bp = launch_order_by_xcd(items);
+        const size_t b_items = items.size() * sizeof(Item), b_tiles = tile_items.size() * sizeof(int),
+                     b_order = items.size() * sizeof(int);
+        std::vector<char> h(b_items + 2 * b_order + b_tiles);
+        if (nitems > 0) {
+            memcpy(h.data(), items.data(), b_items);
+            memcpy(h.data() + b_items, order.data(), b_order);
+            memcpy(h.data() + b_items + b_order, order_bp.data(), b_order);
+        }
+        memcpy(h.data() + b_items + 2 * b_order, tile_items.data(), b_tiles);
+        PB_TRY(ensure(P->tables, h.size(), s));
+        P->items = reinterpret_cast<Item *>(P->tables.p);
+        P->order = reinterpret_cast<int *>(P->tables.p + b_items);
+        P->order_bp = reinterpret_cast<int *>(P->tables.p + b_items + b_order);
+        P->tile_items = reinterpret_cast<int *>(P->tables.p + b_items + 2 * b_order);
+        PB_HIP(hipMemcpyAsync(P->tables.p, h.data(), h.size(), hipMemcpyHostToDevice, s));
+        if (nitems > 0)
+            hipLaunchKernelGGL(k_item_wmax, dim3((unsigned)nitems), dim3(256), 0, s, P->wpair.p, P->items);
+        PB_HIP(hipGetLastError());
+        PB_HIP(hipStreamSynchronize(s));
+    }
     P->G = G;
     P->T = T;
     P->tof = use_tof;
@@ -1783,7 +1735,7 @@ int srf_plan_create_ex(const float *lors, int64_t n, int64_t lor_stride, const f
         plan_free(P);
         return rc;
     }
-    free_scratch(P, (hipStream_t)stream);
+    free_scratch(P);
     *out = P;
     return SRF_OK;
 }
@@ -1811,27 +1763,6 @@ int srf_plan_rebuild(srf_plan *plan, const float *lors, int64_t n, int64_t lor_s
 int srf_plan_destroy(srf_plan *plan)
 {
     plan_free(plan);
-    return SRF_OK;
-}
-
-int srf_plan_pool_trim(size_t keep_bytes)
-{
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= POOL_DEVICES) {
-        (void)hipGetLastError();
-        return SRF_ERR_LAUNCH;
-    }
-    hipMemPool_t pool;
-    {
-        std::lock_guard<std::mutex> lock(pool_mu);
-        pool = pools[dev];
-    }
-    if (!pool) return SRF_OK;   // no plan was built on this device
-    // memory freed in stream order becomes releasable once that work is done
-    if (hipDeviceSynchronize() != hipSuccess || hipMemPoolTrimTo(pool, keep_bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        return SRF_ERR_LAUNCH;
-    }
     return SRF_OK;
 }
 
@@ -1923,7 +1854,7 @@ int srf_plan_project(srf_plan *P, const float *image, float *out, void *stream)
     hipStream_t s = (hipStream_t)stream;
     mark_before(P, s);
     if (P->nitems > 0)
-        PLAN_DISPATCH(k_fp_tiled, <<<P->nitems, TILE_THREADS, 0, s>>>(P->recs.p, P->items.p, P->order.p, image, P->G, P->T,
+        PLAN_DISPATCH(k_fp_tiled, <<<P->nitems, TILE_THREADS, 0, s>>>(P->recs.p, P->items, P->order, image, P->G, P->T,
                                                                        P->partial.p));
     mark_after(P, s);
     hipLaunchKernelGGL(k_seg_reduce, dim3((unsigned)((P->n + 255) / 256)), dim3(256), 0, s, P->partial.p, P->ev_off.p,
@@ -1941,7 +1872,7 @@ int srf_plan_project_ratio(srf_plan *P, const float *image, const float *y, srf_
     hipStream_t s = (hipStream_t)stream;
     mark_before(P, s);
     if (P->nitems > 0)
-        PLAN_DISPATCH(k_fp_tiled, <<<P->nitems, TILE_THREADS, 0, s>>>(P->recs.p, P->items.p, P->order.p, image, P->G, P->T,
+        PLAN_DISPATCH(k_fp_tiled, <<<P->nitems, TILE_THREADS, 0, s>>>(P->recs.p, P->items, P->order, image, P->G, P->T,
                                                                        P->partial.p));
     mark_after(P, s);
     hipLaunchKernelGGL(k_seg_reduce, dim3((unsigned)((P->n + 255) / 256)), dim3(256), 0, s, P->partial.p, P->ev_off.p,
@@ -1967,12 +1898,12 @@ static int plan_bp(srf_plan *P, const float *values, const float *y, const float
         return launch_status();
     }
     mark_before(P, s);
-    PLAN_DISPATCH(k_bp_tiled, <<<P->nitems, TILE_THREADS, 0, s>>>(P->recs.p, P->items.p, P->order_bp.p, values, y, p,
+    PLAN_DISPATCH(k_bp_tiled, <<<P->nitems, TILE_THREADS, 0, s>>>(P->recs.p, P->items, P->order_bp, values, y, p,
                                                                    kind, eps, (int)(mode == SRF_BP_ADJOINT), P->G, P->T,
                                                                    P->rec_ev.p, P->tile_buf.p));
     mark_after(P, s);
     dim3 grid((TVOX + 255) / 256, (unsigned)P->T.ntiles);
-    hipLaunchKernelGGL(k_tile_reduce, grid, dim3(256), 0, s, P->tile_buf.p, P->tile_items.p, P->G, P->T, accumulate,
+    hipLaunchKernelGGL(k_tile_reduce, grid, dim3(256), 0, s, P->tile_buf.p, P->tile_items, P->G, P->T, accumulate,
                        image);
     return launch_status();
 }
@@ -1989,7 +1920,7 @@ int srf_plan_digest(srf_plan *P, srf_bp_mode_t mode, uint64_t *hash, int32_t *co
     hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((P->n + 255) / 256)), dim3(256), 0, s, (unsigned *)count, 0u,
                        P->n);
     if (P->nitems > 0)
-        PLAN_DISPATCH(k_digest_tiled, <<<P->nitems, TILE_THREADS, 0, s>>>(P->recs.p, P->rec_ev.p, P->items.p,
+        PLAN_DISPATCH(k_digest_tiled, <<<P->nitems, TILE_THREADS, 0, s>>>(P->recs.p, P->rec_ev.p, P->items,
                                                                            (int)(mode == SRF_BP_ADJOINT), P->G,
                                                                            P->T, (unsigned long long *)hash, count));
     return launch_status();
@@ -2014,12 +1945,12 @@ int srf_plan_backproject_update(srf_plan *P, const float *values, float *x, cons
         return launch_status();
     }
     mark_before(P, s);
-    PLAN_DISPATCH(k_bp_tiled, <<<P->nitems, TILE_THREADS, 0, s>>>(P->recs.p, P->items.p, P->order_bp.p, values,
+    PLAN_DISPATCH(k_bp_tiled, <<<P->nitems, TILE_THREADS, 0, s>>>(P->recs.p, P->items, P->order_bp, values,
                                                                    nullptr, nullptr, 0, 0.0f, 0, P->G, P->T,
                                                                    P->rec_ev.p, P->tile_buf.p));
     mark_after(P, s);
     dim3 grid((TVOX + 255) / 256, (unsigned)P->T.ntiles);
-    hipLaunchKernelGGL(k_tile_update, grid, dim3(256), 0, s, P->tile_buf.p, P->tile_items.p, P->G, P->T, emap,
+    hipLaunchKernelGGL(k_tile_update, grid, dim3(256), 0, s, P->tile_buf.p, P->tile_items, P->G, P->T, emap,
                        zero_guard, x);
     return launch_status();
 }
@@ -2115,9 +2046,9 @@ int srf_batch_create(srf_plan *const *plans, const srf_batch_scan_t *scans, int3
         d.G = P->G;
         d.T = P->T;
         d.recs = P->recs.p;
-        d.items = P->items.p;
+        d.items = P->items;
         d.rec_ev = P->rec_ev.p;
-        d.tile_items = P->tile_items.p;
+        d.tile_items = P->tile_items;
         d.ev_off = P->ev_off.p;
         d.ev_flag = P->ev_flag.p;
         d.partial = P->partial.p;
@@ -2131,7 +2062,7 @@ int srf_batch_create(srf_plan *const *plans, const srf_batch_scan_t *scans, int3
         tile_base[(size_t)i + 1] = tile_base[(size_t)i] + P->T.ntiles;
         if (P->nitems > 0) {
             std::vector<Item> items((size_t)P->nitems);
-            SRF_HIP(hipMemcpyAsync(items.data(), P->items.p, items.size() * sizeof(Item), hipMemcpyDeviceToHost, s));
+            SRF_HIP(hipMemcpyAsync(items.data(), P->items, items.size() * sizeof(Item), hipMemcpyDeviceToHost, s));
             SRF_HIP(hipStreamSynchronize(s));
             for (int k = 0; k < P->nitems; ++k) {
                 work.push_back(Work{i, k});

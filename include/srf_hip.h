@@ -5,8 +5,9 @@
  *  - All pointers are device pointers (HBM) unless the comment says otherwise.
  *    The caller owns every buffer; the library allocates device memory only in
  *    srf_plan_create[_ex], srf_plan_rebuild and srf_batch_create (freed by the
- *    matching *_destroy) and transient scratch in srf_sinogram_lors and
- *    srf_event_order.
+ *    matching *_destroy) and transient scratch in srf_sinogram_lors,
+ *    srf_event_order and, for long lists outside graph capture, srf_project
+ *    (which runs without it where it is not to be had).
  *  - LORs are AoS rows of `lor_stride` floats [x1,y1,z1,x2,y2,z2,(tof,...)] in
  *    mm, exactly Lors.data of srfnef/data/lors.py:12-22 (stride 6 or 7).
  *  - TOF values are read from `tof_values[e * tof_stride]`; pass

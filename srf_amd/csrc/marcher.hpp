@@ -19,8 +19,9 @@
 //                 (conservative; the exact per-slab tests still decide)
 //   fp_cut_range  the projector's segment cuts (siddon.cu.cc:56-57,203-204;
 //                 siddon_tof.cu.cc:67-74,228-235) as an exact slab interval
-//   march_slabs   the slab loop: carried boundary values, flattened branch tree,
-//                 up to three predicated terms per slab handed to a sink
+//   slab_cells, slab_fractions   one slab: cells, crossings, term fractions (the
+//                 flattened branch tree); slab_eval: both
+//   march_slabs   the slab loop: carried boundary values, every slab handed to a sink
 //   march_event   all of the above for one event (one-event-per-lane kernels)
 #pragma once
 #include <hip/hip_runtime.h>
@@ -57,6 +58,44 @@ __device__ __forceinline__ uint64_t mix64(uint64_t z)
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
     z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
     return z ^ (z >> 31);
+}
+
+// v_cvt_flr_i32_f32: floor and convert in one VALU op (NaN -> 0, saturating,
+// as v_floor_f32 + v_cvt_i32_f32).
+__device__ __forceinline__ int cvt_flr(float v)
+{
+    int r;
+    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(v));
+    return r;
+}
+
+// med3(x, lo, hi) = min(max(x, lo), hi) for lo <= hi, one v_med3_i32 (the
+// compiler emits it only for constant bounds), and a * b + c with a and b taken
+// as signed 24-bit integers (v_mad_i32_i24: the clamped cell index is -1 on
+// the low-edge halo of a tile at the image origin, which the unsigned form
+// would read as 2^24 - 1).  Plain ALU instructions, no memory access.
+__device__ __forceinline__ int med3_i32(int x, int lo, int hi)
+{
+    int r;
+    asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "v"(lo), "v"(hi));
+    return r;
+}
+__device__ __forceinline__ int mad_i24(int a, int b, int c)
+{
+    int r;
+    asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
+// Minimum / maximum of two non-negative finite floats as integer operations on
+// their bit patterns (which order the same way): no NaN canonicalisation.
+__device__ __forceinline__ float min_nonneg(float a, float b)
+{
+    return __uint_as_float(min(__float_as_uint(a), __float_as_uint(b)));
+}
+__device__ __forceinline__ float max_nonneg(float a, float b)
+{
+    return __uint_as_float(max(__float_as_uint(a), __float_as_uint(b)));
 }
 
 // Branch-independent part of one event.
@@ -237,97 +276,189 @@ __device__ __forceinline__ void fp_cut_range(const Branch &B, int lo, int hi, in
     if (b < a) b = a;
 }
 
-// TOF Gaussian parameters of one branch: d(ip) = ((pc - p1) * inv_pd - ratio1) * L
-struct TofLine {
-    float inv_pd, ratio1, L;
+// TOF Gaussian of siddon_tof.cu.cc:55-59 as a linear function of the slab's
+// lower boundary pp1 = ip - np2 (exact in float):
+//   pc = ((ip - np/2) + 0.5) * pd_tof = (pp1 + off) * pd_tof, off = np2 - np/2 + 0.5
+//   d  = ((pc - p1) / (p2 - p1) - ratio1) * L
+//   exp(-d^2 / (2 tse)) = exp2(-(d * sqrt(log2(e) / (2 tse)))^2)
+// Coefficients in double, rounded once.
+template <bool TOF>
+__device__ __forceinline__ void tof_coeffs_d(const Branch &B, const RaySetup &r, const LaunchGeom &G, double &tA,
+                                             double &tB)
+{
+    tA = tB = 0.0;
+    if (!TOF) return;
+    const double off = (double)B.np2 - (double)(B.np / 2) + 0.5;
+    const double s = sqrt(0.5 * 1.4426950408889634 / (double)G.tse);
+    const double k = (double)r.L / ((double)B.p2 - (double)B.p1);
+    tA = (double)B.pd_tof * k * s;
+    tB = ((off * (double)B.pd_tof - (double)B.p1) * k - (double)r.ratio1 * (double)r.L) * s;
+}
+
+template <bool TOF>
+__device__ __forceinline__ void tof_coeffs(const Branch &B, const RaySetup &r, const LaunchGeom &G, float &tA,
+                                           float &tB)
+{
+    double a, b;
+    tof_coeffs_d<TOF>(B, r, G, a, b);
+    tA = (float)a;
+    tB = (float)b;
+}
+
+// One slab of a ray: its cells, crossings and term fractions.  With cs1 <= cs2
+// the two secondary cells the slab spans and cz1 <= cz2 the axial ones, the
+// reference's branch tree (siddon.cu.cc:86-189 x-dominant, 231-333 y-dominant;
+// siddon_tof.cu.cc:102-210, 244-366) is, flattened:
+//   term 1, fraction r1, cell (cs1, cz1);
+//   term 2, fraction r2, cell (cs1, cz2) if rs > rz, else (cs2, cz1): where both
+//           axes cross;
+//   term 3, fraction r3, cell (cs2, cz2): where an axis crosses;
+// each where its cell lies in the image, and term 2 only with cz1 >= -1 (resp.
+// cs1 >= -1), term 3 with both (the top-level tests cs1 >= (crossing ? -1 : 0)
+// && cs1 < ns, and the same along z, are implied by these).
+struct Slab {
+    int cs1, cs2, cz1, cz2;
+    bool bs, bz;       // the slab crosses a secondary / axial cell boundary
+    bool sgt;          // rs > rz
+    float r1, r2, r3;
+    float sl, sh, zl, zh;
 };
 
-// The slab loop over [a, b).  Act provides
-//   void term(int ip, int cs, int cz, int branch, float weight)
-// with (ip, cs, cz) the primary slab, secondary and axial cell of the term.
-template <bool TOF, bool DIV_S, bool DIV_Z, class Act>
-__device__ __forceinline__ void march_slabs(const Branch &B, float z1, const LaunchGeom &G, int a, int b, float W,
-                                            const TofLine &T, Act &act)
+// S0, Z0 (S1, Z1): secondary and axial coordinate at the slab's lower (upper)
+// boundary.
+__device__ __forceinline__ void slab_cells(Slab &c, float S0, float S1, float Z0, float Z1, bool ks_pos, bool kz_pos)
 {
-    const bool ks_pos = B.ks >= 0.0f;
-    const bool kz_pos = B.kz >= 0.0f;
-    const int ns = B.ns, nz = G.nz;
-    float pp1 = (float)a - B.np2;
-    float S0, Z0;
-    {
-        float s = B.sec1 + B.ks * (pp1 - B.p1);
-        S0 = (DIV_S ? s / B.ds : s) + B.ns2;
-        float z = z1 + B.kz * (pp1 - B.p1);
-        Z0 = (DIV_Z ? z / G.dz : z) + G.nz2;
+    c.sl = ks_pos ? S0 : S1;
+    c.sh = ks_pos ? S1 : S0;
+    c.zl = kz_pos ? Z0 : Z1;
+    c.zh = kz_pos ? Z1 : Z0;
+    c.cs1 = cvt_flr(c.sl);
+    c.cs2 = cvt_flr(c.sh);
+    c.cz1 = cvt_flr(c.zl);
+    c.cz2 = cvt_flr(c.zh);
+    c.bs = c.cs1 != c.cs2;
+    c.bz = c.cz1 != c.cz2;
+}
+
+// Fractions from reciprocal estimates; exact quotients only where those cannot
+// decide rs > rz, which picks term 2's cell (they lie in (0, 1]: the absolute
+// margin is far above the estimates' few-ulp error).
+__device__ __forceinline__ void slab_fractions(Slab &c)
+{
+    const float dsv = c.sh - c.sl, dzv = c.zh - c.zl;
+    const float ns_ = (float)c.cs2 - c.sl, nz_ = (float)c.cz2 - c.zl;
+    const float es_ = ns_ * __builtin_amdgcn_rcpf(dsv), ez_ = nz_ * __builtin_amdgcn_rcpf(dzv);
+    float rs = c.bs ? es_ : 1.0f, rz = c.bz ? ez_ : 1.0f;
+    float dr = rs - rz;
+    if (c.bs && c.bz && !(fabsf(dr) > 4e-6f)) {
+        rs = ns_ / dsv;
+        rz = nz_ / dzv;
+        dr = rs - rz;
     }
+    asm("" : "+v"(dr));   // keeps |dr| a source modifier of its uses
+    c.sgt = dr > 0.0f;
+    c.r1 = min_nonneg(rs, rz);
+    c.r2 = fabsf(dr);
+    c.r3 = 1.0f - ((c.bs && c.bz) ? max_nonneg(rs, rz) : c.r1);
+}
+
+__device__ __forceinline__ Slab slab_eval(float S0, float S1, float Z0, float Z1, bool ks_pos, bool kz_pos)
+{
+    Slab c;
+    slab_cells(c, S0, S1, Z0, Z1, ks_pos, kz_pos);
+    slab_fractions(c);
+    return c;
+}
+
+// Which of a slab's terms apply, and term 2's cell.
+struct SlabTerms {
+    bool v1, v2, v3;
+    int csm, czm;
+};
+__device__ __forceinline__ SlabTerms slab_terms(const Slab &c, int ns, int nz)
+{
+    const bool s1 = (unsigned)c.cs1 < (unsigned)ns, s2 = (unsigned)c.cs2 < (unsigned)ns;
+    const bool z1 = (unsigned)c.cz1 < (unsigned)nz, z2 = (unsigned)c.cz2 < (unsigned)nz;
+    const bool los = c.cs1 >= -1, loz = c.cz1 >= -1, both = c.bs && c.bz;
+    SlabTerms t;
+    t.v1 = s1 && z1;
+    t.v2 = both && (c.sgt ? (s1 && z2 && loz) : (s2 && z1 && los));
+    t.v3 = (c.bs || c.bz) && s2 && z2 && los && loz;
+    t.csm = c.sgt ? c.cs1 : c.cs2;
+    t.czm = c.sgt ? c.cz2 : c.cz1;
+    return t;
+}
+
+// Branch labels of a slab's terms (the digest's): siddon.cu.cc's cases in order.
+__device__ __forceinline__ int slab_label1(const Slab &c) { return c.bs ? (c.bz ? (c.sgt ? 5 : 8) : 3) : (c.bz ? 1 : 0); }
+__device__ __forceinline__ int slab_label2(const Slab &c) { return c.sgt ? 6 : 9; }
+__device__ __forceinline__ int slab_label3(const Slab &c) { return c.bs ? (c.bz ? (c.sgt ? 7 : 10) : 4) : 2; }
+
+// Secondary / axial coordinate of a ray at primary coordinate pp, in the
+// reference's operations.
+template <bool DIV_S>
+__device__ __forceinline__ float coord_s(const Branch &B, float pp)
+{
+    const float s = B.sec1 + B.ks * (pp - B.p1);
+    return (DIV_S ? s / B.ds : s) + B.ns2;
+}
+template <bool DIV_Z>
+__device__ __forceinline__ float coord_z(const Branch &B, float z1, const LaunchGeom &G, float pp)
+{
+    const float z = z1 + B.kz * (pp - B.p1);
+    return (DIV_Z ? z / G.dz : z) + G.nz2;
+}
+
+// The slab loop over [a, b).  Act provides
+//   void slab(int ip, const Slab &c, float e)
+// with ip the primary slab and e the TOF Gaussian at it (1 without TOF).
+template <bool TOF, bool DIV_S, bool DIV_Z, class Act>
+__device__ __forceinline__ void march_slabs(const Branch &B, float z1, const LaunchGeom &G, int a, int b, float tA,
+                                            float tB, Act &act)
+{
+    const bool ks_pos = B.ks >= 0.0f, kz_pos = B.kz >= 0.0f;
+    float pp1 = (float)a - B.np2;
+    float S0 = coord_s<DIV_S>(B, pp1), Z0 = coord_z<DIV_Z>(B, z1, G, pp1);
     for (int ip = a; ip < b; ++ip) {
         const float pp2 = pp1 + 1.0f;
-        float S1, Z1;
-        {
-            float s = B.sec1 + B.ks * (pp2 - B.p1);
-            S1 = (DIV_S ? s / B.ds : s) + B.ns2;
-            float z = z1 + B.kz * (pp2 - B.p1);
-            Z1 = (DIV_Z ? z / G.dz : z) + G.nz2;
+        const float S1 = coord_s<DIV_S>(B, pp2), Z1 = coord_z<DIV_Z>(B, z1, G, pp2);
+        const Slab c = slab_eval(S0, S1, Z0, Z1, ks_pos, kz_pos);
+        float e = 1.0f;
+        if (TOF) {
+            const float d = fmaf(pp1, tA, tB);
+            e = __builtin_amdgcn_exp2f(-(d * d));
         }
-        const float sl = ks_pos ? S0 : S1, sh = ks_pos ? S1 : S0;
-        const float zl = kz_pos ? Z0 : Z1, zh = kz_pos ? Z1 : Z0;
-        const int cs1 = floor_to_int(sl), cs2 = floor_to_int(sh);
-        const int cz1 = floor_to_int(zl), cz2 = floor_to_int(zh);
-        const bool bs = cs1 != cs2, bz = cz1 != cz2;
-        // top-level tests of siddon.cu.cc:86-189 (x) / 231-333 (y)
-        const bool ok = cs1 >= (bs ? -1 : 0) && cs1 < ns && cz1 >= (bz ? -1 : 0) && cz1 < nz;
-        if (ok) {
-            float wg = W;
-            if (TOF) {
-                // siddon_tof.cu.cc:55-59: Gaussian at the slab centre on the primary axis
-                const float pc = ((float)(ip - B.np / 2) + 0.5f) * B.pd_tof;
-                const float d = ((pc - B.p1) * T.inv_pd - T.ratio1) * T.L;
-                wg = W * __builtin_amdgcn_exp2f(d * d * G.tof_c1);
-            }
-            // exact quotients: the rs > rz comparison picks a voxel
-            const float rs = bs ? ((float)cs2 - sl) / (sh - sl) : 1.0f;
-            const float rz = bz ? ((float)cz2 - zl) / (zh - zl) : 1.0f;
-            const bool sgt = rs > rz;
-            {
-                const float r1 = bs ? (bz ? (sgt ? rz : rs) : rs) : (bz ? rz : 1.0f);
-                const int br = bs ? (bz ? (sgt ? 5 : 8) : 3) : (bz ? 1 : 0);
-                if (cs1 >= 0 && cz1 >= 0) act.term(ip, cs1, cz1, br, r1 * wg);
-            }
-            if (bs && bz) {
-                const int c_s = sgt ? cs1 : cs2, c_z = sgt ? cz2 : cz1;
-                const bool c2 = sgt ? (cs1 >= 0 && cz2 < nz) : (cs2 < ns && cz1 >= 0);
-                const float r2 = sgt ? (rs - rz) : (rz - rs);
-                if (c2) act.term(ip, c_s, c_z, sgt ? 6 : 9, r2 * wg);
-            }
-            if (bs || bz) {
-                const float r3 = bs ? (bz ? (sgt ? 1.0f - rs : 1.0f - rz) : 1.0f - rs) : 1.0f - rz;
-                const int br = bs ? (bz ? (sgt ? 7 : 10) : 4) : 2;
-                if (cs2 < ns && cz2 < nz) act.term(ip, cs2, cz2, br, r3 * wg);
-            }
-        }
+        act.slab(ip, c, e);
         pp1 = pp2;
         S0 = S1;
         Z0 = Z1;
     }
 }
 
-// Adapts a flat-index sink  void term(int voxel, int branch, float w)  to march_slabs.
-template <class Flat>
-struct FlatIndex {
-    Flat &f;
-    int stride_p, stride_s, stride_z;
-    __device__ __forceinline__ void term(int ip, int cs, int cz, int br, float w)
-    {
-        f.term(ip * stride_p + cs * stride_s + cz * stride_z, br, w);
-    }
-};
+// The slab interval and branch of one event, as one reference device function:
+// [a, b) is empty where the event has no terms.  Not for r.nan events.
+template <bool TOF, int VAR>
+__device__ __forceinline__ void event_slabs(const RaySetup &r, const LaunchGeom &G, Branch &B, int &a, int &b)
+{
+    const bool xdom = (!TOF && VAR == V_FP) ? r.xdom_ge : r.xdom_gt;
+    make_branch(r, xdom, G, B);
+    a = b = 0;
+    if (!r.live || (!TOF && VAR == V_FP && r.q2)) return;
+    int lo, hi;
+    clip_range(B, r, G, lo, hi);
+    a = lo;
+    b = hi;
+    if (VAR == V_FP) fp_cut_range<TOF>(B, lo, hi, a, b);
+}
 
-// One event, as one reference device function.  Act must provide
-//   void term(int voxel, int branch, float weight)   (flat kernel-layout index)
-//   void nan_event()                                  (non-finite endpoints)
+// One event: Act provides
+//   void begin(const Branch &B, float W)          its branch and weight constant
+//   void slab(int ip, const Slab &c, float e)
+//   void nan_event()                              (non-finite endpoints)
+// lane `part` of `parts` takes its share of the event's slabs.
 template <bool TOF, int VAR, bool DIV_S, bool DIV_Z, class Act>
 __device__ __forceinline__ void march_event(const float *__restrict__ lor, float tof_value, const LaunchGeom &G,
-                                            Act &act)
+                                            int part, int parts, Act &act)
 {
     RaySetup r;
     ray_setup<TOF>(lor, tof_value, G, r);
@@ -335,20 +466,19 @@ __device__ __forceinline__ void march_event(const float *__restrict__ lor, float
         act.nan_event();
         return;
     }
-    if (!r.live) return;
-    if (!TOF && VAR == V_FP && r.q2) return;
-    const bool xdom = (!TOF && VAR == V_FP) ? r.xdom_ge : r.xdom_gt;
     Branch B;
-    make_branch(r, xdom, G, B);
-    const float W = branch_weight<TOF>(B, r, G, VAR == V_FP);
-    int lo, hi;
-    clip_range(B, r, G, lo, hi);
-    int a = lo, b = hi;
-    if (VAR == V_FP) fp_cut_range<TOF>(B, lo, hi, a, b);
-    TofLine T{0.0f, r.ratio1, r.L};
-    if (TOF) T.inv_pd = 1.0f / (B.p2 - B.p1);
-    FlatIndex<Act> fi{act, B.stride_p, B.stride_s, G.nx * G.ny};
-    march_slabs<TOF, DIV_S, DIV_Z>(B, r.z1, G, a, b, W, T, fi);
+    int a, b;
+    event_slabs<TOF, VAR>(r, G, B, a, b);
+    if (parts > 1) {
+        const int share = (b - a + parts - 1) / parts;
+        a = min(b, a + part * share);
+        b = min(b, a + share);
+    }
+    if (a >= b) return;
+    float tA, tB;
+    tof_coeffs<TOF>(B, r, G, tA, tB);
+    act.begin(B, branch_weight<TOF>(B, r, G, VAR == V_FP));
+    march_slabs<TOF, DIV_S, DIV_Z>(B, r.z1, G, a, b, tA, tB, act);
 }
 
 }  // namespace srf

@@ -1,13 +1,16 @@
-// srf_project.hip -- projector / backprojector kernels and their C-ABI entry
-// points (declared in include/srf_hip.h).
+// srf_project.hip -- one-shot projector / backprojector kernels (no plan) and their
+// C-ABI entry points (declared in include/srf_hip.h).
 //
-// Kernels (one event per lane, 256-lane workgroups, N/256 workgroups):
-//   k_gather   forward projection            (Projection[Tof] op)
-//   k_scatter  backprojection                (Backprojection[Tof] op / adjoint)
-//   k_digest   per-event term digest         (verification of voxel indexing)
-// All three instantiate the same srf::march_event, so the digest proves the
+//   k_gather   forward projection, 1 to 16 lanes per event   (Projection[Tof] op)
+//   k_bundle   forward projection of a long list, its events sorted into bundles
+//              of neighbouring lines over transposed copies of the image
+//   k_scatter  backprojection, one event per lane   (Backprojection[Tof] op / adjoint)
+//   k_digest   per-event term digest        (verification of voxel indexing)
+// All of them evaluate a slab through srf::slab_eval, so the digest proves the
 // indexing of the projector and backprojector themselves.
 #include <hip/hip_runtime.h>
+#include <hipcub/hipcub.hpp>
+#include <limits.h>
 #include <math.h>
 #include <stdint.h>
 
@@ -17,26 +20,99 @@
 
 namespace srf {
 
+// Kernel-layout voxel of a cell, for one branch.
+struct VoxelIndex {
+    int sp, ss, sz, ns, nz;
+    __device__ __forceinline__ void set(const Branch &B, const LaunchGeom &G)
+    {
+        sp = B.stride_p;
+        ss = B.stride_s;
+        sz = G.nx * G.ny;
+        ns = B.ns;
+        nz = G.nz;
+    }
+    __device__ __forceinline__ unsigned at(int ip, int cs, int cz) const
+    {
+        return (unsigned)ip * (unsigned)sp + (unsigned)cs * (unsigned)ss + (unsigned)cz * (unsigned)sz;
+    }
+};
+
+// Projections are summed in runs of SUM_RUN slabs, and the runs' sums then: along a
+// uniform image the slabs' sums are one constant, which added up one by one in
+// float32 rounds the same way over whole binades (4 times the error at 200 slabs).
+constexpr int SUM_RUN = 16;
+
+// The three loads of a slab are issued together: terms that do not apply read
+// voxel 0 and are replaced by zero.
 struct GatherAct {
     const float *__restrict__ img;
-    float acc;
-    __device__ __forceinline__ void term(int v, int, float w) { acc += img[v] * w; }
-    __device__ __forceinline__ void nan_event() { acc = __builtin_nanf(""); }
+    float sum, part;
+    float W;
+    VoxelIndex V;
+    __device__ __forceinline__ void begin(const Branch &B, float w)
+    {
+        V.set(B, *G);
+        W = w;
+    }
+    __device__ __forceinline__ void slab(int ip, const Slab &c, float e)
+    {
+        const SlabTerms t = slab_terms(c, V.ns, V.nz);
+        const unsigned i1 = t.v1 ? V.at(ip, c.cs1, c.cz1) : 0u;
+        const unsigned i2 = t.v2 ? V.at(ip, t.csm, t.czm) : 0u;
+        const unsigned i3 = t.v3 ? V.at(ip, c.cs2, c.cz2) : 0u;
+        float g1 = img[i1], g2 = img[i2], g3 = img[i3];
+        g1 = t.v1 ? g1 : 0.0f;
+        g2 = t.v2 ? g2 : 0.0f;
+        g3 = t.v3 ? g3 : 0.0f;
+        part = fmaf(fmaf(g1, c.r1, fmaf(g2, c.r2, g3 * c.r3)), e, part);
+        if ((ip & (SUM_RUN - 1)) == SUM_RUN - 1) {
+            sum += part;
+            part = 0.0f;
+        }
+    }
+    __device__ __forceinline__ void nan_event() { sum = __builtin_nanf(""); W = 1.0f; }
+    const LaunchGeom *G;
 };
 
 struct ScatterAct {
     float *__restrict__ img;
     float value;
-    __device__ __forceinline__ void term(int v, int, float w) { unsafeAtomicAdd(img + v, value * w); }
+    float vw;
+    VoxelIndex V;
+    const LaunchGeom *G;
+    __device__ __forceinline__ void begin(const Branch &B, float w)
+    {
+        V.set(B, *G);
+        vw = value * w;
+    }
+    __device__ __forceinline__ void slab(int ip, const Slab &c, float e)
+    {
+        const SlabTerms t = slab_terms(c, V.ns, V.nz);
+        const float v = vw * e;
+        if (t.v1) unsafeAtomicAdd(img + V.at(ip, c.cs1, c.cz1), v * c.r1);
+        if (t.v2) unsafeAtomicAdd(img + V.at(ip, t.csm, t.czm), v * c.r2);
+        if (t.v3) unsafeAtomicAdd(img + V.at(ip, c.cs2, c.cz2), v * c.r3);
+    }
     __device__ __forceinline__ void nan_event() {}
 };
 
 struct DigestAct {
     uint64_t h;
     int cnt;
-    __device__ __forceinline__ void term(int v, int br, float) {
-        h += mix64(((uint64_t)(uint32_t)v << 4) | (uint64_t)br);
+    VoxelIndex V;
+    const LaunchGeom *G;
+    __device__ __forceinline__ void begin(const Branch &B, float) { V.set(B, *G); }
+    __device__ __forceinline__ void add(unsigned v, int br)
+    {
+        h += mix64(((uint64_t)v << 4) | (uint64_t)br);
         cnt += 1;
+    }
+    __device__ __forceinline__ void slab(int ip, const Slab &c, float)
+    {
+        const SlabTerms t = slab_terms(c, V.ns, V.nz);
+        if (t.v1) add(V.at(ip, c.cs1, c.cz1), slab_label1(c));
+        if (t.v2) add(V.at(ip, t.csm, t.czm), slab_label2(c));
+        if (t.v3) add(V.at(ip, c.cs2, c.cz2), slab_label3(c));
     }
     __device__ __forceinline__ void nan_event() {}
 };
@@ -50,17 +126,241 @@ __device__ __forceinline__ float event_ratio(const float *__restrict__ y, const 
     return yy / d;
 }
 
+// 2^lg lanes per event (lg <= 4), each on a run of its slabs: a short list then
+// still fills the chip and its serial chain of dependent loads is shorter.  The
+// lanes' sums are combined by a fixed butterfly.
 template <bool TOF, int VAR, bool DS, bool DZ>
 __global__ __launch_bounds__(256) void k_gather(const float *__restrict__ lors, int64_t n, int stride,
                                                 const float *__restrict__ tofv, int tof_stride,
-                                                const float *__restrict__ img, LaunchGeom G,
+                                                const float *__restrict__ img, LaunchGeom G, int lg,
                                                 float *__restrict__ out)
 {
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t e = t >> lg;
+    const int parts = 1 << lg, part = (int)threadIdx.x & (parts - 1);
+    const bool on = e < n;   // whole groups of lanes: the grid is rounded up to blocks of 256
+    GatherAct act;
+    act.img = img;
+    act.sum = act.part = act.W = 0.0f;
+    act.G = &G;
+    if (on) march_event<TOF, VAR, DS, DZ>(lors + e * stride, TOF ? tofv[e * tof_stride] : 0.0f, G, part, parts, act);
+    float s = (act.sum + act.part) * act.W;
+    for (int k = parts >> 1; k > 0; k >>= 1) s += __shfl_xor(s, k);
+    if (on && part == 0) out[e] = s;
+}
+
+// -------------------------------------------------------- bundled projector --
+// A long list in arbitrary order: with one event per lane every term is a load
+// of its own cache line that misses L2 (a 256 x 256 x 128 image is 32 MiB, an
+// XCD's L2 4 MiB; 5e6 TOF events took 21.2 ms, 2e9 terms at one line each).
+// Instead
+//   - the events are sorted by the line they lie on: a bit-interleaved key of the
+//     dominant axis, the secondary and axial position at the image centre and the
+//     two slopes (k_line_keys, a radix sort of 24 key bits), so that a wavefront
+//     holds a bundle of neighbouring lines;
+//   - the image is copied once per dominant axis with the axial index fastest,
+//     [primary][secondary][axial], inside a one-cell zero border along the last
+//     two (k_border_image), and a wavefront steps through the planes of its
+//     dominant axis together: its 64 lanes read a patch of one plane, a few
+//     rows of a few lines each, from a scalar plane address.  Cells are clamped
+//     into the border instead of being tested (they read zero there).
+// Every XCD takes a contiguous run of bundles, whose lines its L2 keeps.
+
+// The key of a line.
+__device__ __forceinline__ unsigned line_key(const Branch &B, float z1, const LaunchGeom &G)
+{
+    auto cell = [](float v, float hi) { return (unsigned)fminf(fmaxf(v, 0.0f), hi); };
+    const float is = 64.0f / (float)B.ns, iz = 32.0f / (float)G.nz;
+    const float s = (B.sec1 - B.ks * B.p1) / B.ds + B.ns2, z = (z1 - B.kz * B.p1) / G.dz + G.nz2;
+    const float t = B.ks * B.np2 / B.ds + B.ns2, w = B.kz * B.np2 / G.dz + G.nz2;
+    const unsigned qs = cell(s * is, 63.0f), qt = cell(t * is, 63.0f), qz = cell(z * iz, 31.0f), qw = cell(w * iz, 31.0f);
+    unsigned k = B.xdom ? 0u : 1u;
+    auto put = [&](unsigned v, int bit) { k = (k << 1) | ((v >> bit) & 1u); };
+    // positions and slopes of the secondary axis first: a line of 32 axial cells
+    // is one 128-byte cache line, so a bundle may be wider along it
+    put(qs, 5); put(qt, 5); put(qs, 4); put(qt, 4); put(qs, 3); put(qt, 3); put(qz, 4); put(qw, 4);
+    put(qs, 2); put(qt, 2); put(qz, 3); put(qw, 3); put(qs, 1); put(qt, 1); put(qz, 2); put(qw, 2);
+    put(qs, 0); put(qt, 0); put(qz, 1); put(qw, 1); put(qz, 0); put(qw, 0);
+    return k;
+}
+constexpr int LINE_KEY_BITS = 24;
+
+// Key and index of every event; events without terms (and non-finite ones) last.
+template <bool TOF>
+__global__ __launch_bounds__(256) void k_line_keys(const float *__restrict__ lors, int64_t n, int stride, LaunchGeom G,
+                                                   unsigned *__restrict__ key, int *__restrict__ idx)
+{
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (e >= n) return;
-    GatherAct act{img, 0.0f};
-    march_event<TOF, VAR, DS, DZ>(lors + e * stride, TOF ? tofv[e * tof_stride] : 0.0f, G, act);
-    out[e] = act.acc;
+    RaySetup r;
+    ray_setup<false>(lors + e * stride, 0.0f, G, r);
+    unsigned k = (1u << LINE_KEY_BITS) - 1u;
+    if (r.live && (TOF || !r.q2)) {
+        Branch B;
+        make_branch(r, TOF ? r.xdom_gt : r.xdom_ge, G, B);
+        k = line_key(B, r.z1, G);
+    }
+    key[e] = k;
+    idx[e] = (int)e;
+}
+
+// The two bordered copies: zx[x][y + 1][z + 1] and zy[y][x + 1][z + 1], rows of
+// pz = nz + 2.  One workgroup per 32 x 32 (x, z) tile of a y row of the border
+// box, transposed through LDS.
+__global__ __launch_bounds__(256) void k_border_image(const float *__restrict__ img, int nx, int ny, int nz,
+                                                      float *__restrict__ zx, float *__restrict__ zy)
+{
+    __shared__ float tile[32][33];
+    const int x0 = blockIdx.x * 32 - 1, z0 = blockIdx.y * 32 - 1, y = (int)blockIdx.z - 1;
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    const int pz = nz + 2;
+    const bool iny = y >= 0 && y < ny;
+    for (int k = ty; k < 32; k += 8) {
+        const int x = x0 + tx, z = z0 + k;
+        tile[k][tx] = (iny && x >= 0 && x < nx && z >= 0 && z < nz) ? img[x + (int64_t)nx * (y + (int64_t)ny * z)] : 0.0f;
+    }
+    __syncthreads();
+    for (int k = ty; k < 32; k += 8) {
+        const int x = x0 + k, z = z0 + tx;
+        if (x > nx || z > nz) continue;
+        const float v = tile[tx][k];
+        if (x >= 0 && x < nx) zx[((int64_t)x * (ny + 2) + y + 1) * pz + z + 1] = v;
+        if (iny) zy[((int64_t)y * (nx + 2) + x + 1) * pz + z + 1] = v;
+    }
+}
+
+__device__ __forceinline__ int wave_min(int v)
+{
+    for (int k = 32; k > 0; k >>= 1) v = min(v, __shfl_xor(v, k));
+    return __builtin_amdgcn_readfirstlane(v);
+}
+__device__ __forceinline__ int wave_max(int v)
+{
+    for (int k = 32; k > 0; k >>= 1) v = max(v, __shfl_xor(v, k));
+    return __builtin_amdgcn_readfirstlane(v);
+}
+
+// Sum over the slabs [a, b) of every lane's ray (a >= b: none), the wavefront in
+// step through the planes of a bordered copy of pl floats per plane; of `parts`
+// wavefronts with the same rays, number `part` takes its share of the planes.
+template <bool TOF, bool DS, bool DZ>
+__device__ __forceinline__ float bundle_sum(const Branch &B, float z1, const LaunchGeom &G, int a, int b, float tA,
+                                            float tB, const float *__restrict__ copy, int64_t pl, int pz, int part, int parts)
+{
+    const bool on = a < b;
+    int ia = wave_min(on ? a : INT_MAX), ib = wave_max(on ? b : INT_MIN);
+    const int share = (ib - ia + parts - 1) / parts;
+    ia = __builtin_amdgcn_readfirstlane(ia + part * share);
+    ib = min(ib, ia + share);
+    if (ia >= ib) return 0.0f;
+    const bool ks_pos = B.ks >= 0.0f, kz_pos = B.kz >= 0.0f;
+    // border clamps, row pitch and origin held in vector registers (v_med3 and
+    // v_mad read at most one scalar register)
+    int lo = -1, ns = B.ns, nz = G.nz, row = 4 * pz, org = 4 * (pz + 1);
+    asm volatile("" : "+v"(lo), "+v"(ns), "+v"(nz), "+v"(row), "+v"(org));
+    const float *plane = copy + ia * pl;
+    float pp1 = (float)ia - B.np2;
+    float S0 = coord_s<DS>(B, pp1), Z0 = coord_z<DZ>(B, z1, G, pp1);
+    float acc = 0.0f, sum = 0.0f;
+    const unsigned len = on ? (unsigned)(b - a) : 0u;
+    int ip = ia;
+    auto slab = [&]() {
+        const float pp2 = pp1 + 1.0f;
+        const float S1 = coord_s<DS>(B, pp2), Z1 = coord_z<DZ>(B, z1, G, pp2);
+        if ((unsigned)(ip - a) < len) {
+            Slab c;
+            slab_cells(c, S0, S1, Z0, Z1, ks_pos, kz_pos);
+            const bool los = c.cs1 >= -1, loz = c.cz1 >= -1;
+            // byte offsets in the plane; offset 0 is a border cell
+            const int c1 = med3_i32(c.cs1, lo, ns), c2 = med3_i32(c.cs2, lo, ns);
+            const int d1 = med3_i32(c.cz1, lo, nz), d2 = med3_i32(c.cz2, lo, nz);
+            const int A = mad_i24(c1, row, org), C = mad_i24(c2, row, org);
+            const int j2a = A + 4 * d2, j2b = C + 4 * d1, j3 = C + 4 * d2;
+            unsigned i1 = (unsigned)(A + 4 * d1);
+            unsigned i2a = (c.bs && c.bz && loz) ? (unsigned)j2a : 0u, i2b = (c.bs && c.bz && los) ? (unsigned)j2b : 0u;
+            unsigned i3 = ((c.bs || c.bz) && los && loz) ? (unsigned)j3 : 0u;
+            // here: sunk past the branch in slab_fractions, their lane masks would
+            // be carried across it as 0/1 vectors
+            asm volatile("" : "+v"(i1), "+v"(i2a), "+v"(i2b), "+v"(i3));
+            slab_fractions(c);
+            const unsigned i2 = c.sgt ? i2a : i2b;
+            const char *p = reinterpret_cast<const char *>(plane);
+            const float g1 = *reinterpret_cast<const float *>(p + i1);
+            const float g2 = *reinterpret_cast<const float *>(p + i2);
+            const float g3 = *reinterpret_cast<const float *>(p + i3);
+            float e = 1.0f;
+            if (TOF) {
+                const float dd = fmaf(pp1, tA, tB);
+                e = __builtin_amdgcn_exp2f(-(dd * dd));
+            }
+            const float s = fmaf(g1, c.r1, fmaf(g2, c.r2, g3 * c.r3));
+            acc = TOF ? fmaf(s, e, acc) : acc + s;
+        }
+        if ((ip & (SUM_RUN - 1)) == SUM_RUN - 1) {   // a scalar test: the wavefront is in step
+            sum += acc;
+            acc = 0.0f;
+        }
+        pp1 = pp2;
+        S0 = S1;
+        Z0 = Z1;
+        plane += pl;
+        ++ip;
+    };
+    // twice per trip, so that the values carried from slab to slab alternate
+    // registers instead of moving
+    while (ip < ib) {
+        slab();
+        if (!(ip < ib)) break;
+        slab();
+    }
+    return sum + acc;
+}
+
+template <bool TOF, bool DS, bool DZ>
+__global__ __launch_bounds__(256) void k_bundle(const float *__restrict__ lors, int64_t n, int stride,
+                                                const float *__restrict__ tofv, int tof_stride,
+                                                const int *__restrict__ order, const float *__restrict__ zx,
+                                                const float *__restrict__ zy, LaunchGeom G, int lgp, int nblk,
+                                                float *__restrict__ out)
+{
+    __shared__ float part_sum[256];
+    // workgroup i runs on XCD i % 8: a contiguous run of bundles per XCD
+    const int per = gridDim.x >> 3;
+    const int blk = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if (blk >= nblk) return;
+    // 2^lgp wavefronts of the workgroup share a bundle
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int parts = 1 << lgp, part = wave & (parts - 1);
+    const int64_t i = (int64_t)blk * (256 >> lgp) + (wave >> lgp) * 64 + (threadIdx.x & 63);
+    const bool in = i < n;
+    const int64_t e = in ? order[i] : 0;
+    RaySetup r;
+    ray_setup<TOF>(lors + e * stride, TOF ? tofv[e * tof_stride] : 0.0f, G, r);
+    Branch B;
+    int a, b;
+    event_slabs<TOF, V_FP>(r, G, B, a, b);
+    if (!in || r.nan) a = b = 0;
+    float tA, tB;
+    tof_coeffs<TOF>(B, r, G, tA, tB);
+    const float W = branch_weight<TOF>(B, r, G, true);
+    const int pz = G.nz + 2;
+    float s = 0.0f;
+    // a wavefront holds one branch, but for the one where the sorted list changes over
+    if (__any(a < b && B.xdom))
+        s = bundle_sum<TOF, DS, DZ>(B, r.z1, G, a, B.xdom ? b : a, tA, tB, zx, (int64_t)(G.ny + 2) * pz, pz,
+                                    part, parts);
+    if (__any(a < b && !B.xdom)) {
+        const float t = bundle_sum<TOF, DS, DZ>(B, r.z1, G, a, B.xdom ? a : b, tA, tB, zy, (int64_t)(G.nx + 2) * pz, pz,
+                                                  part, parts);
+        s = B.xdom ? s : t;
+    }
+    if (lgp > 0) {
+        part_sum[threadIdx.x] = s;
+        __syncthreads();
+        if (part != 0) return;
+        for (int k = 1; k < parts; ++k) s += part_sum[threadIdx.x + 64 * k];
+    }
+    if (in) out[e] = r.nan ? __builtin_nanf("") : (a < b ? s * W : 0.0f);
 }
 
 // values == nullptr: all ones.  y/p != nullptr: value = ratio(y, p).
@@ -76,8 +376,11 @@ __global__ __launch_bounds__(256) void k_scatter(const float *__restrict__ lors,
     float v = 1.0f;
     if (y) v = event_ratio(y, p, e, kind, eps);
     else if (values) v = values[e];
-    ScatterAct act{img, v};
-    march_event<TOF, VAR, DS, DZ>(lors + e * stride, TOF ? tofv[e * tof_stride] : 0.0f, G, act);
+    ScatterAct act;
+    act.img = img;
+    act.value = v;
+    act.G = &G;
+    march_event<TOF, VAR, DS, DZ>(lors + e * stride, TOF ? tofv[e * tof_stride] : 0.0f, G, 0, 1, act);
 }
 
 template <bool TOF, int VAR, bool DS, bool DZ>
@@ -87,8 +390,11 @@ __global__ __launch_bounds__(256) void k_digest(const float *__restrict__ lors, 
 {
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= n) return;
-    DigestAct act{0ull, 0};
-    march_event<TOF, VAR, DS, DZ>(lors + e * stride, TOF ? tofv[e * tof_stride] : 0.0f, G, act);
+    DigestAct act;
+    act.h = 0ull;
+    act.cnt = 0;
+    act.G = &G;
+    march_event<TOF, VAR, DS, DZ>(lors + e * stride, TOF ? tofv[e * tof_stride] : 0.0f, G, 0, 1, act);
     hash[e] = act.h;
     count[e] = act.cnt;
 }
@@ -158,6 +464,113 @@ static int check_events(const float *lors, int64_t n, int64_t stride, const floa
 
 static inline unsigned blocks_for(int64_t n) { return (unsigned)((n + 255) / 256); }
 
+// Lists of at least BUNDLE_SLABS slabs (events times the longer transaxial side of
+// the image; twice that where the image fits an XCD's 4 MiB L2) are bundled,
+// BUNDLE_CHUNK events at a time (the scratch of a chunk is about 20 bytes per event
+// plus the two copies).  Images that fit L2 several times over never are.  Measured,
+// us, bundled / one event per lane:
+//   256 x 256 x 128   65536 events 148 / 126, 98304 188 / 230, 2^18 317 / 548, 2^20 780 / 2838
+//   181 x 217 x 91    65536 109 / 97, 98304 141 / 167, 2^18 245 / 346, 2^20 630 / 1567
+//   128 x 128 x 64    2^17 110 / 90, 2^18 183 / 174, 2^19 272 / 340, 2^20 442 / 672
+//   48 x 48 x 24      2^20 275 / 189
+// 5e6 TOF events on 256 x 256 x 128: 2.49 ms against 21.3 ms (each term a line of its
+// own from beyond L2).  Now VALU bound: about 75 instructions per slab.
+constexpr int64_t BUNDLE_SLABS = 20000000;
+constexpr int64_t BUNDLE_IMAGE_MIN = 1 << 20;
+constexpr int64_t BUNDLE_IMAGE_L2 = 4 << 20;
+constexpr int64_t BUNDLE_CHUNK = 1 << 23;
+constexpr int64_t BUNDLE_SPLIT = 1 << 17;
+constexpr int64_t BUNDLE_IMAGE_BYTES = 1 << 30;   // of both copies
+
+// True on a stream that is being captured (no scratch can be taken for it then),
+// or whose state cannot be told.
+static bool capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
+// The bundled projection; false where it does not apply (nothing is queued then).
+static bool project_bundled(const float *lors, int64_t n, int stride, const float *tofv, int tof_stride,
+                            const float *image, const LaunchGeom &G, bool tof, bool ds, bool dz, float *out,
+                            hipStream_t s, int &rc)
+{
+    const int64_t bytes = (int64_t)G.nx * G.ny * G.nz * 4, slabs = n * (G.nx > G.ny ? G.nx : G.ny);
+    if (bytes < BUNDLE_IMAGE_MIN || slabs < (bytes > BUNDLE_IMAGE_L2 + (BUNDLE_IMAGE_L2 >> 2) ? 1 : 2) * BUNDLE_SLABS) return false;
+    const int64_t pz = (int64_t)G.nz + 2, px = (int64_t)(G.ny + 2) * pz, py = (int64_t)(G.nx + 2) * pz;
+    const int64_t vx = G.nx * px, vy = G.ny * py;
+    // 24-bit row pitch and cell, 16-bit grid extents
+    if (4 * (vx + vy) > BUNDLE_IMAGE_BYTES || 4 * pz >= (1 << 23) || G.nx >= (1 << 22) || G.ny > 65533 ||
+        (G.nz + 33) / 32 > 65535 || capturing(s))
+        return false;
+    const int64_t chunk = n < BUNDLE_CHUNK ? n : BUNDLE_CHUNK;
+    size_t sort_bytes = 0;
+    unsigned *k0 = nullptr, *k1 = nullptr;
+    int *i0 = nullptr, *i1 = nullptr;
+    if (hipcub::DeviceRadixSort::SortPairs(nullptr, sort_bytes, k0, k1, i0, i1, (int)chunk, 0, LINE_KEY_BITS, s) !=
+        hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+    const size_t b_list = up((size_t)chunk * 4), b_x = up((size_t)vx * 4), b_y = up((size_t)vy * 4);
+    char *w = static_cast<char *>(pool_get(4 * b_list + b_x + b_y + sort_bytes, s));
+    if (!w) return false;
+    k0 = reinterpret_cast<unsigned *>(w);
+    k1 = reinterpret_cast<unsigned *>(w + b_list);
+    i0 = reinterpret_cast<int *>(w + 2 * b_list);
+    i1 = reinterpret_cast<int *>(w + 3 * b_list);
+    float *zx = reinterpret_cast<float *>(w + 4 * b_list), *zy = reinterpret_cast<float *>(w + 4 * b_list + b_x);
+    void *tmp = w + 4 * b_list + b_x + b_y;
+    hipLaunchKernelGGL(k_border_image, dim3((unsigned)((G.nx + 33) / 32), (unsigned)((G.nz + 33) / 32), (unsigned)(G.ny + 2)),
+                       dim3(256), 0, s, image, G.nx, G.ny, G.nz, zx, zy);
+    rc = launch_status();
+    for (int64_t c = 0; c < n && rc == SRF_OK; c += chunk) {
+        const int64_t m = n - c < chunk ? n - c : chunk;
+        const float *L = lors + c * stride, *T = tof ? tofv + c * tof_stride : nullptr;
+        if (tof)
+            hipLaunchKernelGGL(k_line_keys<true>, dim3(blocks_for(m)), dim3(256), 0, s, L, m, stride, G, k0, i0);
+        else
+            hipLaunchKernelGGL(k_line_keys<false>, dim3(blocks_for(m)), dim3(256), 0, s, L, m, stride, G, k0, i0);
+        if (hipcub::DeviceRadixSort::SortPairs(tmp, sort_bytes, k0, k1, i0, i1, (int)m, 0, LINE_KEY_BITS, s) != hipSuccess) {
+            (void)hipGetLastError();
+            rc = SRF_ERR_LAUNCH;
+            break;
+        }
+        // up to four wavefronts per bundle while there are few bundles (2^16 events on
+        // 256 x 256 x 128: 148 us with four, 267 with one; 2^18: 345, 317)
+        const int lgp = m <= BUNDLE_SPLIT ? 2 : m <= 2 * BUNDLE_SPLIT ? 1 : 0;
+        const int nb = (int)blocks_for(m << lgp);
+        const dim3 grid((unsigned)((nb + 7) / 8 * 8));
+#define SRF_BUNDLE(T_, S_, Z_) \
+    hipLaunchKernelGGL((k_bundle<T_, S_, Z_>), grid, dim3(256), 0, s, L, m, stride, T, tof_stride, i1, zx, zy, G, lgp, nb,  \
+                       out + c)
+        if (tof) {
+            if (ds) { if (dz) SRF_BUNDLE(true, true, true); else SRF_BUNDLE(true, true, false); }
+            else { if (dz) SRF_BUNDLE(true, false, true); else SRF_BUNDLE(true, false, false); }
+        } else {
+            if (ds) { if (dz) SRF_BUNDLE(false, true, true); else SRF_BUNDLE(false, true, false); }
+            else { if (dz) SRF_BUNDLE(false, false, true); else SRF_BUNDLE(false, false, false); }
+        }
+#undef SRF_BUNDLE
+        rc = launch_status();
+    }
+    pool_put(w, s);
+    return true;
+}
+
+// Lanes per event of k_gather (log2): enough for about 2^17 lanes, at most 16.
+static int gather_lanes(int64_t n)
+{
+    int lg = 0;
+    while (lg < 4 && (n << (lg + 1)) <= (1 << 17)) ++lg;
+    return lg;
+}
+
 }  // namespace srf
 
 using namespace srf;
@@ -175,9 +588,13 @@ int srf_project(const float *lors, int64_t n, int64_t lor_stride, const float *t
     if (n == 0) return SRF_OK;
     hipStream_t s = (hipStream_t)stream;
     const bool ds = G.dy != 1.0f, dz = G.dz != 1.0f;
+    if (project_bundled(lors, n, (int)lor_stride, tof_values, (int)tof_stride, image, G, tof != nullptr, ds, dz, out, s,
+                        rc))
+        return rc;
+    const int lg = gather_lanes(n);
     SRF_DISPATCH(k_gather, tof != nullptr, V_FP, ds, dz,
-                 <<<blocks_for(n), 256, 0, s>>>(lors, n, (int)lor_stride, tof_values, (int)tof_stride, image, G,
-                                                out));
+                 <<<blocks_for(n << lg), 256, 0, s>>>(lors, n, (int)lor_stride, tof_values, (int)tof_stride, image, G,
+                                                      lg, out));
     return launch_status();
 }
 

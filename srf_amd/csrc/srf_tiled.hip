@@ -148,14 +148,6 @@ __device__ __forceinline__ void for_each_segment(const Branch &B, const RaySetup
     }
 }
 
-// Every segment of one event: f(tile, cls, a, b, Branch, SegCtx).  Non-TOF
-// ties (|xd| == |yd|) march different branches in the projector (>=,
-// siddon.cu.cc:46) and the backprojector (>, :372): both are binned, each
-// marked for its own direction.
-template <bool TOF>
-__device__ __forceinline__ void tof_coeffs_d(const Branch &B, const RaySetup &r, const LaunchGeom &G, double &tA,
-                                             double &tB);
-
 // TOF window (twin > 0): of the slabs [lo, hi), keep those whose Gaussian
 // factor exp2(-(pp1 tA + tB)^2) is at least 2^-twin of the largest factor in
 // [lo, hi) -- the peak inside the image, not the Gaussian's own peak, which
@@ -184,6 +176,10 @@ __device__ __forceinline__ void tof_window(const Branch &B, const RaySetup &r, c
     hi = min(hi, dbl_to_int(floor(fmax(u1, u2) + np2)) + 2);
 }
 
+// Every segment of one event: f(tile, cls, a, b, Branch, SegCtx).  Non-TOF
+// ties (|xd| == |yd|) march different branches in the projector (>=,
+// siddon.cu.cc:46) and the backprojector (>, :372): both are binned, each
+// marked for its own direction.
 template <bool TOF, class F>
 __device__ __forceinline__ void for_each_event_segment(const RaySetup &r, const LaunchGeom &G, const TileCfg &T,
                                                        float twin, F &&f)
@@ -227,35 +223,6 @@ __device__ __forceinline__ uint32_t pack_ab(int a, int b, bool xd)
 __device__ __forceinline__ int ab_a(uint32_t ab) { return (int)(ab & 0x7fffu); }
 __device__ __forceinline__ int ab_b(uint32_t ab) { return (int)(ab >> 16); }
 __device__ __forceinline__ bool ab_xd(uint32_t ab) { return (ab >> 15) & 1u; }
-
-// TOF Gaussian of siddon_tof.cu.cc:55-59 as a linear function of the slab's
-// lower boundary pp1 = ip - np2 (exact in float):
-//   pc = ((ip - np/2) + 0.5) * pd_tof = (pp1 + off) * pd_tof, off = np2 - np/2 + 0.5
-//   d  = ((pc - p1) / (p2 - p1) - ratio1) * L
-//   exp(-d^2 / (2 tse)) = exp2(-(d * sqrt(log2(e) / (2 tse)))^2)
-// Coefficients in double, rounded once.
-template <bool TOF>
-__device__ __forceinline__ void tof_coeffs_d(const Branch &B, const RaySetup &r, const LaunchGeom &G, double &tA,
-                                             double &tB)
-{
-    tA = tB = 0.0;
-    if (!TOF) return;
-    const double off = (double)B.np2 - (double)(B.np / 2) + 0.5;
-    const double s = sqrt(0.5 * 1.4426950408889634 / (double)G.tse);
-    const double k = (double)r.L / ((double)B.p2 - (double)B.p1);
-    tA = (double)B.pd_tof * k * s;
-    tB = ((off * (double)B.pd_tof - (double)B.p1) * k - (double)r.ratio1 * (double)r.L) * s;
-}
-
-template <bool TOF>
-__device__ __forceinline__ void tof_coeffs(const Branch &B, const RaySetup &r, const LaunchGeom &G, float &tA,
-                                           float &tB)
-{
-    double a, b;
-    tof_coeffs_d<TOF>(B, r, G, a, b);
-    tA = (float)a;
-    tB = (float)b;
-}
 
 template <bool TOF>
 __global__ __launch_bounds__(BIN_THREADS) void k_bin_count(const float *__restrict__ lors, int64_t n, int stride,
@@ -334,15 +301,6 @@ __global__ __launch_bounds__(BIN_THREADS) void k_bin_emit(const float *__restric
 
 // ------------------------------------------------------------ tile kernels --
 
-// v_cvt_flr_i32_f32: floor and convert in one VALU op (NaN -> 0, saturating,
-// as v_floor_f32 + v_cvt_i32_f32).
-__device__ __forceinline__ int cvt_flr(float v)
-{
-    int r;
-    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(v));
-    return r;
-}
-
 enum : int { M_GATHER = 0, M_SCATTER = 1, M_DIGEST = 2, M_SCATTER_FX = 3 };
 
 // A term v * r (v already scaled by the item's 2^shift, |v * r| < 2^49 by the
@@ -355,35 +313,6 @@ __device__ __forceinline__ unsigned long long fixed_term(double v, float r)
 {
     const double s = fma(v, (double)r, 6755399441055744.0);
     return (unsigned long long)__double_as_longlong(s) - 0x4338000000000000ull;
-}
-
-// med3(x, lo, hi) = min(max(x, lo), hi) for lo <= hi, one v_med3_i32 (the
-// compiler emits it only for constant bounds), and a * b + c with a and b taken
-// as signed 24-bit integers (v_mad_i32_i24: the clamped cell index is -1 on
-// the low-edge halo of a tile at the image origin, which the unsigned form
-// would read as 2^24 - 1).  Plain ALU instructions, no memory access.
-__device__ __forceinline__ int med3_i32(int x, int lo, int hi)
-{
-    int r;
-    asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "v"(lo), "v"(hi));
-    return r;
-}
-__device__ __forceinline__ int mad_i24(int a, int b, int c)
-{
-    int r;
-    asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-
-// Minimum / maximum of two non-negative finite floats as integer operations on
-// their bit patterns (which order the same way): no NaN canonicalisation.
-__device__ __forceinline__ float min_nonneg(float a, float b)
-{
-    return __uint_as_float(min(__float_as_uint(a), __float_as_uint(b)));
-}
-__device__ __forceinline__ float max_nonneg(float a, float b)
-{
-    return __uint_as_float(max(__float_as_uint(a), __float_as_uint(b)));
 }
 
 // State of one segment walk inside one LDS tile (layout: tile_word).  Terms

@@ -335,15 +335,24 @@ int srf_batch_em_step(srf_batch *batch, srf_ratio_kind_t kind, float eps, float 
  *   bins    (n_bins, 2)  detector pairs; out (n_bins)
  *   tables  543 floats: 511/E', window efficiency, KN/sigma_KN per integer
  *           scattering angle 0..180 degrees.
- * Below 32768 bins (a few rings, e.g. a surrogate's check subset) each bin's
- * sum over points is split across a wavefront and combined in a fixed order;
- * above, one lane sums one bin serially.  The two agree to float rounding. */
+ * Each bin's sum over points is split over wavefronts and, where there are few
+ * bins, over workgroups (then through transient scratch, outside graph capture),
+ * and combined in a fixed order. */
 size_t srf_sss_rows_bytes(int32_t n_det, int32_t n_points);
 int srf_sss_prepare(const float *det, int32_t n_det, const float *points, int32_t n_points,
                     const float *em_int, const float *mu_int, void *rows, size_t rows_bytes, void *stream);
 int srf_sss_sinogram(const void *rows, int32_t n_det, const float *points, int32_t n_points,
                      const int32_t *bins, int32_t n_bins, const float *tables, float scale, float *out,
                      void *stream);
+
+/* out[d * n_points + s] = line integral of `image` (kernel layout, per mm) from
+ * detector d (rows of 4 floats, as srf_sss_prepare) to point s (rows of
+ * point_stride >= 3 floats): srf_project along the LOR (detector, point), which
+ * the projector's segment cut ends at the point, times L^2 in units of dx_
+ * (scatter/preprocess.py:21-43).  Uses transient scratch for a copy of the image
+ * where that can be had. */
+int srf_sss_integrals(const float *det, int32_t n_det, const float *points, int32_t n_points, int32_t point_stride,
+                      const float *image, srf_grid_t grid, float *out, void *stream);
 
 /* Scatter correction of list-mode values (ScatterCorrect.__call__,
  * srfnef/corrections/scattering/scatter.py:51-53):

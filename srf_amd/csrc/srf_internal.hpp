@@ -26,6 +26,18 @@ int fill_f32(float *dst, float v, int64_t n, hipStream_t s);
 void *pool_get(size_t bytes, hipStream_t s);
 void pool_put(void *p, hipStream_t s, bool idle = false);
 
+// True on a stream that is being captured (no scratch can be taken for it then),
+// or whose state cannot be told.
+inline bool capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
 struct LaunchGeom;
 // Validates a grid (and TOF parameters) and derives the per-launch constants.
 int make_geom(const srf_grid_t &g, const srf_tof_t *tof, LaunchGeom &G);

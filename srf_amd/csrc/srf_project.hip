@@ -399,6 +399,58 @@ __global__ __launch_bounds__(256) void k_digest(const float *__restrict__ lors, 
     count[e] = act.cnt;
 }
 
+// --------------------------------------------------- point line integrals --
+// Integral of an image from every detector to every scatter point: the projector
+// along the LOR detector -> point, without the 1 / L^2 of its weight, so without
+// an LOR array, its lengths and a product with them (4 of 48 ms of an estimate of
+// 4096 detectors x 2e4 points) and without a sort: a wavefront takes 64 points in
+// a row of one detector, a bundle by itself (its points lie on a few columns of the
+// grid).  BORDER: over the axial-fastest copies of k_border_image, in step through
+// their planes; else one ray per lane on the image as it is.
+template <bool BORDER, bool DS, bool DZ>
+__global__ __launch_bounds__(256) void k_point_integrals(const float *__restrict__ det, int nd,
+                                                         const float *__restrict__ pts, int ns, int pstride,
+                                                         const float *__restrict__ img, const float *__restrict__ zx,
+                                                         const float *__restrict__ zy, LaunchGeom G, int64_t nblk,
+                                                         float *__restrict__ out)
+{
+    const int64_t per = (int64_t)gridDim.x >> 3;   // a contiguous run of detectors per XCD
+    const int64_t blk = (int64_t)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (blk >= nblk) return;
+    const int nsb = (ns + 255) / 256;
+    const int d = __builtin_amdgcn_readfirstlane((int)(blk / nsb));
+    const int s = (int)(blk % nsb) * 256 + (int)threadIdx.x;
+    const bool in = s < ns;
+    const float *P = pts + (int64_t)(in ? s : 0) * pstride;
+    const float lor[6] = {det[4 * d], det[4 * d + 1], det[4 * d + 2], P[0], P[1], P[2]};
+    RaySetup r;
+    ray_setup<false>(lor, 0.0f, G, r);
+    Branch B;
+    int a, b;
+    event_slabs<false, V_FP>(r, G, B, a, b);
+    if (!in || r.nan) a = b = 0;
+    float sum = 0.0f;
+    if (BORDER) {
+        const int pz = G.nz + 2;
+        if (__any(a < b && B.xdom))
+            sum = bundle_sum<false, DS, DZ>(B, r.z1, G, a, B.xdom ? b : a, 0.0f, 0.0f, zx, (int64_t)(G.ny + 2) * pz, pz, 0, 1);
+        if (__any(a < b && !B.xdom)) {
+            const float t = bundle_sum<false, DS, DZ>(B, r.z1, G, a, B.xdom ? a : b, 0.0f, 0.0f, zy,
+                                                      (int64_t)(G.nx + 2) * pz, pz, 0, 1);
+            sum = B.xdom ? sum : t;
+        }
+    } else if (a < b) {
+        GatherAct act;
+        act.img = img;
+        act.sum = act.part = 0.0f;
+        act.G = &G;
+        act.begin(B, 1.0f);
+        march_slabs<false, DS, DZ>(B, r.z1, G, a, b, 0.0f, 0.0f, act);
+        sum = act.sum + act.part;
+    }
+    if (in) out[(int64_t)d * ns + s] = r.nan ? __builtin_nanf("") : (a < b ? sum * (B.sq * G.dx_) : 0.0f);
+}
+
 // ----------------------------------------------------------------- host side --
 
 int make_geom(const srf_grid_t &g, const srf_tof_t *tof, LaunchGeom &G)
@@ -482,16 +534,21 @@ constexpr int64_t BUNDLE_CHUNK = 1 << 23;
 constexpr int64_t BUNDLE_SPLIT = 1 << 17;
 constexpr int64_t BUNDLE_IMAGE_BYTES = 1 << 30;   // of both copies
 
-// True on a stream that is being captured (no scratch can be taken for it then),
-// or whose state cannot be told.
-static bool capturing(hipStream_t s)
+// The bordered copies: floats of one (np planes), whether they and their 24-bit
+// cell addresses fit (and the grid of k_border_image), and the copying.
+static int64_t border_floats(int np, int ns, int nz) { return (int64_t)np * (ns + 2) * ((int64_t)nz + 2); }
+
+static bool border_fits(const LaunchGeom &G)
 {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
-        (void)hipGetLastError();
-        return true;
-    }
-    return st != hipStreamCaptureStatusNone;
+    return 4 * (border_floats(G.nx, G.ny, G.nz) + border_floats(G.ny, G.nx, G.nz)) <= BUNDLE_IMAGE_BYTES &&
+           4 * ((int64_t)G.nz + 2) < (1 << 23) && G.nx < (1 << 22) && G.ny <= 65533 && (G.nz + 33) / 32 <= 65535;
+}
+
+static int border_image(const float *image, const LaunchGeom &G, float *zx, float *zy, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_border_image, dim3((unsigned)((G.nx + 33) / 32), (unsigned)((G.nz + 33) / 32), (unsigned)(G.ny + 2)),
+                       dim3(256), 0, s, image, G.nx, G.ny, G.nz, zx, zy);
+    return launch_status();
 }
 
 // The bundled projection; false where it does not apply (nothing is queued then).
@@ -501,12 +558,7 @@ static bool project_bundled(const float *lors, int64_t n, int stride, const floa
 {
     const int64_t bytes = (int64_t)G.nx * G.ny * G.nz * 4, slabs = n * (G.nx > G.ny ? G.nx : G.ny);
     if (bytes < BUNDLE_IMAGE_MIN || slabs < (bytes > BUNDLE_IMAGE_L2 + (BUNDLE_IMAGE_L2 >> 2) ? 1 : 2) * BUNDLE_SLABS) return false;
-    const int64_t pz = (int64_t)G.nz + 2, px = (int64_t)(G.ny + 2) * pz, py = (int64_t)(G.nx + 2) * pz;
-    const int64_t vx = G.nx * px, vy = G.ny * py;
-    // 24-bit row pitch and cell, 16-bit grid extents
-    if (4 * (vx + vy) > BUNDLE_IMAGE_BYTES || 4 * pz >= (1 << 23) || G.nx >= (1 << 22) || G.ny > 65533 ||
-        (G.nz + 33) / 32 > 65535 || capturing(s))
-        return false;
+    if (!border_fits(G) || capturing(s)) return false;
     const int64_t chunk = n < BUNDLE_CHUNK ? n : BUNDLE_CHUNK;
     size_t sort_bytes = 0;
     unsigned *k0 = nullptr, *k1 = nullptr;
@@ -517,7 +569,8 @@ static bool project_bundled(const float *lors, int64_t n, int stride, const floa
         return false;
     }
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
-    const size_t b_list = up((size_t)chunk * 4), b_x = up((size_t)vx * 4), b_y = up((size_t)vy * 4);
+    const size_t b_list = up((size_t)chunk * 4), b_x = up((size_t)border_floats(G.nx, G.ny, G.nz) * 4),
+                 b_y = up((size_t)border_floats(G.ny, G.nx, G.nz) * 4);
     char *w = static_cast<char *>(pool_get(4 * b_list + b_x + b_y + sort_bytes, s));
     if (!w) return false;
     k0 = reinterpret_cast<unsigned *>(w);
@@ -526,9 +579,7 @@ static bool project_bundled(const float *lors, int64_t n, int stride, const floa
     i1 = reinterpret_cast<int *>(w + 3 * b_list);
     float *zx = reinterpret_cast<float *>(w + 4 * b_list), *zy = reinterpret_cast<float *>(w + 4 * b_list + b_x);
     void *tmp = w + 4 * b_list + b_x + b_y;
-    hipLaunchKernelGGL(k_border_image, dim3((unsigned)((G.nx + 33) / 32), (unsigned)((G.nz + 33) / 32), (unsigned)(G.ny + 2)),
-                       dim3(256), 0, s, image, G.nx, G.ny, G.nz, zx, zy);
-    rc = launch_status();
+    rc = border_image(image, G, zx, zy, s);
     for (int64_t c = 0; c < n && rc == SRF_OK; c += chunk) {
         const int64_t m = n - c < chunk ? n - c : chunk;
         const float *L = lors + c * stride, *T = tof ? tofv + c * tof_stride : nullptr;
@@ -596,6 +647,48 @@ int srf_project(const float *lors, int64_t n, int64_t lor_stride, const float *t
                  <<<blocks_for(n << lg), 256, 0, s>>>(lors, n, (int)lor_stride, tof_values, (int)tof_stride, image, G,
                                                       lg, out));
     return launch_status();
+}
+
+int srf_sss_integrals(const float *det, int32_t n_det, const float *points, int32_t n_points, int32_t point_stride,
+                      const float *image, srf_grid_t grid, float *out, void *stream)
+{
+    if (n_det <= 0 || n_points <= 0 || point_stride < 3) return SRF_ERR_INVALID_ARG;
+    if (!det || !points || !image || !out) return SRF_ERR_INVALID_ARG;
+    LaunchGeom G;
+    int rc = make_geom(grid, nullptr, G);
+    if (rc) return rc;
+    const int64_t nblk = (int64_t)n_det * ((n_points + 255) / 256);
+    if (nblk >= ((int64_t)1 << 31) - 8) return SRF_ERR_UNSUPPORTED;
+    hipStream_t s = (hipStream_t)stream;
+    const bool ds = G.dy != 1.0f, dz = G.dz != 1.0f;
+    const dim3 blocks((unsigned)((nblk + 7) / 8 * 8));
+    float *zx = nullptr, *zy = nullptr;
+    // the copies pay for themselves from a few thousand rays on
+    if (nblk >= 64 && border_fits(G) && !capturing(s)) {
+        const size_t nx = (size_t)border_floats(G.nx, G.ny, G.nz), ny = (size_t)border_floats(G.ny, G.nx, G.nz);
+        zx = static_cast<float *>(pool_get((nx + ny) * sizeof(float), s));
+        if (zx) {
+            zy = zx + nx;
+            if ((rc = border_image(image, G, zx, zy, s))) {
+                pool_put(zx, s);
+                return rc;
+            }
+        }
+    }
+#define SRF_POINTS(B_, S_, Z_)                                                                                        \
+    hipLaunchKernelGGL((k_point_integrals<B_, S_, Z_>), blocks, dim3(256), 0, s, det, n_det, points, n_points,       \
+                       point_stride, image, zx, zy, G, nblk, out)
+    if (zx) {
+        if (ds) { if (dz) SRF_POINTS(true, true, true); else SRF_POINTS(true, true, false); }
+        else { if (dz) SRF_POINTS(true, false, true); else SRF_POINTS(true, false, false); }
+    } else {
+        if (ds) { if (dz) SRF_POINTS(false, true, true); else SRF_POINTS(false, true, false); }
+        else { if (dz) SRF_POINTS(false, false, true); else SRF_POINTS(false, false, false); }
+    }
+#undef SRF_POINTS
+    rc = launch_status();
+    pool_put(zx, s);
+    return rc;
 }
 
 static int backproject_impl(const float *lors, int64_t n, int64_t lor_stride, const float *tof_values,

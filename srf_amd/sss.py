@@ -230,23 +230,23 @@ class SingleScatterSimulation:
         L2 = ((lors[:, 3:6] - lors[:, 0:3]) ** 2).sum(1)
         return lors, (L2 / (self.dx_ * self.dx_)).contiguous()     # Project * L^2 / dx_^2 = integral
 
-    def _integrals(self, img_xyz, lors, to_integral, plan=None):
-        img_k = ops.to_kernel_layout(img_xyz.contiguous())
-        if plan is not None:
-            p = plan.project(img_k)
-        else:
-            p = ops.project(lors, img_k, self.shape, self.geom, False, 0.0, 0.0)
-        return (p * to_integral).reshape(self.nd, -1).contiguous()
-
     def line_integrals(self, img_xyz, pts=None):
         """(nd, ns) integrals from each detector to each point of `pts`
         ((ns, 4) or (ns, 3); default: the full grid)."""
-        img_xyz = img_xyz.to(self.dev, torch.float32)
-        if pts is None and not self.compact:
-            return self._integrals(img_xyz, self.lors, self.to_integral, self.plan)
-        xyz = self.pts_xyz if pts is None else pts[:, :3].contiguous()
-        lors, ti = self._lors(xyz)
-        return self._integrals(img_xyz, lors, ti)
+        img_k = ops.to_kernel_layout(img_xyz.to(self.dev, torch.float32).contiguous())
+        if pts is None and self.plan is not None:
+            return (self.plan.project(img_k) * self.to_integral).reshape(self.nd, -1)
+        ops._check_image(img_k, self.shape)
+        xyz = (self.pts_xyz if pts is None else pts).contiguous()
+        ns = int(xyz.shape[0])
+        out = torch.empty((self.nd, ns), dtype=torch.float32, device=self.dev)
+        if ns == 0:
+            return out
+        with torch.cuda.device(self.dev):
+            check(lib().srf_sss_integrals(self.det.data_ptr(), self.nd, xyz.data_ptr(), ns, int(xyz.shape[1]),
+                                          img_k.data_ptr(), ops._grid(self.shape, self.geom), out.data_ptr(),
+                                          stream_handle(self.dev)), "srf_sss_integrals")
+        return out
 
     def points(self, mu_xyz):
         mu = mu_xyz.detach().to(self.dev, torch.float32).reshape(-1)[self.pts_flat]

@@ -9,11 +9,10 @@
 // holds
 //   k_sss_pairs   per (detector, scatter point): unit vector S->D, the
 //                 obliquity / distance factor g = ((D-S).n_D)/|D-S|^3, and the
-//                 emission and attenuation integrals packed as one 32-byte row;
+//                 emission and attenuation integrals, in the order the bin sum
+//                 reads them (RowLayout);
 //   k_sss_bins    per sinogram bin: the sum over scatter points, one bin per
-//                 lane.  Bins are ordered by ring and detector A, so the lanes
-//                 of a wavefront share A's row (a broadcast read) and stream B's.
-//   k_sss_bins_wave  the same with one wavefront per bin (small sinograms).
+//                 lane, the points split over wavefronts and workgroups.
 // Energy-dependent factors depend only on the integer scattering angle
 // (the reference quantises it to whole degrees, kn_formula.py:41), so E', the
 // window efficiency and the KN factor are 181-entry tables.
@@ -26,118 +25,190 @@
 
 namespace srf {
 
-struct __align__(16) PairRow {
-    float ux, uy, uz, g;    // unit vector S -> D, obliquity / |D-S|^2 factor
-    float em, mu, pad0, pad1;
+// The rows of the (detector, point) table: 24 bytes each, as 16 (unit vector, g) and
+// 8 (emission integral, attenuation integral times log2 e), point groups of GS
+// outermost, then the detector, then the point within its group: a lane's 4 points
+// of one detector are 64 + 32 consecutive bytes, whether its neighbours read
+// neighbouring detectors (a ring sinogram) or any (counted crystal pairs).
+// 131072 bins of 2e4 points, 4096 detectors: 4.8 ms, VALU bound (about 61 issue
+// cycles a pair); one point per group 6.0 ms (rows 64 KiB apart) and 1.8 instead of
+// 0.7 ms to write them.  Detector-major rows with acosf per pair and one bin per
+// lane over all points, as before: 14.2 ms.
+template <int GS>
+struct RowLayout {
+    int64_t nd;
+    int ns;
+    __host__ __device__ int64_t padded() const { return nd * ((ns + GS - 1) / GS * GS); }
+    __device__ __forceinline__ int64_t at(int64_t d, int s) const { return ((int64_t)(s / GS) * nd + d) * GS + s % GS; }
 };
 
+// Points per group: 4, or 1 where rounding ns up to 4 would outgrow the workspace (32
+// bytes per pair).
+constexpr int SSS_GROUP = 4;
+static bool grouped_rows(int n_points) { return n_points >= 16; }
+
 // det: (nd, 4) x, y, z, normal angle; sp: (ns, 4) x, y, z, mu(S);
-// em, mu: (nd, ns) line integrals (row-major by detector).
+// em, mu: (nd, ns) line integrals (row-major by detector).  A workgroup takes 64
+// points of 4 detectors; points past ns fill their group with zero rows.
+template <int GS>
 __global__ __launch_bounds__(256) void k_sss_pairs(const float *__restrict__ det, const float *__restrict__ sp,
                                                    const float *__restrict__ em, const float *__restrict__ mu,
-                                                   int nd, int ns, PairRow *__restrict__ rows)
+                                                   int nd, int ns, float4 *__restrict__ dir, float2 *__restrict__ val)
 {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= (int64_t)nd * ns) return;
-    const int d = (int)(i / ns), s = (int)(i % ns);
-    const float vx = det[4 * d] - sp[4 * s], vy = det[4 * d + 1] - sp[4 * s + 1], vz = det[4 * d + 2] - sp[4 * s + 2];
-    const float r2 = vx * vx + vy * vy + vz * vz;
-    const float r = sqrtf(r2);
-    const float inv = 1.0f / r;
-    const float a = det[4 * d + 3];
-    PairRow R;
-    R.ux = vx * inv;
-    R.uy = vy * inv;
-    R.uz = vz * inv;
-    R.g = (vx * cosf(a) + vy * sinf(a)) * inv / r2;
-    R.em = em[i];
-    R.mu = mu[i];
-    R.pad0 = R.pad1 = 0.0f;
-    rows[i] = R;
+    const int nsb = (ns + 63) / 64;
+    const int s = blockIdx.x % nsb * 64 + (threadIdx.x & 63), d = blockIdx.x / nsb * 4 + (threadIdx.x >> 6);
+    if (d >= nd || s >= (ns + GS - 1) / GS * GS) return;
+    const RowLayout<GS> R{nd, ns};
+    float4 u = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float2 v = make_float2(0.0f, 0.0f);
+    if (s < ns) {
+        const float vx = det[4 * d] - sp[4 * s], vy = det[4 * d + 1] - sp[4 * s + 1], vz = det[4 * d + 2] - sp[4 * s + 2];
+        const float r2 = vx * vx + vy * vy + vz * vz;
+        const float inv = 1.0f / sqrtf(r2);
+        const float a = det[4 * d + 3];
+        const int64_t i = (int64_t)d * ns + s;
+        u = make_float4(vx * inv, vy * inv, vz * inv, (vx * cosf(a) + vy * sinf(a)) * inv / r2);
+        v = make_float2(em[i], mu[i] * 1.44269504f);
+    }
+    dir[R.at(d, s)] = u;
+    val[R.at(d, s)] = v;
+}
+
+// The whole-degree scattering angle k = (int)(acos(x) 180 / pi) of a pair
+// (kn_formula.py:41) from two small tables instead of acosf: t = sqrt(1 - |x|) is
+// nearly linear in the angle (0.0087 to 0.0123 per degree), so a cell of 1/256 in t
+// holds at most one whole degree.  A cell stores the float x below which the angle
+// has passed that degree, found with acosf itself, and the smaller angle.
+constexpr int DEG_CELLS = 257;
+
+constexpr int BINS_WG = 1024;
+
+struct DegTable {
+    float2 cell[2 * DEG_CELLS];   // x >= 0, then x < 0: threshold in x, angle index (as bits)
+    float2 fac[181 + 1];          // 511 / E', window efficiency times KN / sigma_KN
+};
+
+__device__ __forceinline__ int degrees_of(float x)
+{
+    return min((int)(acosf(fminf(1.0f, fmaxf(-1.0f, x))) * 57.295779513082323f), 180);
 }
 
 // tables: [0,181) 511/E', [181,362) window efficiency, [362,543) KN / sigma_KN
-__global__ __launch_bounds__(256) void k_sss_bins(const PairRow *__restrict__ rows, const float *__restrict__ sp,
-                                                  int nd, int ns, const int *__restrict__ bins, int nb,
-                                                  const float *__restrict__ tables, float scale,
+__device__ __forceinline__ void build_degrees(DegTable &T, float *thr, const float *__restrict__ tables)
+{
+    // thr[k], 1 <= k <= 180: the angle is at least k for x below it (to 1e-9, from
+    // a bracket of 8e-6 about cos k)
+    for (int k = threadIdx.x; k <= 180; k += BINS_WG) {
+        const float c = cosf((float)k * 0.017453292519943295f);
+        float lo = c - 4e-6f, hi = c + 4e-6f;
+        for (int i = 0; i < 13; ++i) {
+            const float m = 0.5f * (lo + hi);
+            if (degrees_of(m) >= k) lo = m;
+            else hi = m;
+        }
+        thr[k] = hi;
+        T.fac[k] = make_float2(tables[k], tables[181 + k] * tables[362 + k]);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 2 * DEG_CELLS; i += BINS_WG) {
+        const bool neg = i >= DEG_CELLS;
+        const float t0 = (float)(i - (neg ? DEG_CELLS : 0)) / 256.0f, t1 = t0 + 1.0f / 256.0f;
+        const float m0 = 1.0f - t0 * t0, m1 = fmaxf(0.0f, 1.0f - t1 * t1);
+        // the smaller angle of the cell, and the degree it passes (if any)
+        const int k0 = degrees_of(neg ? -m1 : m0), k1 = degrees_of(neg ? -m0 : m1);
+        T.cell[i] = make_float2(k1 > k0 ? thr[k0 + 1] : -2.0f, __int_as_float(k0));
+    }
+    __syncthreads();
+}
+
+// One pair of rows: g g' eff KN (I_a + I_b) at the angle between the two unit vectors.
+__device__ __forceinline__ float pair_term(const DegTable &T, const float4 ua, const float4 ub, const float2 va,
+                                           const float2 vb)
+{
+    // scattering angle = pi - angle(A S B) (law of cosines, kn_formula.py:36-41)
+    const float x = -fmaf(ua.x, ub.x, fmaf(ua.y, ub.y, ua.z * ub.z));
+    const float t = __builtin_amdgcn_sqrtf(fminf(fmaxf(1.0f - fabsf(x), 0.0f), 1.0f));
+    const int ci = (int)(t * 256.0f) + (x < 0.0f ? DEG_CELLS : 0);
+    const float2 c = T.cell[ci];
+    const float2 f = T.fac[__float_as_int(c.y) + (x < c.x ? 1 : 0)];
+    const float Ia = __builtin_amdgcn_exp2f(-fmaf(vb.y, f.x, va.y)) * va.x;
+    const float Ib = __builtin_amdgcn_exp2f(-fmaf(va.y, f.x, vb.y)) * vb.x;
+    return ua.w * ub.w * f.y * (Ia + Ib);
+}
+
+// One bin per lane, BINS_WG consecutive bins per workgroup, part p of the points per
+// workgroup (., p).  The wavefronts of a workgroup walk the same points side by
+// side: the bins of neighbouring angles use mostly the same detectors, whose rows
+// then come from L1 (64 bins per workgroup and a quarter of the points per wavefront
+// instead: 5.9 ms, each row read from L2 26 times).  The parts are summed by
+// k_sss_sum in order; parts == 1 writes the sinogram itself.
+template <int GS>
+__global__ __launch_bounds__(BINS_WG) void k_sss_bins(const float4 *__restrict__ dir, const float2 *__restrict__ val,
+                                                  const float *__restrict__ sp, int nd, int ns,
+                                                  const int *__restrict__ bins, int nb,
+                                                  const float *__restrict__ tables, float scale, int parts,
                                                   float *__restrict__ out)
 {
-    __shared__ float tab[543];
-    for (int i = threadIdx.x; i < 543; i += 256) tab[i] = tables[i];
-    __syncthreads();
+    __shared__ DegTable T;
+    __shared__ float thr[181];
+    build_degrees(T, thr, tables);
+    const int b = blockIdx.x * BINS_WG + threadIdx.x;
+    const bool in = b < nb;
+    const int da = in ? bins[2 * b] : 0, db = in ? bins[2 * b + 1] : 0;
+    const bool ok = da >= 0 && da < nd && db >= 0 && db < nd;
+    // byte offsets of the detectors' rows in a point group
+    const unsigned oa = ok ? (unsigned)da * (16u * GS) : 0u, ob = ok ? (unsigned)db * (16u * GS) : 0u;
+    // four points per trip: their 16 loads are in flight together
+    constexpr int U = 4;
+    const int ng = (ns + U - 1) / U, per = (ng + parts - 1) / parts;
+    const int g0 = (int)blockIdx.y * per, g1 = min(ng, g0 + per);
+    float acc = 0.0f;
+    for (int g = g0; g < g1; ++g) {
+        float m[U];
+        bool any = false;
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            m[j] = U * g + j < ns ? sp[4 * (U * g + j) + 3] : 0.0f;
+            any |= m[j] != 0.0f;
+        }
+        if (!any) continue;   // the kn term is proportional to mu(S) (kn_formula.py:16)
+        float4 ua[U], ub[U];
+        float2 va[U], vb[U];
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            // (GS == 1 has no padding rows)
+            const int64_t row = (int64_t)(GS == 1 ? min(U * g + j, ns - 1) : U * g) * nd;
+            const char *D = reinterpret_cast<const char *>(dir + row), *V = reinterpret_cast<const char *>(val + row);
+            const int k = GS == 1 ? 0 : j;
+            ua[j] = *reinterpret_cast<const float4 *>(D + oa + 16 * k);
+            ub[j] = *reinterpret_cast<const float4 *>(D + ob + 16 * k);
+            va[j] = *reinterpret_cast<const float2 *>(V + (oa >> 1) + 8 * k);
+            vb[j] = *reinterpret_cast<const float2 *>(V + (ob >> 1) + 8 * k);
+        }
+        float sum = 0.0f;
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            const float t = fmaf(m[j], pair_term(T, ua[j], ub[j], va[j], vb[j]), sum);
+            sum = m[j] == 0.0f ? sum : t;
+        }
+        acc += sum;
+    }
+    if (!in) return;
+    // a detector index outside the table gives NaN
+    if (!ok) acc = __builtin_nanf("");
+    if (parts == 1) out[b] = acc * scale;
+    else out[(int64_t)blockIdx.y * nb + b] = acc;
+}
+
+__global__ __launch_bounds__(256) void k_sss_sum(const float *__restrict__ part, int parts, int nb, float scale,
+                                                 float *__restrict__ out)
+{
     const int b = blockIdx.x * 256 + threadIdx.x;
     if (b >= nb) return;
-    const int da = bins[2 * b], db = bins[2 * b + 1];
-    if (da < 0 || da >= nd || db < 0 || db >= nd) {   // detector index outside the table
-        out[b] = __builtin_nanf("");
-        return;
-    }
-    const PairRow *ra = rows + (int64_t)da * ns;
-    const PairRow *rb = rows + (int64_t)db * ns;
     float acc = 0.0f;
-    for (int s = 0; s < ns; ++s) {
-        const float m = sp[4 * s + 3];
-        if (m == 0.0f) continue;   // kn term is proportional to mu(S) (kn_formula.py:16)
-        const PairRow A = ra[s], B = rb[s];
-        // scattering angle = pi - angle(A S B) (law of cosines, kn_formula.py:36-41)
-        const float x = -(A.ux * B.ux + A.uy * B.uy + A.uz * B.uz);
-        int k = (int)(acosf(fminf(1.0f, fmaxf(-1.0f, x))) * 57.295779513082323f);
-        k = min(k, 180);
-        const float rr = tab[k];
-        const float Ia = __expf(-(A.mu + B.mu * rr)) * A.em;
-        const float Ib = __expf(-(A.mu * rr + B.mu)) * B.em;
-        acc += A.g * B.g * tab[181 + k] * tab[362 + k] * m * (Ia + Ib);
-    }
+    for (int p = 0; p < parts; ++p) acc += part[(int64_t)p * nb + b];
     out[b] = acc * scale;
 }
-
-// The same sum with one wavefront per bin, for sinograms too small to fill
-// the GPU one bin per lane (a few rings: a check subset).  Lane j takes the
-// points s = j, j + 64, ...; the A and B rows are then read contiguously.
-// The 64 partial sums are combined by a fixed butterfly, so the result is
-// deterministic (it differs from the serial order of k_sss_bins only by
-// float rounding).
-constexpr int SSS_WAVE = 64;
-
-__global__ __launch_bounds__(256) void k_sss_bins_wave(const PairRow *__restrict__ rows,
-                                                       const float *__restrict__ sp, int nd, int ns,
-                                                       const int *__restrict__ bins, int nb,
-                                                       const float *__restrict__ tables, float scale,
-                                                       float *__restrict__ out)
-{
-    __shared__ float tab[543];
-    for (int i = threadIdx.x; i < 543; i += 256) tab[i] = tables[i];
-    __syncthreads();
-    const int b = blockIdx.x * (256 / SSS_WAVE) + (int)(threadIdx.x / SSS_WAVE);
-    const int lane = (int)(threadIdx.x % SSS_WAVE);
-    if (b >= nb) return;   // whole wavefronts leave together
-    const int da = bins[2 * b], db = bins[2 * b + 1];
-    if (da < 0 || da >= nd || db < 0 || db >= nd) {
-        if (lane == 0) out[b] = __builtin_nanf("");
-        return;
-    }
-    const PairRow *ra = rows + (int64_t)da * ns;
-    const PairRow *rb = rows + (int64_t)db * ns;
-    float acc = 0.0f;
-    for (int s = lane; s < ns; s += SSS_WAVE) {
-        const float m = sp[4 * s + 3];
-        if (m == 0.0f) continue;
-        const PairRow A = ra[s], B = rb[s];
-        const float x = -(A.ux * B.ux + A.uy * B.uy + A.uz * B.uz);
-        int k = (int)(acosf(fminf(1.0f, fmaxf(-1.0f, x))) * 57.295779513082323f);
-        k = min(k, 180);
-        const float rr = tab[k];
-        const float Ia = __expf(-(A.mu + B.mu * rr)) * A.em;
-        const float Ib = __expf(-(A.mu * rr + B.mu)) * B.em;
-        acc += A.g * B.g * tab[181 + k] * tab[362 + k] * m * (Ia + Ib);
-    }
-#pragma unroll
-    for (int off = SSS_WAVE / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, SSS_WAVE);
-    if (lane == 0) out[b] = acc * scale;
-}
-
-// Sinograms below this many bins use k_sss_bins_wave.
-constexpr int SSS_WAVE_BINS = 32768;
 
 // work[0] += sum_e sino[bins[e]], work[1] += sum_e y[e] (double, one atomic per block)
 __device__ __forceinline__ float bin_value(const float *__restrict__ sino, const int32_t *__restrict__ bins,
@@ -204,7 +275,7 @@ extern "C" {
 size_t srf_sss_rows_bytes(int32_t n_det, int32_t n_points)
 {
     if (n_det <= 0 || n_points <= 0) return 0;
-    return (size_t)n_det * (size_t)n_points * sizeof(PairRow);
+    return (size_t)n_det * (size_t)n_points * 32;
 }
 
 int srf_sss_prepare(const float *det, int32_t n_det, const float *points, int32_t n_points, const float *em_int,
@@ -214,9 +285,19 @@ int srf_sss_prepare(const float *det, int32_t n_det, const float *points, int32_
     if (!det || !points || !em_int || !mu_int || !rows) return SRF_ERR_INVALID_ARG;
     if (rows_bytes < srf_sss_rows_bytes(n_det, n_points)) return SRF_ERR_WORKSPACE;
     if ((reinterpret_cast<uintptr_t>(rows) & 15) != 0) return SRF_ERR_INVALID_ARG;
-    const int64_t n = (int64_t)n_det * n_points;
-    hipLaunchKernelGGL(k_sss_pairs, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, det,
-                       points, em_int, mu_int, n_det, n_points, (PairRow *)rows);
+    const int64_t nblk = (int64_t)((n_points + 63) / 64) * ((n_det + 3) / 4);
+    if (nblk >= (int64_t)1 << 31) return SRF_ERR_UNSUPPORTED;   // 16 TiB of rows
+    const dim3 grid((unsigned)nblk);
+    float4 *dir = (float4 *)rows;
+    if (grouped_rows(n_points)) {
+        const RowLayout<SSS_GROUP> R{n_det, n_points};
+        hipLaunchKernelGGL(k_sss_pairs<SSS_GROUP>, grid, dim3(256), 0, (hipStream_t)stream, det, points, em_int, mu_int,
+                           n_det, n_points, dir, (float2 *)(dir + R.padded()));
+    } else {
+        const RowLayout<1> R{n_det, n_points};
+        hipLaunchKernelGGL(k_sss_pairs<1>, grid, dim3(256), 0, (hipStream_t)stream, det, points, em_int, mu_int, n_det,
+                           n_points, dir, (float2 *)(dir + R.padded()));
+    }
     return launch_status();
 }
 
@@ -226,16 +307,41 @@ int srf_sss_sinogram(const void *rows, int32_t n_det, const float *points, int32
     if (n_bins < 0 || n_det <= 0 || n_points <= 0) return SRF_ERR_INVALID_ARG;
     if (n_bins == 0) return SRF_OK;
     if (!rows || !points || !bins || !tables || !out) return SRF_ERR_INVALID_ARG;
-    if (n_bins < SSS_WAVE_BINS) {
-        constexpr int per_block = 256 / SSS_WAVE;
-        hipLaunchKernelGGL(k_sss_bins_wave, dim3((unsigned)((n_bins + per_block - 1) / per_block)), dim3(256), 0,
-                           (hipStream_t)stream, (const PairRow *)rows, points, n_det, n_points, bins, n_bins, tables,
-                           scale, out);
-    } else {
-        hipLaunchKernelGGL(k_sss_bins, dim3((unsigned)((n_bins + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
-                           (const PairRow *)rows, points, n_det, n_points, bins, n_bins, tables, scale, out);
+    hipStream_t s = (hipStream_t)stream;
+    const int nblk = (n_bins + BINS_WG - 1) / BINS_WG;
+    // parts of the points: two rounds of workgroups on the chip, each part with at
+    // least 64 points
+    int parts = (1024 + nblk - 1) / nblk;
+    if (parts > n_points / 64) parts = n_points / 64;
+    if (parts > 256) parts = 256;
+    if (parts < 1) parts = 1;
+    float *part = nullptr;
+    if (parts > 1) {
+        part = capturing(s) ? nullptr : static_cast<float *>(pool_get((size_t)parts * n_bins * sizeof(float), s));
+        if (!part) parts = 1;
     }
-    return launch_status();
+    const float4 *dir = (const float4 *)rows;
+    const dim3 grid((unsigned)nblk, (unsigned)parts);
+    float *dst = part ? part : out;
+    if (grouped_rows(n_points)) {
+        const RowLayout<SSS_GROUP> R{n_det, n_points};
+        hipLaunchKernelGGL(k_sss_bins<SSS_GROUP>, grid, dim3(BINS_WG), 0, s, dir, (const float2 *)(dir + R.padded()), points,
+                           n_det, n_points, bins, n_bins, tables, scale, parts, dst);
+    } else {
+        const RowLayout<1> R{n_det, n_points};
+        hipLaunchKernelGGL(k_sss_bins<1>, grid, dim3(BINS_WG), 0, s, dir, (const float2 *)(dir + R.padded()), points, n_det,
+                           n_points, bins, n_bins, tables, scale, parts, dst);
+    }
+    int rc = launch_status();
+    if (part) {
+        if (rc == SRF_OK) {
+            hipLaunchKernelGGL(k_sss_sum, dim3((unsigned)((n_bins + 255) / 256)), dim3(256), 0, s, part, parts, n_bins,
+                               scale, out);
+            rc = launch_status();
+        }
+        pool_put(part, s);
+    }
+    return rc;
 }
 
 int srf_scatter_correct(const float *y, const float *weight, const int32_t *bins, const float *sino, int64_t n_bins,

@@ -180,42 +180,54 @@ __device__ __forceinline__ float branch_weight(const Branch &B, const RaySetup &
     return W;
 }
 
-// Interval of primary coordinate x on which value(x) = (c + k*(x - p1))/d + n2
-// lies in [lo_v, hi_v]; empty => a > b.
-__device__ __forceinline__ void axis_window(double c, double k, double p1, double d, double n2, double lo_v,
-                                            double hi_v, double &a, double &b)
+// Margin in cells for a coordinate (c + k (x - p1)) / d + n2 over |x| <= np2: a
+// hundredth of a cell and 8 float ulps of its largest intermediate value, above the
+// rounding of both the float estimates below and the marcher's own coordinates.
+__device__ __forceinline__ float cell_margin(float c, float k, float p1, float np2, float d, float n2)
 {
-    if (k == 0.0) {
-        double v = c / d + n2;
-        if (v >= lo_v && v <= hi_v) { a = -1e30; b = 1e30; }
-        else { a = 1e30; b = -1e30; }
+    return 1e-2f + 1e-6f * ((fabsf(c) + fabsf(k) * (np2 + fabsf(p1))) / d + n2);
+}
+
+// Interval of primary coordinate x on which value(x) = (c + k*(x - p1))/d + n2
+// lies in [lo_v, hi_v] (a margin wider than exact, see cell_margin); empty => a > b.
+__device__ __forceinline__ void axis_window(float c, float k, float p1, float d, float n2, float lo_v, float hi_v,
+                                            float &a, float &b)
+{
+    if (k == 0.0f) {
+        const float v = c / d + n2;
+        if (v >= lo_v && v <= hi_v) { a = -1e30f; b = 1e30f; }
+        else { a = 1e30f; b = -1e30f; }
     } else {
-        double xa = p1 + ((lo_v - n2) * d - c) / k;
-        double xb = p1 + ((hi_v - n2) * d - c) / k;
-        a = fmin(xa, xb);
-        b = fmax(xa, xb);
+        const float xa = p1 + ((lo_v - n2) * d - c) / k;
+        const float xb = p1 + ((hi_v - n2) * d - c) / k;
+        a = fminf(xa, xb);
+        b = fmaxf(xa, xb);
     }
 }
 
 // Slabs [lo, hi) that can hold a term: the secondary and axial coordinates of
-// a slab must reach [-1, n] (widened by a margin far above float round-off, and
-// by one slab on each side).
+// a slab must reach [-1, n] (widened by the margin, and by one slab on each side).
 __device__ __forceinline__ void clip_range(const Branch &B, const RaySetup &r, const LaunchGeom &G, int &lo, int &hi)
 {
-    const double m = 0.01;
-    double sa, sb, za, zb;
-    axis_window((double)B.sec1, (double)B.ks, (double)B.p1, (double)B.ds, (double)B.ns2, -1.0 - m,
-                (double)B.ns + m, sa, sb);
-    axis_window((double)r.z1, (double)B.kz, (double)B.p1, (double)G.dz, (double)G.nz2, -1.0 - m,
-                (double)G.nz + m, za, zb);
-    const double xl = fmax(fmax(-(double)B.np2, sa - 1.0), za - 1.0);
-    const double xh = fmin(fmin((double)B.np2, sb + 1.0), zb + 1.0);
-    if (xl > xh) {
+    const float ms = cell_margin(B.sec1, B.ks, B.p1, B.np2, B.ds, B.ns2);
+    const float mz = cell_margin(r.z1, B.kz, B.p1, B.np2, G.dz, G.nz2);
+    float sa, sb, za, zb;
+    axis_window(B.sec1, B.ks, B.p1, B.ds, B.ns2, -1.0f - ms, (float)B.ns + ms, sa, sb);
+    axis_window(r.z1, B.kz, B.p1, G.dz, G.nz2, -1.0f - mz, (float)G.nz + mz, za, zb);
+    const float xl = fmaxf(fmaxf(-B.np2, sa - 1.0f), za - 1.0f);
+    const float xh = fminf(fminf(B.np2, sb + 1.0f), zb + 1.0f);
+    if (!(xl <= xh)) {
         lo = 0; hi = 0;
     } else {
-        lo = max(0, (int)floor(xl + (double)B.np2) - 1);
-        hi = min(B.np, (int)ceil(xh + (double)B.np2) + 1);
+        lo = max(0, (int)floorf(xl + B.np2) - 1);
+        hi = min(B.np, (int)ceilf(xh + B.np2) + 1);
     }
+}
+
+// (int) of a float clamped far inside the int range.
+__device__ __forceinline__ int flt_to_int(float v)
+{
+    return (int)fminf(fmaxf(v, -1.0e9f), 1.0e9f);
 }
 
 // (int) of a double clamped far inside the int range.
@@ -249,28 +261,28 @@ __device__ __forceinline__ void fp_cut_range(const Branch &B, int lo, int hi, in
         // siddon.cu.cc:56-57 / 203-204: skip (p1<p2 && pp2>p2) || (p1>=p2 && pp1<p2)
         if (p1 < p2) {
             auto cut = [&](int ip) { return ((float)ip - np2) + 1.0f > p2; };
-            b = first_true(cut, lo, hi, dbl_to_int(floor((double)p2 + (double)np2)));
+            b = first_true(cut, lo, hi, flt_to_int(floorf(p2 + np2)));
         } else {
             auto keep = [&](int ip) { return (float)ip - np2 >= p2; };
-            a = first_true(keep, lo, hi, dbl_to_int(ceil((double)p2 + (double)np2)));
+            a = first_true(keep, lo, hi, flt_to_int(ceilf(p2 + np2)));
         }
     } else if (B.xdom) {
         // siddon_tof.cu.cc:67-74: skip (p2>p1 && pp1<=p1) || (p2<p1 && pp2>=p1)
         if (p2 > p1) {
             auto keep = [&](int ip) { return (float)ip - np2 > p1; };
-            a = first_true(keep, lo, hi, dbl_to_int(floor((double)p1 + (double)np2)) + 1);
+            a = first_true(keep, lo, hi, flt_to_int(floorf(p1 + np2)) + 1);
         } else if (p2 < p1) {
             auto cut = [&](int ip) { return ((float)ip - np2) + 1.0f >= p1; };
-            b = first_true(cut, lo, hi, dbl_to_int(ceil((double)p1 + (double)np2)) - 1);
+            b = first_true(cut, lo, hi, flt_to_int(ceilf(p1 + np2)) - 1);
         }
     } else {
         // siddon_tof.cu.cc:228-235: skip (p2>p1 && pp1<p1) || (p2<p1 && pp2>p1)
         if (p2 > p1) {
             auto keep = [&](int ip) { return (float)ip - np2 >= p1; };
-            a = first_true(keep, lo, hi, dbl_to_int(ceil((double)p1 + (double)np2)));
+            a = first_true(keep, lo, hi, flt_to_int(ceilf(p1 + np2)));
         } else if (p2 < p1) {
             auto cut = [&](int ip) { return ((float)ip - np2) + 1.0f > p1; };
-            b = first_true(cut, lo, hi, dbl_to_int(floor((double)p1 + (double)np2)));
+            b = first_true(cut, lo, hi, flt_to_int(floorf(p1 + np2)));
         }
     }
     if (b < a) b = a;

@@ -13,10 +13,10 @@
 // Binning (once per event list, reused by every iteration and both directions):
 //   k_bin_count  segments per event and per (tile, length class) key
 //   scan         event offsets (hipcub) and key offsets (host, <= 16384 keys)
-//   k_bin_emit   48-byte segment records, grouped by key: records of one tile
-//                are contiguous and sorted into slab-count classes, then (radix
-//                sort) by branch and slab count, so a wavefront runs one
-//                branch's marcher over similar lengths.
+//   k_bin_emit   sort key and (event, first slab, ordinal) per segment, in event order
+//   radix sort   by tile, slab-count class, branch and slab count, so a wavefront
+//                runs one branch's marcher over similar lengths
+//   k_bin_records  the 48-byte segment records in that order, from the events' LORs
 // A record carries everything the marcher needs (the event's exact branch
 // parameters), so the passes stream records instead of gathering event data.
 //
@@ -101,7 +101,8 @@ struct SegCtx {
     int fa, fb;            // projector's exact cut range on this branch
 };
 
-// Calls f(tile, cls, a, b) for every segment of slabs [lo, hi) of branch B.
+// Calls f(tile, a, b) for every segment of slabs [lo, hi) of branch B: a segment lies in
+// one tile column along the primary axis, so it has at most 32 slabs.
 template <class F>
 __device__ __forceinline__ void for_each_segment(const Branch &B, const RaySetup &r, const LaunchGeom &G,
                                                  const TileCfg &T, int lo, int hi, F &&f)
@@ -109,40 +110,35 @@ __device__ __forceinline__ void for_each_segment(const Branch &B, const RaySetup
     const int TP = B.xdom ? TX : TY;
     const int TS = B.xdom ? TY : TX;
     const int nts = B.xdom ? T.nty : T.ntx;
-    const double eps = 1e-2;
-    const double p1 = B.p1, np2 = B.np2;
+    const float p1 = B.p1, np2 = B.np2;
+    const float es = cell_margin(B.sec1, B.ks, p1, np2, B.ds, B.ns2), ez = cell_margin(r.z1, B.kz, p1, np2, G.dz, G.nz2);
     for (int c = lo / TP; c * TP < hi; ++c) {
         const int ca = max(lo, c * TP), cb = min(hi, (c + 1) * TP);
         if (ca >= cb) continue;
-        const double xa = (double)ca - np2, xb = (double)cb - np2;
-        const double Sa = ((double)B.sec1 + (double)B.ks * (xa - p1)) / (double)B.ds + (double)B.ns2;
-        const double Sb = ((double)B.sec1 + (double)B.ks * (xb - p1)) / (double)B.ds + (double)B.ns2;
-        const double Za = ((double)r.z1 + (double)B.kz * (xa - p1)) / (double)G.dz + (double)G.nz2;
-        const double Zb = ((double)r.z1 + (double)B.kz * (xb - p1)) / (double)G.dz + (double)G.nz2;
-        const int ts0 = max(0, dbl_to_int(floor((fmin(Sa, Sb) - eps) / TS)));
-        const int ts1 = min(nts - 1, dbl_to_int(floor((fmax(Sa, Sb) + eps) / TS)));
-        const int tz0 = max(0, dbl_to_int(floor((fmin(Za, Zb) - eps) / TZ)));
-        const int tz1 = min(T.ntz - 1, dbl_to_int(floor((fmax(Za, Zb) + eps) / TZ)));
+        const float xa = (float)ca - np2, xb = (float)cb - np2;
+        const float Sa = (B.sec1 + B.ks * (xa - p1)) / B.ds + B.ns2, Sb = (B.sec1 + B.ks * (xb - p1)) / B.ds + B.ns2;
+        const float Za = (r.z1 + B.kz * (xa - p1)) / G.dz + G.nz2, Zb = (r.z1 + B.kz * (xb - p1)) / G.dz + G.nz2;
+        const int ts0 = max(0, flt_to_int(floorf((fminf(Sa, Sb) - es) / TS)));
+        const int ts1 = min(nts - 1, flt_to_int(floorf((fmaxf(Sa, Sb) + es) / TS)));
+        const int tz0 = max(0, flt_to_int(floorf((fminf(Za, Zb) - ez) / TZ)));
+        const int tz1 = min(T.ntz - 1, flt_to_int(floorf((fmaxf(Za, Zb) + ez) / TZ)));
         for (int ts = ts0; ts <= ts1; ++ts) {
-            double wa, wb;
-            axis_window((double)B.sec1, (double)B.ks, p1, (double)B.ds, (double)B.ns2, (double)(ts * TS) - eps,
-                        (double)((ts + 1) * TS) + eps, wa, wb);
+            float wa, wb;
+            axis_window(B.sec1, B.ks, p1, B.ds, B.ns2, (float)(ts * TS) - es, (float)((ts + 1) * TS) + es, wa, wb);
             if (wa > wb) continue;
             // slabs [ip - np2, ip - np2 + 1] meeting [wa, wb]
-            const int sa = max(ca, dbl_to_int(ceil(wa + np2)) - 1);
-            const int sb = min(cb, dbl_to_int(floor(wb + np2)) + 1);
+            const int sa = max(ca, flt_to_int(ceilf(wa + np2)) - 1);
+            const int sb = min(cb, flt_to_int(floorf(wb + np2)) + 1);
             if (sa >= sb) continue;
             for (int tz = tz0; tz <= tz1; ++tz) {
-                double za, zb;
-                axis_window((double)r.z1, (double)B.kz, p1, (double)G.dz, (double)G.nz2, (double)(tz * TZ) - eps,
-                            (double)((tz + 1) * TZ) + eps, za, zb);
+                float za, zb;
+                axis_window(r.z1, B.kz, p1, G.dz, G.nz2, (float)(tz * TZ) - ez, (float)((tz + 1) * TZ) + ez, za, zb);
                 if (za > zb) continue;
-                const int a = max(sa, dbl_to_int(ceil(za + np2)) - 1);
-                const int b = min(sb, dbl_to_int(floor(zb + np2)) + 1);
+                const int a = max(sa, flt_to_int(ceilf(za + np2)) - 1);
+                const int b = min(sb, flt_to_int(floorf(zb + np2)) + 1);
                 if (a >= b) continue;
                 const int tile = B.xdom ? c + T.ntx * (ts + T.nty * tz) : ts + T.ntx * (c + T.nty * tz);
-                const int cls = min(NCLASS - 1, ((b - a - 1) * NCLASS) / TP);
-                f(tile, cls, a, b);
+                f(tile, a, b);
             }
         }
     }
@@ -176,7 +172,7 @@ __device__ __forceinline__ void tof_window(const Branch &B, const RaySetup &r, c
     hi = min(hi, dbl_to_int(floor(fmax(u1, u2) + np2)) + 2);
 }
 
-// Every segment of one event: f(tile, cls, a, b, Branch, SegCtx).  Non-TOF
+// Every segment of one event: f(tile, a, b, Branch, SegCtx).  Non-TOF
 // ties (|xd| == |yd|) march different branches in the projector (>=,
 // siddon.cu.cc:46) and the backprojector (>, :372): both are binned, each
 // marked for its own direction.
@@ -211,7 +207,7 @@ __device__ __forceinline__ void for_each_event_segment(const RaySetup &r, const 
         tof_window<TOF>(B, r, G, twin, lo, hi);
         tof_window<TOF>(B, r, G, twin, ctx.fa, ctx.fb);
         int elo = ctx.bp_use ? lo : ctx.fa, ehi = ctx.bp_use ? hi : ctx.fb;
-        for_each_segment(B, r, G, T, elo, ehi, [&](int tile, int cls, int a, int b) { f(tile, cls, a, b, B, ctx); });
+        for_each_segment(B, r, G, T, elo, ehi, [&](int tile, int a, int b) { f(tile, a, b, B, ctx); });
     }
 }
 
@@ -224,12 +220,27 @@ __device__ __forceinline__ int ab_a(uint32_t ab) { return (int)(ab & 0x7fffu); }
 __device__ __forceinline__ int ab_b(uint32_t ab) { return (int)(ab >> 16); }
 __device__ __forceinline__ bool ab_xd(uint32_t ab) { return (ab >> 15) & 1u; }
 
+// Sort key of a segment: (tile, slab-count class), then the branch (a wavefront
+// mostly runs one branch's marcher), then slab count (longest first: its lanes march
+// similar lengths).  A stable sort keeps slot order within a key.
+constexpr int CLASS_SLABS = 32 / NCLASS;   // slab counts per class
+constexpr int SUB_BITS = 4;                // branch, slab count within the class
+static_assert(TX == 32 && TY == 32 && CLASS_SLABS == 8, "segments of 1 to 32 slabs, 3 bits of slab count per class");
+
+__device__ __forceinline__ unsigned seg_class(int tile, int len) { return (unsigned)(tile * NCLASS + (len - 1) / CLASS_SLABS); }
+__device__ __forceinline__ unsigned seg_key(int tile, int len, bool xdom)
+{
+    return (seg_class(tile, len) << SUB_BITS) | ((unsigned)xdom << 3) | (7u - (unsigned)((len - 1) % CLASS_SLABS));
+}
+
+// Segments per event and per key; the event's projector interval (its exact cut range
+// within the TOF window, on the branch that serves the projector) for k_bin_records.
 template <bool TOF>
 __global__ __launch_bounds__(BIN_THREADS) void k_bin_count(const float *__restrict__ lors, int64_t n, int stride,
                                                            const float *__restrict__ tofv, int tof_stride,
                                                            LaunchGeom G, TileCfg T, float twin,
                                                            int *__restrict__ ev_cnt,
-                                                           uint8_t *__restrict__ ev_flag,
+                                                           uint8_t *__restrict__ ev_flag, unsigned *__restrict__ ev_cut,
                                                            unsigned *__restrict__ key_count)
 {
     extern __shared__ unsigned hist[];
@@ -240,63 +251,113 @@ __global__ __launch_bounds__(BIN_THREADS) void k_bin_count(const float *__restri
         RaySetup r;
         ray_setup<TOF>(lors + e * stride, TOF ? tofv[e * tof_stride] : 0.0f, G, r);
         int cnt = 0;
-        for_each_event_segment<TOF>(r, G, T, twin, [&](int tile, int cls, int, int, const Branch &, const SegCtx &) {
-            atomicAdd(&hist[tile * NCLASS + cls], 1u);
+        unsigned cut = 0u;
+        for_each_event_segment<TOF>(r, G, T, twin, [&](int tile, int a, int b, const Branch &, const SegCtx &c) {
+            atomicAdd(&hist[seg_class(tile, b - a)], 1u);
             ++cnt;
+            if (c.fp_use) cut = (unsigned)min(c.fa, 0xffff) | (unsigned)max(c.fb, 0) << 16;   // slabs below 2^15
         });
         ev_cnt[e] = cnt;
         ev_flag[e] = r.nan ? 1 : 0;
+        ev_cut[e] = cut;
     }
     __syncthreads();
     for (int i = threadIdx.x; i < T.nkeys; i += BIN_THREADS)
         if (hist[i]) atomicAdd(&key_count[i], hist[i]);
 }
 
-// Each record is written at its segment slot (ev_off[e] + k: event order, a
-// deterministic position) with its sort key; the sort that follows groups the
-// records by key.
+// Sort key and (event, first slab within the tile column, ordinal within the event) of
+// every segment, at its slot (ev_off[e] + ordinal: event order, a deterministic
+// position).  12 bytes per segment go through the sort; the 48-byte records are made
+// after it, in their final order (k_bin_records).  Records emitted here and permuted
+// after the sort took 3.5 of the 5.4 ms of binning 5.9e7 segments.
+constexpr int REL_BITS = 5;   // first slab, 0..31
+
 template <bool TOF>
 __global__ __launch_bounds__(BIN_THREADS) void k_bin_emit(const float *__restrict__ lors, int64_t n, int stride,
                                                           const float *__restrict__ tofv, int tof_stride,
-                                                          LaunchGeom G, TileCfg T, float twin, int prescale,
+                                                          LaunchGeom G, TileCfg T, float twin,
                                                           const int *__restrict__ ev_off,
-                                                          SegRec *__restrict__ recs, int *__restrict__ slot_ev,
-                                                          unsigned *__restrict__ rec_sk)
+                                                          unsigned *__restrict__ key, uint2 *__restrict__ seg)
 {
     const int64_t e = (int64_t)blockIdx.x * BIN_THREADS + threadIdx.x;
     if (e >= n) return;
     RaySetup r;
     ray_setup<TOF>(lors + e * stride, TOF ? tofv[e * tof_stride] : 0.0f, G, r);
-    int j = ev_off[e];
-    for_each_event_segment<TOF>(r, G, T, twin, [&](int tile, int cls, int a, int b, const Branch &B,
-                                                   const SegCtx &c) {
-        const int pos = j++;
-        SegRec R;
-        R.p1 = B.p1;
-        // prescale bit 0 / 1: the secondary / axial voxel edge is a power of
-        // two, and the record holds the line's constants divided by it (exact):
-        // the marcher's (c + k (p - p1)) / d then equals c / d + (k / d) (p - p1)
-        // bit for bit and runs without the division
-        const float ss = (prescale & 1) ? 1.0f / B.ds : 1.0f, zs = (prescale & 2) ? 1.0f / G.dz : 1.0f;
-        R.sec1 = B.sec1 * ss;
-        R.ks = B.ks * ss;
-        R.z1 = r.z1 * zs;
-        R.kz = B.kz * zs;
-        R.Wbp = branch_weight<TOF>(B, r, G, false);
-        R.Wfp = branch_weight<TOF>(B, r, G, true);
-        tof_coeffs<TOF>(B, r, G, R.tA, R.tB);
-        R.slot = pos;
-        R.ab_bp = c.bp_use ? pack_ab(a, b, B.xdom) : 0u;
-        const int fa = max(a, c.fa), fb = min(b, c.fb);
-        R.ab_fp = (c.fp_use && fa < fb) ? pack_ab(fa, fb, B.xdom) : 0u;
-        recs[pos] = R;
-        slot_ev[pos] = (int)e;
-        // sort key: (tile, class), then the branch (a wavefront mostly runs
-        // one branch's marcher), then slab count (longest first: its lanes
-        // march similar lengths); a stable sort keeps slot order within a key
-        const unsigned len = (unsigned)min(b - a, 63);
-        rec_sk[pos] = ((unsigned)(tile * NCLASS + cls) << 7) | ((unsigned)B.xdom << 6) | (63u - len);
+    const int j0 = ev_off[e];
+    unsigned k = 0;
+    for_each_event_segment<TOF>(r, G, T, twin, [&](int tile, int a, int b, const Branch &B, const SegCtx &) {
+        key[j0 + (int)k] = seg_key(tile, b - a, B.xdom);
+        seg[j0 + (int)k] = make_uint2((unsigned)e, (k << REL_BITS) | (unsigned)(a & 31));
+        ++k;
     });
+}
+
+// The records in sorted order, from their events' LORs: neighbouring records mostly
+// belong to neighbouring events.  Also the event of every record (for the
+// backprojector's value gathers) and its weights (for the items' maxima).
+template <bool TOF>
+__global__ __launch_bounds__(256) void k_bin_records(const float *__restrict__ lors, int stride,
+                                                     const float *__restrict__ tofv, int tof_stride, LaunchGeom G,
+                                                     TileCfg T, int prescale, const unsigned *__restrict__ key,
+                                                     const uint2 *__restrict__ seg, int64_t nseg,
+                                                     const int *__restrict__ ev_off, const unsigned *__restrict__ ev_cut,
+                                                     SegRec *__restrict__ recs, int *__restrict__ rec_ev,
+                                                     float2 *__restrict__ rec_w)
+{
+    // the workgroup's records are one run of memory: staged in LDS (in three planes of
+    // 16 bytes), stored by consecutive lanes
+    __shared__ float4 stage[3][256];
+    const int64_t base = (int64_t)blockIdx.x * 256;
+    const int64_t i = min(base + threadIdx.x, nseg - 1);   // the last workgroup's spare lanes repeat its last record
+    const uint2 sg = seg[i];
+    const unsigned k = key[i];
+    const int64_t e = sg.x;
+    const unsigned cut = ev_cut[e];
+    const int off = ev_off[e];
+    RaySetup r;
+    ray_setup<TOF>(lors + e * stride, TOF ? tofv[e * tof_stride] : 0.0f, G, r);
+    const bool xdom = (k >> 3) & 1u;
+    const unsigned tc = k >> SUB_BITS;
+    const int tile = (int)(tc / NCLASS), len = (int)(tc % NCLASS) * CLASS_SLABS + 8 - (int)(k & 7u);
+    const int col = xdom ? tile % T.ntx : (tile / T.ntx) % T.nty;
+    const int a = col * 32 + (int)(sg.y & ((1u << REL_BITS) - 1u)), b = a + len;
+    // as for_each_event_segment: ties march different branches per direction
+    const bool xfp = TOF ? r.xdom_gt : r.xdom_ge, xbp = r.xdom_gt;
+    const bool bp_use = xdom == xbp, fp_use = xdom == xfp && (TOF || !r.q2);
+    Branch B;
+    make_branch(r, xdom, G, B);
+    SegRec R;
+    R.p1 = B.p1;
+    // prescale bit 0 / 1: the secondary / axial voxel edge is a power of
+    // two, and the record holds the line's constants divided by it (exact):
+    // the marcher's (c + k (p - p1)) / d then equals c / d + (k / d) (p - p1)
+    // bit for bit and runs without the division
+    const float ss = (prescale & 1) ? 1.0f / B.ds : 1.0f, zs = (prescale & 2) ? 1.0f / G.dz : 1.0f;
+    R.sec1 = B.sec1 * ss;
+    R.ks = B.ks * ss;
+    R.z1 = r.z1 * zs;
+    R.kz = B.kz * zs;
+    R.Wbp = branch_weight<TOF>(B, r, G, false);
+    R.Wfp = branch_weight<TOF>(B, r, G, true);
+    tof_coeffs<TOF>(B, r, G, R.tA, R.tB);
+    R.slot = off + (int)(sg.y >> REL_BITS);
+    R.ab_bp = bp_use ? pack_ab(a, b, xdom) : 0u;
+    const int fa = max(a, (int)(cut & 0xffffu)), fb = min(b, (int)(cut >> 16));
+    R.ab_fp = (fp_use && fa < fb) ? pack_ab(fa, fb, xdom) : 0u;
+    rec_ev[i] = (int)e;
+    rec_w[i] = make_float2(R.Wbp, R.Wfp);
+    const float4 *q = reinterpret_cast<const float4 *>(&R);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) stage[j][threadIdx.x] = q[j];
+    __syncthreads();
+    float4 *out = reinterpret_cast<float4 *>(recs + base);
+    const int words = 3 * (int)min((int64_t)256, nseg - base);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const int t = j * 256 + (int)threadIdx.x;
+        if (t < words) out[t] = stage[t % 3][t / 3];
+    }
 }
 
 // ------------------------------------------------------------ tile kernels --
@@ -947,8 +1008,8 @@ __global__ __launch_bounds__(256) void k_update_empty(const float *__restrict__ 
 }
 
 // Per item, the largest weight constant of its records in each mode.
-// The records' (Wbp, Wfp) pairs are read from the compact copy the
-// permutation writes (8 B per record instead of a 48 B record).
+// The records' (Wbp, Wfp) pairs are read from the compact copy that
+// k_bin_records writes (8 B per record instead of a 48 B record).
 __global__ __launch_bounds__(256) void k_item_wmax(const float2 *__restrict__ w, Item *__restrict__ items)
 {
     __shared__ float sb[256], sf[256];
@@ -1040,12 +1101,6 @@ __global__ void k_fill_u32(unsigned *__restrict__ d, unsigned v, int64_t n)
     if (i < n) d[i] = v;
 }
 
-__global__ void k_iota_i32(int *__restrict__ d, int64_t n)
-{
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) d[i] = (int)i;
-}
-
 // Geometric event order (srf_event_order).  One 64-bit key per entry j of the
 // caller's index list: bits 33.. the subset j / nps (clamped to n_sub, so a
 // remainder sorts last), then the transaxial angle of the LOR direction folded
@@ -1088,21 +1143,6 @@ __global__ void k_event_keys(const float *__restrict__ lors, int64_t n_lors, int
     const unsigned rb = order_bin(floorf(r) + 32768.0f, 65535.0f);
     k |= ((uint64_t)ab << 26) | ((uint64_t)zb << 16) | rb;
     key[j] = k;
-}
-
-// Records permuted into the order `idx`; their event ids (slot_ev, by slot)
-// are written beside them for the backprojector's value gathers.
-__global__ void k_permute_recs(const SegRec *__restrict__ recs, const int *__restrict__ slot_ev,
-                               const int *__restrict__ idx, int64_t n, SegRec *__restrict__ out,
-                               int *__restrict__ out_ev, float2 *__restrict__ out_w)
-{
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const int j = idx[i];
-    const SegRec R = recs[j];
-    out[i] = R;
-    out_ev[i] = slot_ev[j];
-    out_w[i] = make_float2(R.Wbp, R.Wfp);
 }
 
 // ---------------------------------------------------------------- batches --
@@ -1337,10 +1377,9 @@ struct srf_plan {
     DevBuf<unsigned> key_count;
     DevBuf<char> scan_tmp, sort_tmp;
     DevBuf<unsigned> sk, sk2;
-    DevBuf<int> idx, idx2;
-    DevBuf<float2> wpair;   // (Wbp, Wfp) per record in the sorted order
-    DevBuf<SegRec> recs2;
-    DevBuf<int> slot_ev;    // event id per record slot, before the sort
+    DevBuf<uint2> sg, sg2;
+    DevBuf<float2> wpair;     // (Wbp, Wfp) per record in the sorted order
+    DevBuf<unsigned> ev_cut;  // projector interval per event
 };
 
 namespace {
@@ -1401,11 +1440,10 @@ void free_scratch(srf_plan *P)
     dfree(P->sort_tmp, s, true);
     dfree(P->sk, s, true);
     dfree(P->sk2, s, true);
-    dfree(P->idx, s, true);
-    dfree(P->idx2, s, true);
+    dfree(P->sg, s, true);
+    dfree(P->sg2, s, true);
     dfree(P->wpair, s, true);
-    dfree(P->recs2, s, true);
-    dfree(P->slot_ev, s, true);
+    dfree(P->ev_cut, s, true);
 }
 
 // Destroy: the plan may have been used on any stream, so the device is
@@ -1516,6 +1554,7 @@ int plan_build(srf_plan *P, const float *lors, int64_t n, int64_t lor_stride, co
     PB_TRY(ensure(P->ev_off, (size_t)n + 1, s));
     PB_TRY(ensure(P->ev_flag, (size_t)n, s));
     PB_TRY(ensure(P->ev_cnt, (size_t)n + 1, s));
+    PB_TRY(ensure(P->ev_cut, (size_t)n, s));
     PB_TRY(ensure(P->key_count, (size_t)T.nkeys, s));
     hipLaunchKernelGGL(k_fill_u32, dim3((T.nkeys + 255) / 256), dim3(256), 0, s, P->key_count.p, 0u,
                        (int64_t)T.nkeys);
@@ -1525,10 +1564,12 @@ int plan_build(srf_plan *P, const float *lors, int64_t n, int64_t lor_stride, co
     if (n > 0) {
         if (use_tof)
             hipLaunchKernelGGL(k_bin_count<true>, dim3(nb), dim3(BIN_THREADS), shm, s, lors, n, (int)lor_stride,
-                               tof_values, (int)tof_stride, G, T, twin, P->ev_cnt.p, P->ev_flag.p, P->key_count.p);
+                               tof_values, (int)tof_stride, G, T, twin, P->ev_cnt.p, P->ev_flag.p, P->ev_cut.p,
+                               P->key_count.p);
         else
             hipLaunchKernelGGL(k_bin_count<false>, dim3(nb), dim3(BIN_THREADS), shm, s, lors, n, (int)lor_stride,
-                               tof_values, (int)tof_stride, G, T, twin, P->ev_cnt.p, P->ev_flag.p, P->key_count.p);
+                               tof_values, (int)tof_stride, G, T, twin, P->ev_cnt.p, P->ev_flag.p, P->ev_cut.p,
+                               P->key_count.p);
     }
     PB_HIP(hipGetLastError());
     // event offsets: exclusive scan of the per-event counts (ev_off[n] = total)
@@ -1550,45 +1591,42 @@ int plan_build(srf_plan *P, const float *lors, int64_t n, int64_t lor_stride, co
     PB_TRY(ensure(P->partial, (size_t)nseg, s));
     // the records are built and sorted on the device while the host lays out the
     // work items below (the items come from the key counts alone)
-    if (n > 0) {
+    if (nseg > 0) {
         PB_TRY(ensure(P->sk, (size_t)nseg, s));
         PB_TRY(ensure(P->sk2, (size_t)nseg, s));
-        PB_TRY(ensure(P->idx, (size_t)nseg, s));
-        PB_TRY(ensure(P->idx2, (size_t)nseg, s));
-        PB_TRY(ensure(P->recs2, (size_t)nseg, s));
+        PB_TRY(ensure(P->sg, (size_t)nseg, s));
+        PB_TRY(ensure(P->sg2, (size_t)nseg, s));
         PB_TRY(ensure(P->wpair, (size_t)nseg, s));
-        PB_TRY(ensure(P->slot_ev, (size_t)nseg, s));
         if (use_tof)
             hipLaunchKernelGGL(k_bin_emit<true>, dim3(nb), dim3(BIN_THREADS), 0, s, lors, n, (int)lor_stride,
-                               tof_values, (int)tof_stride, G, T, twin, prescale, P->ev_off.p, P->recs.p, P->slot_ev.p,
-                               P->sk.p);
+                               tof_values, (int)tof_stride, G, T, twin, P->ev_off.p, P->sk.p, P->sg.p);
         else
             hipLaunchKernelGGL(k_bin_emit<false>, dim3(nb), dim3(BIN_THREADS), 0, s, lors, n, (int)lor_stride,
-                               tof_values, (int)tof_stride, G, T, twin, prescale, P->ev_off.p, P->recs.p, P->slot_ev.p,
-                               P->sk.p);
-        // Record order: a stable sort of the slot-ordered records by (key,
+                               tof_values, (int)tof_stride, G, T, twin, P->ev_off.p, P->sk.p, P->sg.p);
+        // Record order: a stable sort of the slot-ordered segments by (key,
         // branch, slab count) -- within one, slot order.  The order (and with
         // it the split into work items and each item's fixed-point scale) is a
         // function of the events alone, so every plan of the same events is
         // bit-identical, and each wavefront gets one branch's segments of
         // similar length.
-        if (nseg > 0) {
-            const unsigned nbs = (unsigned)((nseg + 255) / 256);
-            hipLaunchKernelGGL(k_iota_i32, dim3(nbs), dim3(256), 0, s, P->idx.p, nseg);
-            int key_bits = 1;
-            while ((1 << key_bits) < T.nkeys) ++key_bits;
-            if (7 + key_bits > 32) return SRF_ERR_UNSUPPORTED;
-            size_t sort_bytes = 0;
-            PB_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, sort_bytes, P->sk.p, P->sk2.p, P->idx.p, P->idx2.p,
-                                                       (int)nseg, 0, 7 + key_bits, s));
-            PB_TRY(ensure(P->sort_tmp, sort_bytes, s));
-            PB_HIP(hipcub::DeviceRadixSort::SortPairs(P->sort_tmp.p, sort_bytes, P->sk.p, P->sk2.p, P->idx.p,
-                                                       P->idx2.p, (int)nseg, 0, 7 + key_bits, s));
-            hipLaunchKernelGGL(k_permute_recs, dim3(nbs), dim3(256), 0, s, P->recs.p, P->slot_ev.p, P->idx2.p,
-                               nseg, P->recs2.p, P->rec_ev.p, P->wpair.p);
-            PB_HIP(hipGetLastError());
-            std::swap(P->recs, P->recs2);
-        }
+        int key_bits = 1;
+        while ((1 << key_bits) < T.nkeys) ++key_bits;
+        size_t sort_bytes = 0;
+        PB_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, sort_bytes, P->sk.p, P->sk2.p, P->sg.p, P->sg2.p, (int)nseg,
+                                                  0, SUB_BITS + key_bits, s));
+        PB_TRY(ensure(P->sort_tmp, sort_bytes, s));
+        PB_HIP(hipcub::DeviceRadixSort::SortPairs(P->sort_tmp.p, sort_bytes, P->sk.p, P->sk2.p, P->sg.p, P->sg2.p,
+                                                  (int)nseg, 0, SUB_BITS + key_bits, s));
+        const dim3 nbs((unsigned)((nseg + 255) / 256));
+        if (use_tof)
+            hipLaunchKernelGGL(k_bin_records<true>, nbs, dim3(256), 0, s, lors, (int)lor_stride, tof_values,
+                               (int)tof_stride, G, T, prescale, P->sk2.p, P->sg2.p, nseg, P->ev_off.p, P->ev_cut.p,
+                               P->recs.p, P->rec_ev.p, P->wpair.p);
+        else
+            hipLaunchKernelGGL(k_bin_records<false>, nbs, dim3(256), 0, s, lors, (int)lor_stride, tof_values,
+                               (int)tof_stride, G, T, prescale, P->sk2.p, P->sg2.p, nseg, P->ev_off.p, P->ev_cut.p,
+                               P->recs.p, P->rec_ev.p, P->wpair.p);
+        PB_HIP(hipGetLastError());
     }
     // work items from the key counts (keys are tile-major, so a tile's items are contiguous)
     std::vector<Item> items;

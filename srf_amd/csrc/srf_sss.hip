@@ -67,7 +67,13 @@ __global__ __launch_bounds__(256) void k_sss_pairs(const float *__restrict__ det
         const float inv = 1.0f / sqrtf(r2);
         const float a = det[4 * d + 3];
         const int64_t i = (int64_t)d * ns + s;
-        u = make_float4(vx * inv, vy * inv, vz * inv, (vx * cosf(a) + vy * sinf(a)) * inv / r2);
+        // the unit vector's length corrected to 1 (the rounding of r2 and inv scales all
+        // three components, and with them the cosine whose whole degree is taken)
+        const double l2 = fma((double)(vx * inv), (double)(vx * inv),
+                              fma((double)(vy * inv), (double)(vy * inv), (double)(vz * inv) * (double)(vz * inv)));
+        const float h = (float)(0.5 * (1.0 - l2));
+        u = make_float4(fmaf(vx * inv, h, vx * inv), fmaf(vy * inv, h, vy * inv), fmaf(vz * inv, h, vz * inv),
+                        (vx * cosf(a) + vy * sinf(a)) * inv / r2);
         v = make_float2(em[i], mu[i] * 1.44269504f);
     }
     dir[R.at(d, s)] = u;
@@ -77,8 +83,10 @@ __global__ __launch_bounds__(256) void k_sss_pairs(const float *__restrict__ det
 // The whole-degree scattering angle k = (int)(acos(x) 180 / pi) of a pair
 // (kn_formula.py:41) from two small tables instead of acosf: t = sqrt(1 - |x|) is
 // nearly linear in the angle (0.0087 to 0.0123 per degree), so a cell of 1/256 in t
-// holds at most one whole degree.  A cell stores the float x below which the angle
-// has passed that degree, found with acosf itself, and the smaller angle.
+// holds at most one whole degree.  A cell stores the value of x below which the angle
+// has passed that degree (cos in double, so a float x is put on the right side of
+// it; acosf and the product by 180 / pi misplace x within about 2e-7), and the
+// smaller angle.
 constexpr int DEG_CELLS = 257;
 
 constexpr int BINS_WG = 1024;
@@ -88,25 +96,16 @@ struct DegTable {
     float2 fac[181 + 1];          // 511 / E', window efficiency times KN / sigma_KN
 };
 
-__device__ __forceinline__ int degrees_of(float x)
-{
-    return min((int)(acosf(fminf(1.0f, fmaxf(-1.0f, x))) * 57.295779513082323f), 180);
-}
+__device__ __forceinline__ int degrees_of(float x) { return min((int)(acos((double)x) * 57.29577951308232), 180); }
 
 // tables: [0,181) 511/E', [181,362) window efficiency, [362,543) KN / sigma_KN
 __device__ __forceinline__ void build_degrees(DegTable &T, float *thr, const float *__restrict__ tables)
 {
-    // thr[k], 1 <= k <= 180: the angle is at least k for x below it (to 1e-9, from
-    // a bracket of 8e-6 about cos k)
+    // thr[k]: the angle is at least k where x < thr[k], the float above cos k
     for (int k = threadIdx.x; k <= 180; k += BINS_WG) {
-        const float c = cosf((float)k * 0.017453292519943295f);
-        float lo = c - 4e-6f, hi = c + 4e-6f;
-        for (int i = 0; i < 13; ++i) {
-            const float m = 0.5f * (lo + hi);
-            if (degrees_of(m) >= k) lo = m;
-            else hi = m;
-        }
-        thr[k] = hi;
+        const double c = cos((double)k * 0.017453292519943295);
+        const float f = (float)c;
+        thr[k] = (double)f <= c ? nextafterf(f, 2.0f) : f;
         T.fac[k] = make_float2(tables[k], tables[181 + k] * tables[362 + k]);
     }
     __syncthreads();

@@ -3,8 +3,8 @@ group (1, or 4 above 8192 detectors), points split over workgroups, an index out
 the table, and the point line integrals over the copies and without them.
 
 Bin sums against float64 with the whole-degree angle of each pair taken from the
-float32 cosine as the path defines it (unit vectors, three fused multiply-adds and acos
-in float32), so that no pair sits on another side of a degree: what is left is float32
+float32 cosine the path forms (unit vectors and three fused multiply-adds), so that no
+pair sits on another side of a degree: what is left is float32
 rounding, 1e-5 of the terms' sum as in the other tests, and what lies below float32's
 normal range (2^-126; pairs far outside the energy window)."""
 import math
@@ -25,13 +25,20 @@ def _fma32(a, b, c):
     return (a.double() * b.double() + c.double()).float()
 
 
+def _fma64(x, y, z):
+    return x * x + (y * y + z * z)                         # squares of floats are exact in double
+
+
 def _sum64(det, pts, em, mu, bins, tab):
     v = det[:, None, :3] - pts[None, :, :3]
     r2 = v[..., 0] * v[..., 0] + v[..., 1] * v[..., 1] + v[..., 2] * v[..., 2]
     u = v * (1.0 / torch.sqrt(r2))[..., None]
+    q = u.double()
+    half = (0.5 * (1.0 - _fma64(q[..., 0], q[..., 1], q[..., 2]))).float()
+    u = _fma32(u, half[..., None], u)
     a, b = bins[:, 0].long(), bins[:, 1].long()
     x = -_fma32(u[a, :, 0], u[b, :, 0], _fma32(u[a, :, 1], u[b, :, 1], u[a, :, 2] * u[b, :, 2]))
-    k = torch.clamp((torch.acos(x.clamp(-1, 1)) * 57.295779513082323).long(), 0, 180)
+    k = torch.clamp((torch.acos(x.clamp(-1, 1).double()) * 57.295779513082323).long(), 0, 180)
     v, d = v.double(), det.double()
     r = v.norm(dim=2)
     g = (v[..., 0] * torch.cos(d[:, 3])[:, None] + v[..., 1] * torch.sin(d[:, 3])[:, None]) / r ** 3

@@ -6,8 +6,9 @@
  *    The caller owns every buffer; the library allocates device memory only in
  *    srf_plan_create[_ex], srf_plan_rebuild and srf_batch_create (freed by the
  *    matching *_destroy) and transient scratch in srf_sinogram_lors,
- *    srf_event_order and, for long lists outside graph capture, srf_project
- *    (which runs without it where it is not to be had).
+ *    srf_event_order, the srf_sss_* entry points and, for long lists outside
+ *    graph capture, srf_project and srf_backproject[_ratio], which run without it
+ *    where it is not to be had.
  *  - LORs are AoS rows of `lor_stride` floats [x1,y1,z1,x2,y2,z2,(tof,...)] in
  *    mm, exactly Lors.data of srfnef/data/lors.py:12-22 (stride 6 or 7).
  *  - TOF values are read from `tof_values[e * tof_stride]`; pass
@@ -89,7 +90,10 @@ int srf_project(const float *lors, int64_t n, int64_t lor_stride,
  * siddon_tof.cu.cc:788-812).  image[v] (+)= sum_e values[e] * w_ev.
  * accumulate = 0 zeroes `image` first (the op's cudaMemset, siddon.cc:128);
  * 1 adds into it.  `values` may be NULL, meaning all ones (the sensitivity
- * image, emap_generator.py:169-201). */
+ * image, emap_generator.py:169-201).  A long list is binned into image tiles for
+ * the call (as a plan does; up to about 4 GB of scratch, and `stream` is
+ * synchronised); a short one, and any list under graph capture, goes through
+ * float atomics. */
 int srf_backproject(const float *lors, int64_t n, int64_t lor_stride,
                     const float *tof_values, int64_t tof_stride,
                     const float *values, srf_grid_t grid, const srf_tof_t *tof,

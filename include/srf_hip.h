@@ -261,6 +261,11 @@ int srf_plan_project_ratio(srf_plan *plan, const float *image, const float *y, s
 /* image (+)= backprojection (srf_backproject semantics; values NULL = ones). */
 int srf_plan_backproject(srf_plan *plan, const float *values, srf_bp_mode_t mode,
                          int accumulate, float *image, void *stream);
+/* srf_plan_project of n_images images (nvox floats each, one after the other) into
+ * out (n_images x n): two images share one march of the plan's records.  Per image
+ * bit-identical to the single call.  Takes transient scratch where that can be had
+ * (not under graph capture: then image by image). */
+int srf_plan_project_batch(srf_plan *plan, const float *images, int32_t n_images, float *out, void *stream);
 /* One EM update from a plan: x = x * srf_plan_backproject(values, reference
  * mode) / emap (emap 0 -> zero_guard when it is not 0), the tile sums fused
  * with srf_em_update's operations (bit-identical to the two calls). */

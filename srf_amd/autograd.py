@@ -49,6 +49,14 @@ def _plan_backward(ctx, grad):
 torch.library.register_autograd("srf::plan_project", _plan_backward, setup_context=_plan_setup)
 
 
+def _batch_backward(ctx, grad):
+    handle, n, shape = ctx.meta
+    return None, ops.plan_backproject_batch(handle, grad.contiguous(), n, shape, 1), None, None
+
+
+torch.library.register_autograd("srf::plan_project_batch", _batch_backward, setup_context=_plan_setup)
+
+
 class Projector:
     """p = A x for a fixed LOR set, differentiable in x.
 
@@ -77,6 +85,9 @@ class Projector:
     def __call__(self, x):
         if x.dim() == 3:
             return self._one(x)
+        if self.plan is not None and x.dim() == 4 and x.shape[0] > 0:
+            # one march of the plan's records for several images
+            return self.plan.project_batch(x.permute(0, 3, 2, 1).contiguous())
         return torch.stack([self._one(x[b]) for b in range(x.shape[0])], 0)
 
     def transpose(self, y):

@@ -314,6 +314,10 @@ class Plan:
     def project(self, image_k: Tensor) -> Tensor:
         return plan_project(self.handle, image_k, self.n, self.shape)
 
+    def project_batch(self, images_k: Tensor) -> Tensor:
+        """Projections (B, n) of B kernel-layout images (B, nz, ny, nx)."""
+        return plan_project_batch(self.handle, images_k, self.n, self.shape)
+
     def project_ratio(self, image_k: Tensor, y: Tensor, kind: int, eps: float) -> Tensor:
         """q = ratio(y, project(image)) in one pass (the EM forward half)."""
         return plan_project_ratio(self.handle, image_k, y, int(kind), float(eps), self.n, self.shape)
@@ -382,6 +386,49 @@ def plan_project(handle: int, image_k: Tensor, n: int, shape: List[int]) -> Tens
 @plan_project.register_fake
 def _(handle, image_k, n, shape):
     return image_k.new_empty(n)
+
+
+@torch.library.custom_op("srf::plan_project_batch", mutates_args=())
+def plan_project_batch(handle: int, images_k: Tensor, n: int, shape: List[int]) -> Tensor:
+    """Projections of B images at once (srf_plan_project_batch): (B, n)."""
+    _req(images_k, "images")
+    nx, ny, nz = (int(v) for v in shape)
+    if images_k.dim() != 4 or tuple(images_k.shape[1:]) != (nz, ny, nx):
+        raise ValueError(f"images are {tuple(images_k.shape)}, grid says (B, {nz}, {ny}, {nx})")
+    B = int(images_k.shape[0])
+    out = torch.empty((B, n), dtype=torch.float32, device=images_k.device)
+    with torch.cuda.device(images_k.device):
+        rc = lib().srf_plan_project_batch(handle, images_k.data_ptr(), B, out.data_ptr(), stream_handle(images_k.device))
+    check(rc, "srf_plan_project_batch")
+    return out
+
+
+@plan_project_batch.register_fake
+def _(handle, images_k, n, shape):
+    return images_k.new_empty((images_k.shape[0], n))
+
+
+@torch.library.custom_op("srf::plan_backproject_batch", mutates_args=())
+def plan_backproject_batch(handle: int, values: Tensor, n: int, shape: List[int], mode: int) -> Tensor:
+    """Backprojections of B lists of event values (B, n): (B, nz, ny, nx)."""
+    _req(values, "values")
+    if values.dim() != 2 or values.shape[1] != n:
+        raise ValueError("values must have one row of one entry per event for every image")
+    nx, ny, nz = (int(v) for v in shape)
+    B = int(values.shape[0])
+    img = torch.empty((B, nz, ny, nx), dtype=torch.float32, device=values.device)
+    with torch.cuda.device(values.device):
+        for b in range(B):
+            rc = lib().srf_plan_backproject(handle, values[b].data_ptr(), int(mode), 0, img[b].data_ptr(),
+                                            stream_handle(values.device))
+            check(rc, "srf_plan_backproject")
+    return img
+
+
+@plan_backproject_batch.register_fake
+def _(handle, values, n, shape, mode):
+    nx, ny, nz = shape
+    return values.new_empty((values.shape[0], nz, ny, nx))
 
 
 @torch.library.custom_op("srf::plan_project_ratio", mutates_args=())
@@ -453,5 +500,5 @@ def _(handle, y, p, kind, eps, n, shape, mode):
 # gradients of srf::project / srf::plan_project (adjoint-mode backprojector)
 from . import autograd as _autograd  # noqa: E402,F401
 
-__all__ = ["Plan", "plan_project", "plan_backproject", "plan_backproject_ratio", "project", "backproject", "backproject_ratio", "ratio", "em_update", "lor_digest",
+__all__ = ["Plan", "plan_project", "plan_project_batch", "plan_backproject_batch", "plan_backproject", "plan_backproject_ratio", "project", "backproject", "backproject_ratio", "ratio", "em_update", "lor_digest",
            "to_kernel_layout", "from_kernel_layout", "_lib"]

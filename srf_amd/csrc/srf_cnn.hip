@@ -14,8 +14,9 @@
 // per operand); these networks are small enough that L1/L2 reuse suffices.
 //   k_conv        forward (bias + optional leaky ReLU epilogue), and the
 //                 input gradient as a forward pass of flipped, transposed weights
-//   k_conv_wgrad  weight gradient: per tap, dW[co][ci] += sum_v dY[v][co] X[v+o][ci]
-//                 (split over voxel chunks, FP32 atomics into dW)
+//   k_conv_wgrad_tr  weight gradient: per tap, dW[co][ci] += sum_v dY[v][co] X[v+o][ci]
+//                 (split over runs of tiles, partial sums added by k_wgrad_sum);
+//                 k_conv_wgrad the same for rows that are not 16-byte aligned
 // plus the elementwise kernels of the network (pooling, upsampling, channel
 // copies, activation backward, bias gradient, MSE, Adam, casts).
 #include <hip/hip_runtime.h>
@@ -430,163 +431,236 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(const unsigned short *__rest
 }
 
 // Weight gradient on gfx950's v_mfma_f32_16x16x32_bf16: dW[t][co][ci] +=
-// sum_v dY[v][co] X[v + o_t][ci], an M = cout, N = cin, K = voxels GEMM per
-// tap.  A workgroup owns a 32 x 32 (co, ci) block of all taps and a run of
-// voxel tiles (the forward kernel's tiles; tx a multiple of 8).  Per tile the
-// dY tile and the X halo are staged in LDS channel-major, so that a lane's 8 K
-// values (8 voxels along x) are one aligned 16-byte read of dY; for X the
-// tap's x shift (-1, 0, +1 voxel: 0, 2, 4 bytes past an aligned word) is a
-// funnel shift of an aligned 16-byte and a 4-byte read.  Wavefront w keeps
-// taps w, w + 4, ... for the whole run (27 taps) or K step w (1 tap) in
-// registers and adds them to dW once.  With db, the workgroups of the first
-// cin block also sum the staged dY tile into the bias gradient.
-constexpr int WG_DS = 136;   // dY tile row (128 voxels + 8: rows 272 bytes apart, 4 banks)
+// sum_v dY[v][co] X[v + o_t][ci], per tap a GEMM with K = voxels.  A workgroup owns
+// 16 FB x 16 SB channels of all taps and a run of 8 x 8 x 4 voxel tiles.  The operand
+// with fewer channels is the shifted one: S holds its tile with a halo (X at v + o_t, or
+// dY at u - o_t), F the other's without, so that a fragment read at a tap's shift serves
+// FB products.  Both lie in LDS as they lie in memory, a plane of 16 channels per block,
+// 32 bytes a voxel, and are turned into K-major fragments by the transposing LDS read:
+// four lanes name a voxel, 16 lanes four voxels, and lane i receives channel i of them.
+// Any voxel shift is then an address (a constant beside the lane's own), and staging is
+// 16-byte loads and stores.  Wavefront w keeps taps w, w + 4, ... in registers (27 taps;
+// the 28th place sums the bias gradient, against ones) or takes every fourth K step
+// (1 tap).  Bound by the LDS reads (2 per SB x tap x K step, 8 cycles of the CU's LDS).
+// A workgroup writes its sums to `part`, which k_wgrad_sum adds up in order; without
+// scratch (part null) it adds them to dW with atomics.
+// The 15 layers of the 16-32-64-128 network on four 32 x 64 x 64 samples: 241 us and 123
+// for the sums (1507 with a transposed copy of the tile in LDS, 32 x 32 channel blocks
+// and atomics; 1150 with this kernel and atomics).
+constexpr int WGX = 8, WGY = 8, WGZ = 4, WGV = WGX * WGY * WGZ;
+constexpr int WG_KS = WGV / 32;   // K steps of a tile
+// words of 2 bytes between planes; the 64 bytes over keep two planes in different banks
+constexpr int wg_plane(int R) { return (WGX + 2 * R) * (WGY + 2 * R) * (WGZ + 2 * R) * 16 + 32; }
+static_assert(2 * (2 * wg_plane(1) + 2 * wg_plane(0)) <= 65536, "static LDS");
+// Workgroups of a launch.  The same layers, kernel and sums: 256 432 us, 512 364 us,
+// 1024 397 us (more parts to add up).
+constexpr int64_t WG_WANTED = 512;
+constexpr size_t WG_SCRATCH = 64u << 20;   // bytes of partial sums at most
 
-__device__ __forceinline__ unsigned funnel2(unsigned hi, unsigned lo)
+struct WgCfg {
+    int ntx, nty, ntz;   // tiles of a sample
+    int ntiles, run;     // all tiles; tiles per workgroup
+    int Ds;              // slices of a sample
+    int swap;            // the shifted operand is dY
+    int sstride, fstride;
+    int NF, NS;          // channels of the grid's blocks, F and S
+};
+
+typedef short i16x4 __attribute__((ext_vector_type(4)));
+typedef short i16x8 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) i16x4 *lds_i16x4;
+
+// The fragment (8 K values of this lane's channel) of 32 voxels: lane group q holds voxels
+// 4 q .. 4 q + 3 of p's 16 and of those `next` words on.
+__device__ __forceinline__ bf16x8 wg_frag(const unsigned short *p, int next)
 {
-    return __builtin_amdgcn_alignbyte(hi, lo, 2);
+    const i16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4)p);
+    const i16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4)(p + next));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-template <int TAPS>
-__global__ __launch_bounds__(256) void k_conv_wgrad_lds(const unsigned short *__restrict__ X,
-                                                        const unsigned short *__restrict__ dY, int dy_stride,
-                                                        ConvDims d, ConvTile T, int ntiles, int run, int RW, int CS,
-                                                        float *__restrict__ dW, float *__restrict__ db)
+// NB planes of the tile at (x0, y0, z0), with a halo of R voxels: zero outside the sample's
+// slices [zs0, zs1), outside the plane and past the row's channels.
+template <int NB, int R>
+__device__ __forceinline__ void wg_stage(unsigned short *lds, const unsigned short *__restrict__ src, int stride, int c0,
+                                         int x0, int y0, int z0, int zs0, int zs1, const ConvDims &d)
 {
-    constexpr int R = TAPS == 27 ? 1 : 0;
-    constexpr int NT = TAPS == 27 ? 7 : 1;   // taps per wavefront
-    extern __shared__ unsigned short lds16[];
-    unsigned short *XT = lds16;              // [32 ci][hz][hy][RW]
-    unsigned short *DT = lds16 + 32 * CS;    // [32 co][WG_DS]
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int col = lane & 15, q = lane >> 4;
-    const int co0 = blockIdx.y * 32, ci0 = blockIdx.z * 32;
-    const int hy = T.ty + 2 * R, hz = T.tz + 2 * R, hx = T.tx + 2 * R;
-    const int HV = hx * hy * hz;
-    const int nvox = T.tx * T.ty * T.tz;
-    const int ngx = min(4, (d.cin_p - ci0) >> 3);
-    // this lane's voxel groups (8 along x) of the four K steps
-    int vb[4];
+    constexpr int EX = WGX + 2 * R, EY = WGY + 2 * R, EZ = WGZ + 2 * R, G = 2 * NB, N = EX * EY * EZ * G;
+    constexpr int U = 6, PASSES = (N + 255) / 256;   // loads in flight per thread
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int tv = 32 * k + 8 * q;
-        vb[k] = 0;
-        if (tv < nvox) {
-            const int ltx = tv % T.tx, lty = (tv / T.tx) % T.ty, ltz = tv / (T.tx * T.ty);
-            vb[k] = (ltz * hy + lty) * RW + ltx;
+    for (int b = 0; b < PASSES; b += U) {
+        u16x8 v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (b + u >= PASSES) continue;
+            const int i = threadIdx.x + 256 * (b + u);
+            const int g = i % G, hv = i / G;
+            const int gx = x0 + hv % EX - R, gy = y0 + (hv / EX) % EY - R, gz = z0 + hv / (EX * EY) - R;
+            const int c = c0 + 8 * g;
+            v[u] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
+            if (i < N && (unsigned)gx < (unsigned)d.W && (unsigned)gy < (unsigned)d.H && gz >= zs0 && gz < zs1 && c < stride)
+                v[u] = *reinterpret_cast<const u16x8 *>(src + (unsigned)((gz * d.H + gy) * d.W + gx) * (unsigned)stride + c);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = threadIdx.x + 256 * (b + u);
+            const int g = i % G, hv = i / G;
+            if (b + u < PASSES && i < N)
+                *reinterpret_cast<u16x8 *>(lds + (g >> 1) * wg_plane(R) + 16 * hv + 8 * (g & 1)) = v[u];
         }
     }
-    f32x4 acc[NT][2][2];
+}
+
+template <int TAPS, int FB, int SB>
+__global__ __launch_bounds__(256, 2) void k_conv_wgrad_tr(const unsigned short *__restrict__ S,
+                                                          const unsigned short *__restrict__ F, ConvDims d, WgCfg c,
+                                                          float *__restrict__ part, float *__restrict__ dW,
+                                                          float *__restrict__ db)
+{
+    constexpr int R = TAPS == 27 ? 1 : 0;
+    constexpr int EX = WGX + 2 * R, EXY = EX * (WGY + 2 * R);
+    constexpr int NT = TAPS == 27 ? 7 : 2;   // places per wavefront (the last one of wavefront 3: bias)
+    constexpr int SP = wg_plane(R), FP = wg_plane(0);
+    __shared__ __align__(16) unsigned short lds[SB * SP + FB * FP];
+    unsigned short *Sl = lds, *Fl = lds + SB * SP;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 15, q = lane >> 4;
+    const int f0 = blockIdx.y * 16 * FB, s0 = blockIdx.z * 16 * SB;
+    // this lane's voxel (of the first 16 of a K step) and 4-channel group in the reads
+    const int lv = 4 * q + (col >> 2), lc = 4 * (col & 3);
+    const unsigned short *sb = Sl + 16 * ((lv >> 3) * EX + (lv & 7)) + lc, *fb = Fl + 16 * lv + lc;
+    // with dY fixed the bias sums its rows, else the columns of the shifted one
+    const bool bias = db && (c.swap ? blockIdx.y == 0 : blockIdx.z == 0);
+    const i16x8 ones16 = {0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80};
+    const bf16x8 ones = __builtin_bit_cast(bf16x8, ones16);
+    f32x4 acc[NT][FB][SB];
 #pragma unroll
     for (int i = 0; i < NT; ++i)
 #pragma unroll
-        for (int r = 0; r < 2; ++r)
+        for (int r = 0; r < FB; ++r)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][r][j] = f32x4{0, 0, 0, 0};
-    float bsum = 0.0f;
-    const int t_end = min(ntiles, (int)(blockIdx.x + 1) * run);
-    for (int tile = blockIdx.x * run; tile < t_end; ++tile) {
-        const int bx = tile % T.ntx, by = (tile / T.ntx) % T.nty, bz = tile / (T.ntx * T.nty);
-        const int x0 = bx * T.tx, y0 = by * T.ty, z0 = bz * T.tz;
-        const int zs0 = (z0 / T.Ds) * T.Ds;
+            for (int j = 0; j < SB; ++j) acc[i][r][j] = f32x4{0, 0, 0, 0};
+    const int t_end = min(c.ntiles, (int)(blockIdx.x + 1) * c.run);
+    for (int tile = blockIdx.x * c.run; tile < t_end; ++tile) {
+        const int bx = tile % c.ntx, by = (tile / c.ntx) % c.nty, bz = tile / (c.ntx * c.nty);
+        const int zs0 = (bz / c.ntz) * c.Ds;
+        const int x0 = bx * WGX, y0 = by * WGY, z0 = zs0 + (bz % c.ntz) * WGZ;
         __syncthreads();   // the previous tile's reads are done
-        // X halo, transposed: 16-byte loads of 8 channels, 8 two-byte LDS stores
-        for (int i = threadIdx.x; i < HV * ngx; i += 256) {
-            const int g = i % ngx, hv = i / ngx;
-            const int hxi = hv % hx, hyi = (hv / hx) % hy, hzi = hv / (hx * hy);
-            const int gx = x0 + hxi - R, gy = y0 + hyi - R, gz = z0 + hzi - R;
-            u16x8 val = {0, 0, 0, 0, 0, 0, 0, 0};
-            if (gx >= 0 && gx < d.W && gy >= 0 && gy < d.H && gz >= zs0 && gz < zs0 + T.Ds)
-                val = *reinterpret_cast<const u16x8 *>(X + ((int64_t)(gz * d.H + gy) * d.W + gx) * d.cin_p + ci0 +
-                                                       8 * g);
-            const int pos = (hzi * hy + hyi) * RW + hxi;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) XT[(8 * g + j) * CS + pos] = val[j];
-        }
-        // dY tile, transposed (zero outside the volume, past the tile and for co >= cout)
-        for (int i = threadIdx.x; i < 128 * 4; i += 256) {
-            const int g = i & 3, tv = i >> 2;
-            u16x8 val = {0, 0, 0, 0, 0, 0, 0, 0};
-            const int gx = x0 + tv % T.tx, gy = y0 + (tv / T.tx) % T.ty, gz = z0 + tv / (T.tx * T.ty);
-            const int c = co0 + 8 * g;
-            if (tv < nvox && gx < d.W && gy < d.H && c < dy_stride) {
-                val = *reinterpret_cast<const u16x8 *>(dY + ((int64_t)(gz * d.H + gy) * d.W + gx) * dy_stride + c);
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if (c + j >= d.cout) val[j] = 0;
-            }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) DT[(8 * g + j) * WG_DS + tv] = val[j];
-        }
+        wg_stage<SB, R>(Sl, S, c.sstride, s0, x0, y0, z0, zs0, zs0 + c.Ds, d);
+        wg_stage<FB, 0>(Fl, F, c.fstride, f0, x0, y0, z0, zs0, zs0 + c.Ds, d);
         __syncthreads();
-        if (db && blockIdx.z == 0) {
-            const int c = threadIdx.x >> 3, part = threadIdx.x & 7;
+        if constexpr (TAPS == 27) {
+#pragma unroll 1
+            for (int k = 0; k < WG_KS; ++k) {   // half a slice of the tile each
+                const unsigned short *pk = sb + 16 * ((k >> 1) * EXY + (k & 1) * 4 * EX);
+                bf16x8 f[FB];
 #pragma unroll
-            for (int v = 0; v < 16; ++v) bsum += bf2f(DT[c * WG_DS + part * 16 + v]);
+                for (int r = 0; r < FB; ++r) f[r] = wg_frag(fb + r * FP + 16 * 32 * k, 16 * 16);
+#pragma unroll
+                for (int i = 0; i < NT; ++i) {
+                    // wavefront 3's last place: the bias, of the unshifted tap
+                    const int t = i < NT - 1 || wave < 3 ? wave + 4 * i : 13;
+                    const unsigned short *p = pk + 16 * ((t / 9) * EXY + ((t / 3) % 3) * EX + t % 3);
+                    const bool sums = i == NT - 1 && wave == 3;
+                    if (sums && !bias) continue;
+#pragma unroll
+                    for (int j = 0; j < SB; ++j) {
+                        const bf16x8 s = sums && !c.swap ? ones : wg_frag(p + j * SP, 16 * 2 * EX);
+#pragma unroll
+                        for (int r = 0; r < FB; ++r)
+                            acc[i][r][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sums && c.swap ? ones : f[r], s,
+                                                                                   acc[i][r][j], 0, 0, 0);
+                    }
+                }
+            }
+        } else {
+#pragma unroll
+            for (int h = 0; h < WG_KS / 4; ++h) {
+                const int k = wave + 4 * h;
+                bf16x8 f[FB], s[SB];
+#pragma unroll
+                for (int r = 0; r < FB; ++r) f[r] = wg_frag(fb + r * FP + 16 * 32 * k, 16 * 16);
+#pragma unroll
+                for (int j = 0; j < SB; ++j) s[j] = wg_frag(sb + j * SP + 16 * 32 * k, 16 * 16);
+#pragma unroll
+                for (int r = 0; r < FB; ++r)
+#pragma unroll
+                    for (int j = 0; j < SB; ++j)
+                        acc[0][r][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[r], s[j], acc[0][r][j], 0, 0, 0);
+                if (bias && !c.swap) {
+#pragma unroll
+                    for (int r = 0; r < FB; ++r)
+                        acc[1][r][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[r], ones, acc[1][r][0], 0, 0, 0);
+                } else if (bias) {
+#pragma unroll
+                    for (int j = 0; j < SB; ++j)
+                        acc[1][0][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, s[j], acc[1][0][j], 0, 0, 0);
+                }
+            }
         }
-        // A fragments (dY) of the four K steps, shared by every tap
-        u16x8 a[4][2];
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-#pragma unroll
-            for (int r = 0; r < 2; ++r)
-                a[k][r] = *reinterpret_cast<const u16x8 *>(DT + (r * 16 + col) * WG_DS + 32 * k + 8 * q);
+    }
+    // C layout: lane l holds column (S) l % 16, rows (F) 4 (l / 16) + e
+    if (part) {
+        const int p = TAPS == 27 ? blockIdx.x : blockIdx.x * 4 + wave;
+        const int mine = 4 * q * c.NS + col;
 #pragma unroll
         for (int i = 0; i < NT; ++i) {
-            const int t = TAPS == 27 ? wave + 4 * i : 0;
-            if (t >= TAPS) continue;
-            int shift = 0, tdelta = 0;
-            if (TAPS == 27) {
-                shift = t % 3;   // dx + 1
-                tdelta = (t / 9) * hy * RW + ((t / 3) % 3) * RW;
-            }
+            const int slot = TAPS == 27 ? wave + 4 * i : i;   // TAPS: the bias
+            float *o = part + (((int64_t)p * (TAPS + 1) + slot) * c.NF + f0) * c.NS + s0;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                if (TAPS == 1 && k != wave) continue;
+            for (int r = 0; r < FB; ++r)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const unsigned short *p = XT + (j * 16 + col) * CS + vb[k] + tdelta;
-                    uint4 w = *reinterpret_cast<const uint4 *>(p);
-                    if (shift) {
-                        const unsigned nx = *reinterpret_cast<const unsigned *>(p + 8);
-                        if (shift == 2) {
-                            w = uint4{w.y, w.z, w.w, nx};
-                        } else {
-                            w = uint4{funnel2(w.y, w.x), funnel2(w.z, w.y), funnel2(w.w, w.z), funnel2(nx, w.w)};
-                        }
-                    }
-                    const bf16x8 b = __builtin_bit_cast(bf16x8, w);
+                for (int j = 0; j < SB; ++j)
 #pragma unroll
-                    for (int r = 0; r < 2; ++r)
-                        acc[i][r][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[k][r]), b,
-                                                                               acc[i][r][j], 0, 0, 0);
-                }
-            }
+                    for (int e = 0; e < 4; ++e) o[mine + ((16 * r + e) * c.NS + 16 * j)] = acc[i][r][j][e];
         }
+        return;
     }
-    // C layout: lane l holds column (ci) l % 16, rows (co) 4 * (l / 16) + e
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
-        const int t = TAPS == 27 ? wave + 4 * i : 0;
-        if (t >= TAPS) continue;
+        const int slot = TAPS == 27 ? wave + 4 * i : i;
 #pragma unroll
-        for (int r = 0; r < 2; ++r)
+        for (int r = 0; r < FB; ++r)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int j = 0; j < SB; ++j)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const int co = co0 + r * 16 + 4 * q + e, ci = ci0 + j * 16 + col;
+                    const int f = f0 + 16 * r + 4 * q + e, s = s0 + 16 * j + col;
+                    const int co = c.swap ? s : f, ci = c.swap ? f : s;
                     const float v = acc[i][r][j][e];
-                    if (co < d.cout && ci < d.cin_p && v != 0.0f)
-                        atomicAdd(dW + ((int64_t)t * d.cout_p + co) * d.cin_p + ci, v);
+                    if (co >= d.cout || ci >= d.cin_p || v == 0.0f) continue;
+                    if (slot < TAPS)
+                        atomicAdd(dW + ((int64_t)(c.swap ? TAPS - 1 - slot : slot) * d.cout_p + co) * d.cin_p + ci, v);
+                    else if (bias && ci == 0)
+                        atomicAdd(db + co, v);
                 }
     }
-    if (db && blockIdx.z == 0) {
-        bsum += __shfl_xor(bsum, 1, 8);
-        bsum += __shfl_xor(bsum, 2, 8);
-        bsum += __shfl_xor(bsum, 4, 8);
-        const int c = co0 + (threadIdx.x >> 3);
-        if ((threadIdx.x & 7) == 0 && c < d.cout && bsum != 0.0f) atomicAdd(db + c, bsum);
+}
+
+// dW += the parts of k_conv_wgrad_tr, each element by eight groups of threads (parts g,
+// g + 8, ...) whose sums are added in order.
+__global__ __launch_bounds__(256) void k_wgrad_sum(const float *__restrict__ part, int nparts, int taps, ConvDims d,
+                                                   WgCfg c, float *__restrict__ dW, float *__restrict__ db)
+{
+    __shared__ float red[8][32];
+    const int64_t n = (int64_t)(taps + 1) * c.NF * c.NS;
+    const int64_t i = (int64_t)blockIdx.x * 32 + (threadIdx.x & 31);
+    const int g = threadIdx.x >> 5;
+    const int s = (int)(i % c.NS), f = (int)(i / c.NS % c.NF), slot = (int)(i / ((int64_t)c.NS * c.NF));
+    const int co = c.swap ? s : f, ci = c.swap ? f : s;
+    const bool live = i < n && co < d.cout && (slot == taps ? db && ci == 0 : ci < d.cin_p);
+    float sum = 0.0f;
+    if (live) {
+#pragma unroll 8
+        for (int p = g; p < nparts; p += 8) sum += part[p * n + i];
+    }
+    red[g][threadIdx.x & 31] = sum;
+    __syncthreads();
+    if (g == 0 && live) {
+        for (int k = 1; k < 8; ++k) sum += red[k][threadIdx.x];
+        const int t = c.swap ? taps - 1 - slot : slot;
+        float *out = slot == taps ? db + co : dW + ((int64_t)t * d.cout_p + co) * d.cin_p + ci;
+        *out += sum;
     }
 }
 
@@ -891,34 +965,56 @@ int srf_cnn_conv_wgrad_batch(const void *x, const void *dy, int32_t dy_stride, i
         return SRF_ERR_UNSUPPORTED;
     ConvDims d{N * D, H, W, cin_p, cout, cout_p, 0, 0, taps, -1.0f};
     auto st = (hipStream_t)stream;
-    const int R = taps == 27 ? 1 : 0;
-    ConvTile T;
-    conv_tile(D, H, W, R, T);
-    // the LDS path: x tiles of whole 8-voxel groups, 16-byte aligned rows
-    const int RW = (T.tx + 2 * R + 7) / 8 * 8;
-    int CS = 0;
-    bool lds_ok = T.tx % 8 == 0 && dy_stride % 8 == 0 &&
-                  !((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy)) & 15);
-    if (lds_ok) {
-        const int hv = RW * (T.ty + 2 * R) * (T.tz + 2 * R);
-        CS = (hv + 119) / 128 * 128 + 8;   // >= hv; channel rows 4 banks apart
-        lds_ok = (size_t)64 * (CS + WG_DS) <= CONV_LDS_MAX;
-    }
-    if (lds_ok) {
-        const int ntiles = T.ntx * T.nty * (N * D / T.tz);
-        const int nblk = (cout_p / 32) * ((cin_p + 31) / 32);
-        // about 1024 workgroups, each adding its taps to dW once per run of tiles
-        int run = (int)(((int64_t)ntiles * nblk + 1023) / 1024);
-        run = run < 1 ? 1 : run > 64 ? 64 : run;
-        dim3 grid((unsigned)((ntiles + run - 1) / run), (unsigned)(cout_p / 32), (unsigned)((cin_p + 31) / 32));
-        const size_t lds = (size_t)64 * (CS + WG_DS);
-        if (taps == 27)
-            hipLaunchKernelGGL(k_conv_wgrad_lds<27>, grid, dim3(256), lds, st, (const unsigned short *)x,
-                               (const unsigned short *)dy, dy_stride, d, T, ntiles, run, RW, CS, dw, db);
-        else
-            hipLaunchKernelGGL(k_conv_wgrad_lds<1>, grid, dim3(256), lds, st, (const unsigned short *)x,
-                               (const unsigned short *)dy, dy_stride, d, T, ntiles, run, RW, CS, dw, db);
-        return launch_status();
+    // the LDS path: 16-byte aligned rows of both operands
+    if (dy_stride % 8 == 0 && !((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy)) & 15)) {
+        const int nx = (cin_p + 15) / 16, ny = (cout + 15) / 16;
+        WgCfg c;
+        c.swap = ny < nx ? 1 : 0;
+        const int nf = c.swap ? nx : ny, ns = c.swap ? ny : nx;
+        const int SB = taps == 1 || ns < 2 ? 1 : 2;
+        const int FB = taps == 1 || nf < 2 ? 1 : nf % 3 == 0 && SB == 1 ? 3 : 2;   // (3, 2) would spill
+        const int gf = (nf + FB - 1) / FB, gs = (ns + SB - 1) / SB;
+        c.NF = gf * FB * 16;
+        c.NS = gs * SB * 16;
+        c.sstride = c.swap ? dy_stride : cin_p;
+        c.fstride = c.swap ? cin_p : dy_stride;
+        c.ntx = (W + WGX - 1) / WGX;
+        c.nty = (H + WGY - 1) / WGY;
+        c.ntz = (D + WGZ - 1) / WGZ;
+        c.Ds = D;
+        c.ntiles = c.ntx * c.nty * c.ntz * N;
+        const size_t per = (size_t)(taps + 1) * c.NF * c.NS * sizeof(float) * (taps == 1 ? 4 : 1);
+        // WG_WANTED workgroups, and at most WG_SCRATCH of partial sums
+        int64_t parts = WG_WANTED / ((int64_t)gf * gs);
+        parts = parts < (int64_t)(WG_SCRATCH / per) ? parts : (int64_t)(WG_SCRATCH / per);
+        parts = parts < 1 ? 1 : parts;
+        c.run = (int)((c.ntiles + parts - 1) / parts);
+        dim3 grid((unsigned)((c.ntiles + c.run - 1) / c.run), (unsigned)gf, (unsigned)gs);
+        const int nparts = (int)grid.x * (taps == 1 ? 4 : 1);
+        // no scratch under capture, nor where every element has one writer
+        float *part = nullptr;
+        if (!capturing(st) && nparts > 1 && per * grid.x <= WG_SCRATCH)
+            part = static_cast<float *>(pool_get(per * grid.x, st));
+        auto *S = (const unsigned short *)(c.swap ? dy : x), *F = (const unsigned short *)(c.swap ? x : dy);
+#define SRF_WGRAD(TP, FBK, SBK) \
+    hipLaunchKernelGGL((k_conv_wgrad_tr<TP, FBK, SBK>), grid, dim3(256), 0, st, S, F, d, c, part, dw, db)
+        if (taps == 1) SRF_WGRAD(1, 1, 1);
+        else if (SB == 2) SRF_WGRAD(27, 2, 2);
+        else if (FB == 3) SRF_WGRAD(27, 3, 1);
+        else if (FB == 2) SRF_WGRAD(27, 2, 1);
+        else SRF_WGRAD(27, 1, 1);
+#undef SRF_WGRAD
+        int rc = launch_status();
+        if (part) {
+            const int64_t n = (int64_t)(taps + 1) * c.NF * c.NS;
+            if (rc == SRF_OK) {
+                hipLaunchKernelGGL(k_wgrad_sum, dim3((unsigned)((n + 31) / 32)), dim3(256), 0, st, part, nparts, taps, d,
+                                   c, dw, db);
+                rc = launch_status();
+            }
+            pool_put(part, st);
+        }
+        return rc;
     }
     const int64_t V = (int64_t)N * D * H * W;
     const int chunk = 4096;

@@ -7,12 +7,8 @@
 // activations) in BF16 with FP32 master copies kept by the optimiser.
 //
 // Convolutions (3x3x3 or 1x1x1, stride 1, zero padding) are implicit GEMMs on
-// v_mfma_f32_32x32x8bf16_1k (A: 32 voxels x 8 channels, B: 8 channels x 32
-// output channels, FP32 accumulation).  Each wavefront owns a 32-voxel x
-// 32-channel block of the output; a workgroup stacks four of them along the
-// voxels.  Fragments are loaded straight from global memory (8 bytes per lane
-// per operand); these networks are small enough that L1/L2 reuse suffices.
-//   k_conv        forward (bias + optional leaky ReLU epilogue), and the
+// v_mfma_f32_16x16x32_bf16 (FP32 accumulation) from tiles staged in LDS.
+//   k_conv, k_conv_rows, k_conv_res  forward (bias + optional leaky ReLU epilogue), and the
 //                 input gradient as a forward pass of flipped, transposed weights
 //   k_conv_wgrad_tr  weight gradient: per tap, dW[co][ci] += sum_v dY[v][co] X[v+o][ci]
 //                 (split over runs of tiles, partial sums added by k_wgrad_sum);
@@ -58,30 +54,25 @@ __device__ __forceinline__ void tap_offset(int t, int taps, int &dz, int &dy, in
     dx = t % 3 - 1;
 }
 
-// Convolution as an implicit GEMM on gfx950's v_mfma_f32_16x16x32_bf16
-// (A: 16 voxels x 32 K values, B: 32 K values x 16 output channels, FP32
-// accumulation).  K runs over (tap, group of 8 input channels).
+// Convolution as an implicit GEMM on gfx950's v_mfma_f32_16x16x32_bf16 (A: 16 output
+// channels x 32 K values, B: 32 K values x 16 voxels, FP32 accumulation).  K runs over
+// (tap, group of 8 input channels).
 //
-// A workgroup of four wavefronts owns a tile of up to 128 voxels (tx x ty x tz,
-// x fastest; wavefront w rows 32w..32w+31, two 16-row blocks) and NBW blocks of
-// 16 output channels.  Per chunk of 8, 16 or 32 input channels the tile's input
-// halo is staged in LDS with coalesced 16-byte loads: zero outside the volume
-// and outside the tile's own sample (a batch stacks samples along z, Ds slices
-// each; a tile never straddles two), so taps never read a neighbouring
-// sample.  A lane then reads its 8 K values of a voxel as one 16-byte LDS
-// access; a halo voxel's channel groups are padded to an odd count of 16-byte
-// words so that the 16 voxels of a row block start in different banks.
-// Weights (a few KiB to 440 KiB per layer) are read from global memory
-// through the caches.
+// A workgroup owns a tile of voxels and NBW blocks of 16 output channels.  Per chunk of 8,
+// 16 or 32 input channels the tile's input halo is staged in LDS with coalesced 16-byte
+// loads: zero outside the volume and outside the tile's own sample (a batch stacks samples
+// along z, Ds slices each; a tile never straddles two), so taps never read a neighbouring
+// sample.  A lane then reads its 8 K values of a voxel as one 16-byte LDS access; in
+// k_conv a halo voxel's channel groups are padded to an odd count of 16-byte words so that
+// eight voxels of a row start in different banks.  Weights (a few KiB to 440 KiB per layer)
+// are read from global memory through the caches, some steps ahead (k_conv_res: once).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
 
 struct ConvTile {
-    int tx, ty, tz;             // tile extent
-    int ntx, nty;               // tiles along x and y
-    int Ds;                     // slices per sample (tz divides it)
-    int nblk;                   // tiles of the launch
-    float inv_hx, inv_hyx;      // 1 / halo row, 1 / halo plane (voxels)
-    float inv_tx, inv_txy;      // 1 / tile row, 1 / tile plane
+    int ntx, nty, ntz;   // tiles of a sample
+    int Ds;              // slices per sample
+    int nblk;            // tiles of the launch
 };
 
 // The input of a convolution: channels [0, cc) are the nearest-neighbour 2x
@@ -103,283 +94,611 @@ struct ConvHead {
     float *out;                // one value per voxel
 };
 
-// floor(a / b) for 0 <= a < 2^24 and b >= 1 given inv = 1/b in float: the
-// float quotient is off by at most one, and one integer step corrects it.
-__device__ __forceinline__ int idiv(int a, int b, float inv)
-{
-    int q = (int)((float)a * inv);
-    const int r = a - q * b;
-    q += r >= b ? 1 : 0;
-    q -= r < 0 ? 1 : 0;
-    return q;
-}
-constexpr int CONV_TILE = 128;
-constexpr int CONV_LDS_MAX = 65536;
+constexpr int CX = 8;         // k_conv's tile along x and y
+constexpr int64_t CONV_WANTED = 512;   // workgroups of a launch, where the volume has them
 
-// Offset in halo voxels of tap t from the halo voxel of the tap (-1,-1,-1) corner.
-__device__ __forceinline__ int tap_delta(int t, int taps, int hx, int hyx)
+// Halo voxels of k_conv's tile of cz slices.
+constexpr int halo_voxels(int R, int cz) { return (CX + 2 * R) * (CX + 2 * R) * (cz + 2 * R); }
+
+// k_conv_rows' tile and its halo.
+constexpr int RWX = 16, RWY = 8, RWZ = 4;
+constexpr int RHX = RWX + 2, RHY = RWY + 2, RHV = RHX * RHY * (RWZ + 2);
+constexpr int64_t ROWS_WANTED = 256;   // workgroups that pay for the larger tile
+
+// Where channel group g of a voxel in halo column x lies among its groups.
+template <int NG>
+__device__ __forceinline__ int row_slot(int g, int x) { return NG == 4 ? g ^ ((x >> 2) & 3) : g; }
+
+// The offset of tap t in a halo of rows of ex and planes of exy voxels.
+template <int TAPS>
+__device__ __forceinline__ int tap_delta(int t, int ex, int exy)
 {
-    if (taps == 1) return 0;
-    return (t / 9) * hyx + ((t / 3) % 3) * hx + t % 3;
+    if (TAPS == 1) return 0;
+    return (t / 9) * exy + ((t / 3) % 3) * ex + t % 3;
 }
 
-template <int TAPS, int NG, int NBW>
-__device__ __forceinline__ void conv_chunk(const u16x8 *__restrict__ halo, const int (&hb)[2], int gp, int hx, int hyx,
-                                           const unsigned short *__restrict__ wl, int64_t tap_stride, int nb_stride,
-                                           int q, f32x4 (&acc)[2][NBW])
+// One chunk's products for RB blocks of 16 voxels: two rows of 8 (TX = 8) or a row of 16.
+// v0: this lane's voxel of block 0 in the halo, x0 its column there; w: the weights of the
+// chunk's first channel and output, read PF steps ahead.  The sums run over the taps in
+// order, the channels of a chunk together: every kernel keeps this order, so that a
+// layer's bf16 outputs do not depend on which one computes them.
+template <int TAPS, int NG, int NBW, int RB, int TX>
+__device__ __forceinline__ void conv_chunk(const u16x8 *halo, int v0, int x0, const unsigned short *__restrict__ w,
+                                           int64_t tap_stride, int cin_p, int col, int q, f32x4 (&acc)[RB][NBW])
 {
     constexpr int G = TAPS * NG;          // K groups of 8 in this chunk
     constexpr int S = (G + 3) / 4;        // MFMA steps (4 groups each)
     constexpr int K = 4 / NG;             // taps per step
+    constexpr int R2 = TAPS == 27 ? 2 : 0, EX = TX + R2, EXY = EX * (8 + R2);
+    constexpr int GP = TX == 8 ? NG | 1 : NG, STEP = TX == 8 ? 2 * EX : EX;   // words of a voxel; voxels between blocks
+    constexpr int PF = RB * NBW >= 8 ? 2 : RB * NBW >= 4 ? 3 : RB * NBW >= 2 ? 5 : 10;   // steps ahead: weights,
+    constexpr int AH = RB == 1 ? 4 : RB == 2 ? 2 : RB * NBW == 4 ? 1 : 0;               // and voxels
     // lane l's K group q is (tap K s + q / NG, channel group q % NG)
-    const int g = q & (NG - 1), tq = q / NG;
-    const u16x8 *a0 = halo + hb[0] * gp + g, *a1 = halo + hb[1] * gp + g;
-    const unsigned short *wq = wl + tq * tap_stride + 8 * g;
+    int g = q & (NG - 1), tq = q / NG;
+    asm volatile("" : "+v"(g), "+v"(tq));   // what depends on them is not kept across the chunks
+    const unsigned mine = (unsigned)(col * cin_p + 8 * g) + (unsigned)tq * (unsigned)tap_stride;
+    u16x8 wr[PF + 1][NBW];
+    // in order of s: the place advances by a step's taps and is kept from the optimiser,
+    // which would hold every step's address in registers across the chunks (the place and
+    // not the pointer: that would lose its address space and be read by flat loads)
+    int64_t at = 0;
+    auto fetch = [&](int s, u16x8 (&to)[NBW]) {
+        const bool valid = 4 * s + 3 < G || 4 * s + q < G;
+#pragma unroll
+        for (int j = 0; j < NBW; ++j) {
+            to[j] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
+            if (valid) to[j] = *reinterpret_cast<const u16x8 *>(w + at + 16 * j * cin_p + mine);
+        }
+        at += K * tap_stride;
+        asm volatile("" : "+s"(at));
+    };
+#pragma unroll
+    for (int s = 0; s < PF; ++s)
+        if (s < S) fetch(s, wr[s]);
+    __syncthreads();   // the halo is there
+    u16x8 a[AH + 1][RB];
+    auto read = [&](int s, u16x8 (&to)[RB]) {
+        // the taps of this step: uniform candidates, one picked per lane
+        const int t = K * s;
+        int delta = tap_delta<TAPS>(t, EX, EXY), dx = t % 3;
+#pragma unroll
+        for (int k = 1; k < K; ++k) {
+            const int tk = t + k < TAPS ? t + k : TAPS - 1;
+            delta = tq == k ? tap_delta<TAPS>(tk, EX, EXY) : delta;
+            dx = tq == k ? tk % 3 : dx;
+        }
+        const u16x8 *p = halo + (v0 + delta) * GP + (TX == 8 ? g : row_slot<NG>(g, x0 + (TAPS == 27 ? dx : 0)));
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+            to[r] = p[r * STEP * GP];
+            if (4 * s + 3 >= G && 4 * s + q >= G) to[r] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};   // zeros on both sides past the last tap
+        }
+    };
+#pragma unroll
+    for (int s = 0; s < AH; ++s)
+        if (s < S) read(s, a[s]);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
-        // the tap offsets of this step: uniform candidates, one picked per lane
-        int delta;
-        if constexpr (K == 1) {
-            delta = tap_delta(s, TAPS, hx, hyx);
-        } else if constexpr (K == 2) {
-            const int d0 = tap_delta(2 * s, TAPS, hx, hyx), d1 = tap_delta(2 * s + 1, TAPS, hx, hyx);
-            delta = tq ? d1 : d0;
-        } else {
-            const int d0 = tap_delta(4 * s, TAPS, hx, hyx), d1 = tap_delta(4 * s + 1, TAPS, hx, hyx);
-            const int d2 = tap_delta(4 * s + 2, TAPS, hx, hyx), d3 = tap_delta(4 * s + 3, TAPS, hx, hyx);
-            delta = tq == 0 ? d0 : tq == 1 ? d1 : tq == 2 ? d2 : d3;
-        }
-        const bool valid = (G % 4 == 0 || s < S - 1) || (4 * s + q < G);
-        u16x8 a[2], w[NBW];
+        if (s + PF < S) fetch(s + PF, wr[(s + PF) % (PF + 1)]);
+        if (s + AH < S) read(s + AH, a[(s + AH) % (AH + 1)]);
+        if (AH > 0) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int r = 0; r < 2; ++r) a[r] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-        for (int j = 0; j < NBW; ++j) w[j] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-        if (valid) {
-            a[0] = a0[delta * gp];
-            a[1] = a1[delta * gp];
-            const unsigned short *ws = wq + (int64_t)(K * s) * tap_stride;
-#pragma unroll
-            for (int j = 0; j < NBW; ++j) w[j] = *reinterpret_cast<const u16x8 *>(ws + j * nb_stride);
-        }
-#pragma unroll
-        for (int r = 0; r < 2; ++r)
+        for (int r = 0; r < RB; ++r)
 #pragma unroll
             for (int j = 0; j < NBW; ++j)
-                acc[r][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[r]),
-                                                                    __builtin_bit_cast(bf16x8, w[j]), acc[r][j], 0,
-                                                                    0, 0);
+                acc[r][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wr[s % (PF + 1)][j]),
+                                                                    __builtin_bit_cast(bf16x8, a[s % (AH + 1)][r]),
+                                                                    acc[r][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);   // a few steps' loads ahead, not all of them
     }
 }
 
-template <int TAPS, int NBW>
-__global__ __launch_bounds__(256) void k_conv(ConvIn in, const unsigned short *__restrict__ Wt,
-                                              const float *__restrict__ bias, ConvDims d, ConvTile T,
-                                              unsigned short *__restrict__ Ybf, float *__restrict__ Yf, ConvHead hd)
+// A chunk's input and the sample's slices.  Both inputs are read through buffer resources:
+// places outside the volume or the sample load zeros (an offset past the buffer's end).
+struct HaloSrc {
+    __amdgpu_buffer_rsrc_t p;   // the chunk's first channel
+    int stride, up;             // bytes of a voxel's row; 1: the half-size grid
+    int W, H;
+    int x0, y0, z0, zs0, zs1;   // the tile and its sample
+};
+
+__device__ __forceinline__ HaloSrc halo_source(const ConvIn &in, const ConvDims &d, int c0)
 {
-    constexpr int R = TAPS == 27 ? 1 : 0;
-    constexpr int STAGE = 4;   // halo loads in flight per thread
+    HaloSrc h;
+    h.up = c0 < in.cc ? 1 : 0;   // a chunk lies wholly in one of the two inputs
+    const int ch = h.up ? in.cc : d.cin_p - in.cc, skip = h.up ? c0 : c0 - in.cc;
+    const unsigned vox = (unsigned)(d.D >> h.up) * (unsigned)(d.H >> h.up) * (unsigned)(d.W >> h.up);
+    h.stride = 2 * ch;
+    // (scalar registers, which a resource must be in)
+    const uint64_t at = reinterpret_cast<uint64_t>((h.up ? in.coarse : in.fine) + skip);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)at), hi = __builtin_amdgcn_readfirstlane((unsigned)(at >> 32));
+    h.p = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>((uint64_t)hi << 32 | lo), 0,
+                                            __builtin_amdgcn_readfirstlane((vox * (unsigned)ch - (unsigned)skip) * 2),
+                                            0x00020000);
+    h.W = d.W;
+    h.H = d.H;
+    return h;
+}
+
+// Channel group g of voxel (gx, gy, gz).
+__device__ __forceinline__ u16x8 halo_fetch(const HaloSrc &s, int gx, int gy, int gz, int g, bool ok)
+{
+    const int sh = s.up;
+    const unsigned at = (unsigned)(((gz >> sh) * (s.H >> sh) + (gy >> sh)) * (s.W >> sh) + (gx >> sh)) *
+                            (unsigned)s.stride + 16 * g;
+    ok = ok && (unsigned)gx < (unsigned)s.W && (unsigned)gy < (unsigned)s.H && gz >= s.zs0 && gz < s.zs1;
+    return __builtin_bit_cast(u16x8, __builtin_amdgcn_raw_buffer_load_b128(s.p, ok ? (int)at : -1, 0, 0));
+}
+
+// A layer's epilogue: bias, activation, stores and the head.
+struct ConvOut {
+    const float *bias;
+    unsigned short *Ybf;
+    float *Yf;
+    ConvHead hd;
+};
+
+// Stores 16 voxels x 16 NBW channels from n0 on: lane l holds voxel l % 16 (number vox, if
+// in_vol) and channels 4 (l / 16) + e of each block of 16, 8 (bf16) or 16 bytes (float)
+// of a row where its layout allows.
+template <int NBW>
+__device__ __forceinline__ void conv_store(const f32x4 (&acc)[NBW], const float (&bn)[NBW][4],
+                                           const float (&hw)[NBW][4], const ConvDims &d, const ConvOut &o, int n0, int q, unsigned vox, bool in_vol)
+{
+    const bool even = (d.out_stride | d.out_off) % 4 == 0;
+    const bool vec_bf = even && !(reinterpret_cast<uintptr_t>(o.Ybf) & 7);
+    const bool vec_f = even && !(reinterpret_cast<uintptr_t>(o.Yf) & 15);
+    float sum = 0.0f;   // of the head, in channel order: passed on from lane group to lane group
+    const int from = (threadIdx.x + 48) & 63;
+#pragma unroll
+    for (int j = 0; j < NBW; ++j) {
+        const int n = n0 + 16 * j + 4 * q, left = d.cout - n;   // channels to store
+        const unsigned at = vox * (unsigned)d.out_stride + (unsigned)(d.out_off + n);
+        float y[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            y[e] = acc[j][e] + bn[j][e];
+            if (d.slope >= 0.0f && y[e] < 0.0f) y[e] *= d.slope;
+        }
+        const u16x4 w = {f2bf(y[0]), f2bf(y[1]), f2bf(y[2]), f2bf(y[3])};
+        if (o.hd.out)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (j + k > 0) sum = __shfl(sum, from);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (e < left) sum += bf2f(w[e]) * hw[j][e];   // products of bf16 values are exact
+            }
+        if (!in_vol || left <= 0) continue;
+        if (o.Ybf) {
+            if (vec_bf && left >= 4) *reinterpret_cast<u16x4 *>(o.Ybf + at) = w;
+            else
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (e < left) o.Ybf[at + e] = w[e];
+        }
+        if (o.Yf) {
+            if (vec_f && left >= 4) *reinterpret_cast<float4 *>(o.Yf + at) = float4{y[0], y[1], y[2], y[3]};
+            else
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (e < left) o.Yf[at + e] = y[e];
+        }
+    }
+    if (o.hd.out && q == 3 && in_vol) o.hd.out[vox] = sum + o.hd.b[0];
+}
+
+// This lane's biases and head weights.
+template <int NBW>
+__device__ __forceinline__ void conv_bias(float (&bn)[NBW][4], float (&hw)[NBW][4], const ConvDims &d, const ConvOut &o,
+                                          int n0, int q)
+{
+#pragma unroll
+    for (int j = 0; j < NBW; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int n = n0 + 16 * j + 4 * q + e;
+            bn[j][e] = (o.bias && n < d.cout) ? o.bias[n] : 0.0f;
+            hw[j][e] = (o.hd.out && n < d.cout) ? bf2f(o.hd.w[n]) : 0.0f;
+        }
+}
+
+// Tiles of 8 x 8 x 4 / KW voxels: a slice per wavefront (KW = 1), or KW wavefronts share
+// one, each with 4 / KW of its four blocks of 16 voxels.
+// Bound by the latency of a workgroup's chain (halo, K steps in order, epilogue), so a layer
+// is cut into CONV_WANTED workgroups where it has them: 128 -> 128 channels on four samples
+// of 4 x 8 x 8 voxels 67 us with 16 workgroups of 128 x 64 outputs, 19 with 128 of 64 x 16;
+// 192 -> 64 on four of 8 x 16 x 16 103 -> 45.  (Splitting K over the wavefronts gave 13 and
+// 20, but the sums' order would change the bf16 outputs.)  1024 workgroups: 48 -> 64 us on
+// the layers of 32 x 32 channels.
+template <int TAPS, int NBW, int KW>
+__global__ __launch_bounds__(256, NBW == 1 ? (KW == 2 ? 3 : 4) : NBW == 2 ? 3 : 2) void k_conv(ConvIn in, const unsigned short *__restrict__ Wt, ConvDims d,
+                                              ConvTile T, ConvOut o)
+{
+    constexpr int R = TAPS == 27 ? 1 : 0, CZ = 4 / KW, RB = 4 / KW;
+    constexpr int EX = CX + 2 * R, HV = halo_voxels(R, CZ);
+    constexpr int U = (HV * 4 + 255) / 256;   // 16-byte halo loads of a thread
     extern __shared__ u16x8 halo[];
     // the hardware deals workgroup i to XCD i % 8: give every XCD a contiguous
     // run of tiles, so that the halos neighbouring tiles share hit its L2
     const int per = gridDim.x >> 3;
     const int b = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if (b >= T.nblk) return;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kw = wave % KW, zw = wave / KW;
     const int col = lane & 15, q = lane >> 4;
     const int bx = b % T.ntx, by = (b / T.ntx) % T.nty, bz = b / (T.ntx * T.nty);
-    const int x0 = bx * T.tx, y0 = by * T.ty, z0 = bz * T.tz;
-    const int zs0 = (z0 / T.Ds) * T.Ds;   // first slice of the tile's sample
-    const int hx = T.tx + 2 * R, hy = T.ty + 2 * R, hz = T.tz + 2 * R;
-    const int hyx = hx * hy, HV = hyx * hz;
-    const int txy = T.tx * T.ty, nvox = txy * T.tz;
+    const int zs0 = (bz / T.ntz) * T.Ds, zs1 = zs0 + T.Ds;   // the tile's sample
+    const int x0 = bx * CX, y0 = by * CX, z0 = zs0 + (bz % T.ntz) * CZ;
     const int n0 = blockIdx.y * 16 * NBW;
-    const int Hc = d.H >> 1, Wc = d.W >> 1;
-    // this lane's A rows (clamped into the tile; rows past it are not stored)
-    int hb[2];
+    f32x4 acc[RB][NBW];
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-        const int tv = min(wave * 32 + r * 16 + col, nvox - 1);
-        const int ltz = idiv(tv, txy, T.inv_txy), rem = tv - ltz * txy;
-        const int lty = idiv(rem, T.tx, T.inv_tx), ltx = rem - lty * T.tx;
-        hb[r] = (ltz * hy + lty) * hx + ltx;
-    }
-    f32x4 acc[2][NBW];
-#pragma unroll
-    for (int r = 0; r < 2; ++r)
+    for (int r = 0; r < RB; ++r)
 #pragma unroll
         for (int j = 0; j < NBW; ++j) acc[r][j] = f32x4{0, 0, 0, 0};
     const int64_t tap_stride = (int64_t)d.cout_p * d.cin_p;
-    const int nb_stride = 16 * d.cin_p;
+    // log2 of the 8-channel groups of the chunk at c (a chunk lies in one input)
+    auto groups = [&](int c) {
+        const int left = ((c < in.cc ? in.cc : d.cin_p) - c) >> 3;
+        return left >= 4 ? 2 : left >= 2 ? 1 : 0;
+    };
+    // thread i stages items i, i + 256, ...: 8-channel group g of halo voxel hv
+    u16x8 v[U];
+    auto load = [&](int c0, int lg) {
+        HaloSrc h = halo_source(in, d, c0);
+        h.zs0 = zs0;
+        h.zs1 = zs1;
+        const int g = threadIdx.x & ((1 << lg) - 1);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int hv = ((int)threadIdx.x + 256 * u) >> lg;
+            v[u] = halo_fetch(h, x0 + hv % EX - R, y0 + (hv / EX) % EX - R, z0 + hv / (EX * EX) - R, g, hv < HV);
+        }
+    };
+    constexpr bool AHEAD = KW > 1;
+    int lg = groups(0);
+    if (AHEAD) load(0, lg);
     for (int c0 = 0; c0 < d.cin_p;) {
-        const bool up = c0 < in.cc;   // a chunk lies wholly in one of the two inputs
-        const int left = ((up ? in.cc : d.cin_p) - c0) >> 3;
-        const int lg = left >= 4 ? 2 : left >= 2 ? 1 : 0;   // log2 of the chunk's 8-channel groups
         const int ng = 1 << lg, gp = ng | 1;
-        const unsigned short *src = up ? in.coarse + c0 : in.fine + (c0 - in.cc);
-        const int stride = up ? in.cc : d.cin_p - in.cc;
-        // thread i stages items i, i + 256, ... (item = 8-channel group g of
-        // halo voxel hv); the halo coordinates advance by a fixed step per pass
-        const int g = threadIdx.x & (ng - 1);
-        const int dv = 256 >> lg;                                  // voxels per pass
-        const int sa = dv / hyx, sb = (dv - sa * hyx) / hx, sc = dv - sa * hyx - sb * hx;
-        int hv = threadIdx.x >> lg;
-        int hzi = idiv(hv, hyx, T.inv_hyx);
-        int hyi = idiv(hv - hzi * hyx, hx, T.inv_hx);
-        int hxi = hv - hzi * hyx - hyi * hx;
-        __syncthreads();   // the previous chunk's reads are done
-        while (hv < HV) {
-            u16x8 v[STAGE];
-            int dst[STAGE];
+        if (!AHEAD) load(c0, lg);
+        if (c0 > 0) __syncthreads();   // the previous chunk's reads are done
 #pragma unroll
-            for (int u = 0; u < STAGE; ++u) {
-                v[u] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-                dst[u] = hv < HV ? hv * gp + g : -1;
-                const int gx = x0 + hxi - R, gy = y0 + hyi - R, gz = z0 + hzi - R;
-                if (hv < HV && (unsigned)gx < (unsigned)d.W && (unsigned)gy < (unsigned)d.H && gz >= zs0 &&
-                    gz < zs0 + T.Ds) {
-                    const int vox = up ? ((gz >> 1) * Hc + (gy >> 1)) * Wc + (gx >> 1) : (gz * d.H + gy) * d.W + gx;
-                    v[u] = *reinterpret_cast<const u16x8 *>(src + ((unsigned)vox * (unsigned)stride + 8 * g));
-                }
-                hv += dv;
-                hxi += sc;
-                hyi += sb;
-                hzi += sa;
-                if (hxi >= hx) {
-                    hxi -= hx;
-                    ++hyi;
-                }
-                if (hyi >= hy) {
-                    hyi -= hy;
-                    ++hzi;
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < STAGE; ++u)
-                if (dst[u] >= 0) halo[dst[u]] = v[u];
+        for (int u = 0; u < U; ++u) {
+            const int hv = ((int)threadIdx.x + 256 * u) >> lg;
+            if (hv < HV) halo[hv * gp + (threadIdx.x & (ng - 1))] = v[u];
         }
-        __syncthreads();
-        const unsigned short *wl = Wt + (int64_t)(n0 + col) * d.cin_p + c0;
+        // the next chunk is loaded while this one is multiplied
+        const int next = c0 + 8 * ng, lnext = next < d.cin_p ? groups(next) : 0;
+        if (AHEAD && next < d.cin_p) load(next, lnext);
+        const int v0 = (zw * EX + 2 * RB * kw + (col >> 3)) * EX + (col & 7);
+        const unsigned short *wl = Wt + (int64_t)n0 * d.cin_p + c0;
         if (lg == 2)
-            conv_chunk<TAPS, 4, NBW>(halo, hb, gp, hx, hyx, wl, tap_stride, nb_stride, q, acc);
+            conv_chunk<TAPS, 4, NBW, RB, 8>(halo, v0, 0, wl, tap_stride, d.cin_p, col, q, acc);
         else if (lg == 1)
-            conv_chunk<TAPS, 2, NBW>(halo, hb, gp, hx, hyx, wl, tap_stride, nb_stride, q, acc);
+            conv_chunk<TAPS, 2, NBW, RB, 8>(halo, v0, 0, wl, tap_stride, d.cin_p, col, q, acc);
         else
-            conv_chunk<TAPS, 1, NBW>(halo, hb, gp, hx, hyx, wl, tap_stride, nb_stride, q, acc);
-        c0 += 8 * ng;
+            conv_chunk<TAPS, 1, NBW, RB, 8>(halo, v0, 0, wl, tap_stride, d.cin_p, col, q, acc);
+        c0 = next;
+        lg = lnext;
     }
-    // Epilogue through LDS: the wavefront's 32 x 16 NBW block (bias and
-    // activation applied) goes to LDS in the MFMA layout (lane l holds column
-    // l % 16, rows 4 (l / 16) + i of each 16 x 16 block) and comes back row by
-    // row, so that consecutive lanes store consecutive bytes: 16-byte groups
-    // of 8 bf16 / 4 float channels where the row layout allows, else single
-    // values (the 1-channel head: one value per voxel, consecutive voxels).
-    constexpr int RL = 16 * NBW + 1;   // floats per LDS row
-    __syncthreads();                   // every wavefront is done with the halo
-    float *cbuf = reinterpret_cast<float *>(halo) + wave * (32 * RL + 64);
-    int64_t *orow = reinterpret_cast<int64_t *>(cbuf + 32 * RL);   // row -> global offset
+    const int gz = z0 + zw, gx = x0 + (col & 7);
+    float bn[NBW][4], hw[NBW][4];
+    conv_bias(bn, hw, d, o, n0, q);
 #pragma unroll
-    for (int j = 0; j < NBW; ++j) {
-        const int n = n0 + 16 * j + col;
-        const float bn = (bias && n < d.cout) ? bias[n] : 0.0f;
-#pragma unroll
-        for (int r = 0; r < 2; ++r)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float v = acc[r][j][i] + bn;
-                if (d.slope >= 0.0f && v < 0.0f) v *= d.slope;
-                cbuf[(r * 16 + 4 * q + i) * RL + 16 * j + col] = v;
-            }
-    }
-    // global offset of each row of this wavefront, -1 outside the volume
-    int myvox = -1;
-    if (lane < 32) {
-        const int tv = wave * 32 + lane;
-        const int ltz = idiv(tv, txy, T.inv_txy), rem = tv - ltz * txy;
-        const int lty = idiv(rem, T.tx, T.inv_tx), ltx = rem - lty * T.tx;
-        const int gx = x0 + ltx, gy = y0 + lty, gz = z0 + ltz;
-        if (tv < nvox && gx < d.W && gy < d.H) myvox = (gz * d.H + gy) * d.W + gx;
-        orow[lane] = myvox >= 0 ? (int64_t)myvox * d.out_stride + d.out_off + n0 : -1;
-    }
-    __syncthreads();   // LDS writes visible to the whole wavefront
-    if (hd.out && myvox >= 0) {
-        // the head on this lane's row: products of bf16 values are exact in float
-        const float *src = cbuf + lane * RL;
-        float sum = 0.0f;
-        for (int c = 0; c < d.cout; ++c) sum += bf2f(f2bf(src[c])) * bf2f(hd.w[c]);
-        hd.out[myvox] = sum + hd.b[0];
-    }
-    const int cvalid = min(16 * NBW, d.cout - n0);   // channels of this block to store
-    const bool vec_bf = Ybf && (cvalid % 8 == 0) && ((d.out_stride | d.out_off | n0) % 8 == 0) &&
-                        !(reinterpret_cast<uintptr_t>(Ybf) & 15);
-    const bool vec_f = Yf && (cvalid % 4 == 0) && ((d.out_stride | d.out_off | n0) % 4 == 0) &&
-                       !(reinterpret_cast<uintptr_t>(Yf) & 15);
-    if (Ybf) {
-        const int per = vec_bf ? cvalid >> 3 : cvalid;          // items per row
-        const float inv = 1.0f / (float)per;
-        const int sh = (per & (per - 1)) ? -1 : __builtin_ctz(per);
-        for (int e = lane; e < 32 * per; e += 64) {
-            const int row = sh >= 0 ? e >> sh : idiv(e, per, inv), k = e - row * per;
-            const int64_t o = orow[row];
-            if (o < 0) continue;
-            const float *src = cbuf + row * RL;
-            if (vec_bf) {
-                u16x8 w;
-#pragma unroll
-                for (int c = 0; c < 8; ++c) w[c] = f2bf(src[8 * k + c]);
-                *reinterpret_cast<u16x8 *>(Ybf + o + 8 * k) = w;
-            } else {
-                Ybf[o + k] = f2bf(src[k]);
-            }
-        }
-    }
-    if (Yf) {
-        const int per = vec_f ? cvalid >> 2 : cvalid;
-        const float inv = 1.0f / (float)per;
-        const int sh = (per & (per - 1)) ? -1 : __builtin_ctz(per);
-        for (int e = lane; e < 32 * per; e += 64) {
-            const int row = sh >= 0 ? e >> sh : idiv(e, per, inv), k = e - row * per;
-            const int64_t o = orow[row];
-            if (o < 0) continue;
-            const float *src = cbuf + row * RL;
-            if (vec_f)
-                *reinterpret_cast<float4 *>(Yf + o + 4 * k) =
-                    float4{src[4 * k], src[4 * k + 1], src[4 * k + 2], src[4 * k + 3]};
-            else
-                Yf[o + k] = src[k];
-        }
+    for (int r = 0; r < RB; ++r) {
+        const int gy = y0 + 2 * (RB * kw + r) + (col >> 3);
+        conv_store(acc[r], bn, hw, d, o, n0, q, (unsigned)((gz * d.H + gy) * d.W + gx), gx < d.W && gy < d.H && gz < zs1);
     }
 }
 
-// Tile of k_conv for samples of Ds x H x W: x first (up to 32), then y, then z
-// (a divisor of Ds), at most 128 voxels, and a halo that fits CONV_LDS_MAX
-// with 5 padded 16-byte words per voxel.
-static void conv_tile(int Ds, int H, int W, int R, ConvTile &T)
+// k_conv for larger volumes: tiles of 16 x 8 x 4 voxels, a slice per wavefront and a row of
+// 16 voxels per MFMA, so that a weight read serves eight products and the halo is 2.1
+// times the tile (2.3).  A voxel's channel groups lie side by side, with 32 channels
+// exchanged by x so that eight voxels in a row are in different banks.
+// Bound by latency and LDS reads.  96 -> 32 channels on 32 samples of 16 x 32 x 32: 99 us
+// (176 with k_conv's tiles), 192 -> 64 on 32 of 8 x 16 x 16: 74 (98).
+template <int NBW>
+__global__ __launch_bounds__(256, NBW == 1 ? 3 : 2) void k_conv_rows(ConvIn in, const unsigned short *__restrict__ Wt,
+                                                                     ConvDims d, ConvTile T, ConvOut o)
 {
-    T.tx = W < 32 ? W : 32;
-    T.ty = H < CONV_TILE / T.tx ? H : CONV_TILE / T.tx;
-    T.tz = 1;
-    for (int z = CONV_TILE / (T.tx * T.ty); z > 1; --z)
-        if (Ds % z == 0) {
-            T.tz = z;
-            break;
+    constexpr int U = (RHV * 4 + 255) / 256, UB = 9;   // halo loads of a thread; in flight
+    extern __shared__ u16x8 halo[];
+    const int per = gridDim.x >> 3;   // XCD-contiguous tiles, as in k_conv
+    const int b = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (b >= T.nblk) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 15, q = lane >> 4;
+    const int bx = b % T.ntx, by = (b / T.ntx) % T.nty, bz = b / (T.ntx * T.nty);
+    const int zs0 = (bz / T.ntz) * T.Ds, zs1 = zs0 + T.Ds;   // the tile's sample
+    const int x0 = bx * RWX, y0 = by * RWY, z0 = zs0 + (bz % T.ntz) * RWZ;
+    const int n0 = blockIdx.y * 16 * NBW;
+    f32x4 acc[RWY][NBW];
+#pragma unroll
+    for (int r = 0; r < RWY; ++r)
+#pragma unroll
+        for (int j = 0; j < NBW; ++j) acc[r][j] = f32x4{0, 0, 0, 0};
+    const int64_t tap_stride = (int64_t)d.cout_p * d.cin_p;
+    const int v0 = wave * RHX * RHY + col;
+    for (int c0 = 0; c0 < d.cin_p;) {
+        const int left = ((c0 < in.cc ? in.cc : d.cin_p) - c0) >> 3;
+        const int lg = left >= 4 ? 2 : left >= 2 ? 1 : 0, ng = 1 << lg;
+        HaloSrc h = halo_source(in, d, c0);
+        h.zs0 = zs0;
+        h.zs1 = zs1;
+        const int g = threadIdx.x & (ng - 1);
+        if (c0 > 0) __syncthreads();   // the previous chunk's reads are done
+#pragma unroll
+        for (int u0 = 0; u0 < U; u0 += UB) {
+            if (((256 * u0) >> lg) >= RHV) break;
+            u16x8 v[UB];
+#pragma unroll
+            for (int u = 0; u < UB; ++u) {
+                const int hv = ((int)threadIdx.x + 256 * (u0 + u)) >> lg;
+                v[u] = halo_fetch(h, x0 + hv % RHX - 1, y0 + (hv / RHX) % RHY - 1, z0 + hv / (RHX * RHY) - 1, g, hv < RHV);
+            }
+#pragma unroll
+            for (int u = 0; u < UB; ++u) {
+                const int hv = ((int)threadIdx.x + 256 * (u0 + u)) >> lg;
+                if (hv < RHV) halo[hv * ng + (lg == 2 ? row_slot<4>(g, hv % RHX) : g)] = v[u];
+            }
         }
-    auto bytes = [&] { return (T.tx + 2 * R) * (T.ty + 2 * R) * (T.tz + 2 * R) * 5 * 16; };
-    while (bytes() > CONV_LDS_MAX && T.tz > 1) {
-        int z = T.tz - 1;
-        while (Ds % z) --z;
-        T.tz = z;
+        const unsigned short *wl = Wt + (int64_t)n0 * d.cin_p + c0;
+        if (lg == 2) conv_chunk<27, 4, NBW, RWY, 16>(halo, v0, col, wl, tap_stride, d.cin_p, col, q, acc);
+        else if (lg == 1) conv_chunk<27, 2, NBW, RWY, 16>(halo, v0, col, wl, tap_stride, d.cin_p, col, q, acc);
+        else conv_chunk<27, 1, NBW, RWY, 16>(halo, v0, col, wl, tap_stride, d.cin_p, col, q, acc);
+        c0 += 8 * ng;
     }
-    while (bytes() > CONV_LDS_MAX && T.ty > 1) --T.ty;
-    T.ntx = (W + T.tx - 1) / T.tx;
-    T.nty = (H + T.ty - 1) / T.ty;
-    T.Ds = Ds;
-    T.nblk = 0;
-    const int hx = T.tx + 2 * R, hy = T.ty + 2 * R;
-    T.inv_hx = 1.0f / (float)hx;
-    T.inv_hyx = 1.0f / (float)(hx * hy);
-    T.inv_tx = 1.0f / (float)T.tx;
-    T.inv_txy = 1.0f / (float)(T.tx * T.ty);
+    const int gx = x0 + col, gz = z0 + wave;
+    float bn[NBW][4], hw[NBW][4];
+    conv_bias(bn, hw, d, o, n0, q);
+#pragma unroll
+    for (int r = 0; r < RWY; ++r) {
+        const int gy = y0 + r;
+        conv_store(acc[r], bn, hw, d, o, n0, q, (unsigned)((gz * d.H + gy) * d.W + gx), gx < d.W && gy < d.H && gz < zs1);
+    }
+}
+
+// k_conv_rows for 16 output channels whose weights fit in LDS beside the halo (the layers
+// at full resolution): chunks of NG0 and NG1 groups of 8 input channels (NG1 = 0: one
+// chunk).  The weights are laid there once, as the fragments the lanes read; the
+// workgroups stay and walk runs of tiles of 16 x 8 x 8 voxels (eight wavefronts, a slice
+// each), and the next chunk's halo is loaded into registers while this one is multiplied:
+// no load is waited for inside a chunk.  LDS: 115 KB of halo with 32 channels (one
+// workgroup on a CU), 58 KB with 16 (two).
+// Bound by MFMA and vector issue together (48 -> 16 channels: 72 us of products and 50 of
+// other instructions in 223).  32 samples of 32 x 64 x 64: 8 -> 16 channels 70 us, 16 -> 16
+// 90 (floor by bytes 42 and 56), 48 -> 16 223, 16 -> 16 with the head 118; with tiles of
+// 128 voxels, weights from global memory and every load waited for these were 193, 226,
+// 560 and 255.
+constexpr int RSZ = 8, RSV = RHX * RHY * (RSZ + 2);
+constexpr int RES_CUS = 256;   // workgroups at a time, one a CU
+constexpr int res_frags(int ng) { return (27 * ng + 3) / 4; }   // of a chunk
+constexpr size_t res_lds(int ng0, int ng1) { return (size_t)RSV * ng0 * 16 + 1024 * (res_frags(ng0) + res_frags(ng1)); }
+static_assert(res_lds(4, 2) + 128 <= 160 * 1024 && 2 * (res_lds(2, 0) + 128) <= 160 * 1024, "workgroups of a CU");
+
+// The halo of one chunk between memory and LDS, by the eight wavefronts.  Rows of the
+// tile's 16 columns are whole loads (4 / NG rows of 16 columns a wavefront), so that most
+// of a place and its test are scalar; the two outer columns follow as items of their own.
+template <int NG>
+struct HaloStage {
+    static constexpr int UM = NG == 4 ? 13 : NG == 2 ? 7 : 4;           // row loads of a wavefront
+    static constexpr int EDGE = 2 * NG * RHY * (RSZ + 2), UE = (EDGE + 511) / 512;
+    static constexpr int U = UM + UE;
+
+    // Halo row y, slice z of load u (z past the tile: none); rs: the lane's row of the load.
+    static __device__ __forceinline__ void row(int u, int wave, int rs, int &y, int &z)
+    {
+        if (NG == 4) {          // rows 0-7 one per wavefront, rows 8 and 9 of all slices after them
+            const int r = wave + 8 * (u - 10);
+            y = u < 10 ? wave : 8 + (r & 1);
+            z = u < 10 ? u : r >> 1;
+        } else if (NG == 2) {   // row pairs 0-3 of two slices, then pair 4 of eight
+            y = (u < 5 ? 2 * (wave & 3) : 8) + rs;
+            z = u < 5 ? 2 * u + (wave >> 2) : wave + 8 * (u - 5);
+        } else {                // rows 0-3 and 4-7 of four slices, then rows 8 and 9 of two a wavefront
+            y = u < 3 ? 4 * (wave & 1) + rs : 8 + (rs & 1);
+            z = u < 3 ? (wave >> 1) + 4 * u : 2 * wave + (rs >> 1);
+        }
+    }
+
+    static __device__ __forceinline__ void load(const HaloSrc &s, int lane, int wave, u16x8 (&v)[U])
+    {
+        const int g = lane & (NG - 1), gx = s.x0 + ((lane / NG) & 15), rs = lane / (16 * NG);
+#pragma unroll
+        for (int u = 0; u < UM; ++u) {
+            int y, z;
+            row(u, wave, rs, y, z);
+            v[u] = halo_fetch(s, gx, s.y0 + y - 1, s.z0 + z - 1, g, z < RSZ + 2);
+        }
+#pragma unroll
+        for (int u = 0; u < UE; ++u) {
+            const int e = (int)threadIdx.x + 512 * u, r = e / (2 * NG), x = s.x0 + ((e / NG) & 1 ? RWX : -1);
+            v[UM + u] = halo_fetch(s, x, s.y0 + r % RHY - 1, s.z0 + r / RHY - 1, e & (NG - 1), e < EDGE);
+        }
+    }
+
+    static __device__ __forceinline__ void store(u16x8 *halo, int lane, int wave, const u16x8 (&v)[U])
+    {
+        const int g = lane & (NG - 1), x = ((lane / NG) & 15) + 1, rs = lane / (16 * NG);
+        u16x8 *mine = halo + x * NG + row_slot<NG>(g, x);
+#pragma unroll
+        for (int u = 0; u < UM; ++u) {
+            int y, z;
+            row(u, wave, rs, y, z);
+            if (z < RSZ + 2) mine[(z * RHY + y) * RHX * NG] = v[u];
+        }
+#pragma unroll
+        for (int u = 0; u < UE; ++u) {
+            const int e = (int)threadIdx.x + 512 * u, hx = (e / NG) & 1 ? RHX - 1 : 0;
+            if (e < EDGE) halo[(e / (2 * NG) * RHX + hx) * NG + row_slot<NG>(e & (NG - 1), hx)] = v[UM + u];
+        }
+    }
+};
+
+// The weights of the NG groups from channel c0 on, as the fragments of conv_chunk's steps.
+template <int NG>
+__device__ __forceinline__ void res_weights(u16x8 *wf, const unsigned short *__restrict__ W, const ConvDims &d, int n0, int c0)
+{
+    constexpr int K = 4 / NG;
+    for (int i = threadIdx.x; i < res_frags(NG) * 64; i += 512) {
+        const int col = i & 15, q = (i >> 4) & 3, t = K * (i >> 6) + q / NG;
+        u16x8 w = {0, 0, 0, 0, 0, 0, 0, 0};
+        if (t < 27)
+            w = *reinterpret_cast<const u16x8 *>(W + t * d.cout_p * d.cin_p + (n0 + col) * d.cin_p + c0 +
+                                                 8 * (q & (NG - 1)));
+        wf[i] = w;
+    }
+}
+
+// conv_chunk's sums in its order.  Reads are issued AHEAD places before their use (the
+// order is fixed: left to itself the compiler reads and waits).
+template <int NG>
+__device__ __forceinline__ void conv_res_chunk(const u16x8 *halo, const u16x8 *wf, int lane, int wave,
+                                               f32x4 (&acc)[RWY])
+{
+    constexpr int EXY = RHX * RHY;
+    const int col = lane & 15, q = lane >> 4;
+    int g = q & (NG - 1), tq = q / NG;
+    asm volatile("" : "+v"(g), "+v"(tq));   // addresses are not kept across the chunks
+    const u16x8 *h = halo + (wave * EXY + col) * NG;
+    auto product = [&](const u16x8 &w, const u16x8 &a, int r) {
+        acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, a),
+                                                         acc[r], 0, 0, 0);
+    };
+    if constexpr (NG == 4) {
+        // Per dz the nine weights, then the ten rows of the halo, each at the three dx: what
+        // is read for (y, dx) serves the outputs y, y - 1 and y - 2 (with dy = 0, 1 and 2),
+        // and an output meets its taps in order.  39 reads for 72 products.
+        constexpr int AHEAD = 4;
+        u16x8 w[9], a[2 * AHEAD];
+        const u16x8 *p[3];
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) p[dx] = h + dx * NG + row_slot<NG>(g, col + dx);
+        auto rows = [&](int dz, int k) { a[k % (2 * AHEAD)] = p[k % 3][(dz * EXY + k / 3 * RHX) * NG]; };
+#pragma unroll
+        for (int dz = 0; dz < 3; ++dz) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) w[k] = wf[(9 * dz + k) * 64 + lane];
+#pragma unroll
+            for (int k = 0; k < AHEAD; ++k) rows(dz, k);
+#pragma unroll
+            for (int k = 0; k < 3 * RHY; ++k) {
+                const int y = k / 3, dx = k % 3;
+                if (k < 6) w[3 + k] = wf[(9 * dz + 3 + k) * 64 + lane];   // dy = 1 and 2: first used at y = 1 and 2
+                if (k + AHEAD < 3 * RHY) rows(dz, k + AHEAD);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int dy = 0; dy < 3; ++dy)
+                    if (y - dy >= 0 && y - dy < RWY) product(w[3 * dy + dx], a[k % (2 * AHEAD)], y - dy);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    } else {
+        // A step's two or four taps are picked per lane: a weight and eight rows a step.
+        constexpr int K = 4 / NG, S = (27 + K - 1) / K, AHEAD = 3, PER = 1 + RWY;
+        u16x8 w[2], a[2][RWY];
+        const u16x8 *p = nullptr;
+        auto read = [&](int i) {
+            const int s = i / PER, k = i % PER;
+            if (k == 0) {
+                w[s & 1] = wf[s * 64 + lane];
+                int delta = tap_delta<27>(K * s, RHX, EXY);
+#pragma unroll
+                for (int m = 1; m < K; ++m)
+                    delta = tq == m ? tap_delta<27>(K * s + m < 27 ? K * s + m : 26, RHX, EXY) : delta;
+                p = h + delta * NG + g;
+                return;
+            }
+            a[s & 1][k - 1] = p[(k - 1) * RHX * NG];
+            if (K * s + K > 27 && K * s + tq >= 27) a[s & 1][k - 1] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};   // the weights are zero there too
+        };
+#pragma unroll
+        for (int i = 0; i < 1 + AHEAD; ++i) read(i);
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+#pragma unroll
+            for (int r = 0; r < RWY; ++r) {
+                const int i = PER * s + 1 + r + AHEAD;
+                if (r == RWY - AHEAD && i < PER * S) read(i);   // the next step's weight
+                if (r >= RWY - AHEAD ? i + 1 < PER * S : true) read(r >= RWY - AHEAD ? i + 1 : i);
+                __builtin_amdgcn_sched_barrier(0);
+                product(w[s & 1], a[s & 1][r], r);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+    }
+}
+
+template <int NG0, int NG1>
+__global__ __launch_bounds__(512, NG0 == 4 ? 2 : 4) void k_conv_res(ConvIn in, const unsigned short *__restrict__ Wt,
+                                                                    ConvDims d, ConvTile T, int run, ConvOut o)
+{
+    constexpr int NGB = NG1 ? NG1 : NG0;
+    __shared__ u16x8 lds[res_lds(NG0, NG1) / 16];
+    __shared__ float4 ends[2][4];
+    u16x8 *halo = lds, *wf0 = lds + RSV * NG0, *wf1 = wf0 + 64 * res_frags(NG0);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 15, q = lane >> 4;
+    // contiguous runs of tiles on every XCD
+    const int b = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    const int t1 = min(T.nblk, (b + 1) * run);
+    int tile = b * run;
+    if (tile >= t1) return;
+    const int n0 = 16 * blockIdx.y;
+    res_weights<NG0>(wf0, Wt, d, n0, 0);
+    if constexpr (NG1 > 0) res_weights<NG1>(wf1, Wt, d, n0, 8 * NG0);
+    if (wave == 0) {   // biases and head weights of the lanes: not held in registers
+        float bn[1][4], hw[1][4];
+        conv_bias(bn, hw, d, o, n0, q);
+        if (col == 0) {
+            ends[0][q] = float4{bn[0][0], bn[0][1], bn[0][2], bn[0][3]};
+            ends[1][q] = float4{hw[0][0], hw[0][1], hw[0][2], hw[0][3]};
+        }
+    }
+    auto place = [&](int t, HaloSrc &h) {
+        const int bx = t % T.ntx, by = (t / T.ntx) % T.nty, bz = t / (T.ntx * T.nty);
+        h.zs0 = (bz / T.ntz) * T.Ds;   // the tile's sample
+        h.zs1 = h.zs0 + T.Ds;
+        h.x0 = bx * RWX;
+        h.y0 = by * RWY;
+        h.z0 = h.zs0 + (bz % T.ntz) * RSZ;
+    };
+    HaloSrc h0 = halo_source(in, d, 0), h1 = halo_source(in, d, NG1 ? 8 * NG0 : 0);
+    u16x8 v0[HaloStage<NG0>::U], v1[HaloStage<NGB>::U];
+    place(tile, h0);
+    HaloStage<NG0>::load(h0, lane, wave, v0);
+    for (; tile < t1; ++tile) {
+        f32x4 acc[RWY];
+#pragma unroll
+        for (int r = 0; r < RWY; ++r) acc[r] = f32x4{0, 0, 0, 0};
+        const int gx = h0.x0 + col, gy0 = h0.y0, gz = h0.z0 + wave;
+        const bool inside = gx < d.W && gz < h0.zs1;
+        __syncthreads();   // the previous chunk's reads are done
+        HaloStage<NG0>::store(halo, lane, wave, v0);
+        if constexpr (NG1 > 0) {
+            place(tile, h1);
+            HaloStage<NGB>::load(h1, lane, wave, v1);
+        } else {
+            place(min(tile + 1, t1 - 1), h0);
+            HaloStage<NG0>::load(h0, lane, wave, v0);
+        }
+        __syncthreads();   // the halo (and, at first, the weights) are there
+        conv_res_chunk<NG0>(halo, wf0, lane, wave, acc);
+        if constexpr (NG1 > 0) {
+            __syncthreads();
+            HaloStage<NGB>::store(halo, lane, wave, v1);
+            place(min(tile + 1, t1 - 1), h0);
+            HaloStage<NG0>::load(h0, lane, wave, v0);
+            __syncthreads();
+            conv_res_chunk<NGB>(halo, wf1, lane, wave, acc);
+        }
+        const float4 bq = ends[0][q], hq = ends[1][q];
+        const float bn[1][4] = {{bq.x, bq.y, bq.z, bq.w}}, hw[1][4] = {{hq.x, hq.y, hq.z, hq.w}};
+#pragma unroll
+        for (int r = 0; r < RWY; ++r) {
+            const f32x4 a[1] = {acc[r]};
+            conv_store(a, bn, hw, d, o, n0, q, (unsigned)((gz * d.H + gy0 + r) * d.W + gx), inside && gy0 + r < d.H);
+        }
+    }
 }
 
 // Weight gradient of one tap: dW[t][co][ci] += sum_v dY[v][co] * X[v + o_t][ci]
@@ -885,31 +1204,96 @@ static int conv_launch(ConvIn in, const void *w, const float *bias, int32_t N, i
         return SRF_ERR_UNSUPPORTED;
     ConvDims d{N * D, H, W, cin_p, cout, cout_p, out_stride, out_off, taps, slope};
     const int R = taps == 27 ? 1 : 0;
-    ConvTile T;
-    conv_tile(D, H, W, R, T);
-    T.nblk = T.ntx * T.nty * (N * D / T.tz);
     const int nb = (cout + 15) / 16;
-    const int nbw = (nb >= 4 && cout_p % 64 == 0) ? 4 : nb >= 2 ? 2 : 1;
+    const int widest = (nb >= 4 && cout_p % 64 == 0) ? 4 : nb >= 2 ? 2 : 1;
+    if (hd.out && (nb > widest || !hd.w || !hd.b)) return SRF_ERR_UNSUPPORTED;   // the head needs every channel
+    auto *ws = (const unsigned short *)w;
+    auto st = (hipStream_t)stream;
+    const ConvOut o{bias, (unsigned short *)y_bf16, y_f32, hd};
+    // k_conv_res: up to three blocks of outputs (each reads the halo again: 16 -> 48 channels
+    // 47 us, 76 in k_conv), chunks that it has, at most a quarter more voxels by padding to
+    // its tiles (beyond that k_conv's 8 x 8 ones do less work) and two tiles for every CU.
+    int ng[3] = {0, 0, 0}, nch = 0;
+    for (int c = 0; c < cin_p && nch < 3; ++nch) {
+        const int left = ((c < in.cc ? in.cc : cin_p) - c) >> 3;
+        ng[nch] = left >= 4 ? 4 : left >= 2 ? 2 : 1;
+        c += 8 * ng[nch];
+    }
+    const int64_t stx = (W + RWX - 1) / RWX, stz = (D + RSZ - 1) / RSZ, sblk = stx * ((H + RWY - 1) / RWY) * stz * N;
+    const int kind = ng[2] ? 0 : 10 * ng[0] + ng[1];
+    if (taps == 27 && nb <= 3 && (!hd.out || nb == 1) && (kind == 10 || kind == 20 || kind == 40 || kind == 42) && 4 * stx * RWX <= 5 * W &&
+        4 * stz * RSZ <= 5 * D && sblk >= 2 * RES_CUS) {
+        ConvTile T;
+        T.ntx = (int)stx;
+        T.nty = (H + RWY - 1) / RWY;
+        T.ntz = (int)stz;
+        T.Ds = D;
+        T.nblk = (int)sblk;
+        const int wgs = (ng[0] == 4 ? RES_CUS : 2 * RES_CUS) / nb / 8 * 8, run = (int)((sblk + wgs - 1) / wgs);
+        const dim3 grid((unsigned)wgs, (unsigned)nb);
+        if (kind == 42) hipLaunchKernelGGL((k_conv_res<4, 2>), grid, dim3(512), 0, st, in, ws, d, T, run, o);
+        else if (kind == 40) hipLaunchKernelGGL((k_conv_res<4, 0>), grid, dim3(512), 0, st, in, ws, d, T, run, o);
+        else if (kind == 20) hipLaunchKernelGGL((k_conv_res<2, 0>), grid, dim3(512), 0, st, in, ws, d, T, run, o);
+        else hipLaunchKernelGGL((k_conv_res<1, 0>), grid, dim3(512), 0, st, in, ws, d, T, run, o);
+        return launch_status();
+    }
+    // k_conv_rows from a workgroup for every CU on (half as many: 31 us for 26 in k_conv)
+    const int rbw = nb % 2 == 0 ? 2 : 1;
+    const int64_t rtx = (W + RWX - 1) / RWX, rblk = rtx * ((H + RWY - 1) / RWY) * ((D + RWZ - 1) / RWZ) * N;
+    if (taps == 27 && 4 * rtx * RWX <= 5 * W && rblk * (nb / rbw) >= ROWS_WANTED && (!hd.out || nb <= rbw)) {
+        ConvTile T;
+        T.ntx = (int)rtx;
+        T.nty = (H + RWY - 1) / RWY;
+        T.ntz = (D + RWZ - 1) / RWZ;
+        T.Ds = D;
+        T.nblk = (int)rblk;
+        const int ng = cin_p >= 32 ? 4 : cin_p >= 16 ? 2 : 1;
+        const size_t lds = (size_t)RHV * ng * 16;
+        dim3 grid((unsigned)((rblk + 7) / 8 * 8), (unsigned)(nb / rbw));
+        if (rbw == 2) hipLaunchKernelGGL(k_conv_rows<2>, grid, dim3(256), lds, st, in, ws, d, T, o);
+        else hipLaunchKernelGGL(k_conv_rows<1>, grid, dim3(256), lds, st, in, ws, d, T, o);
+        return launch_status();
+    }
+    // CONV_RULE
+    int nbw = widest, kw = 1;
+    auto blocks = [&] {
+        const int cz = 4 / kw;
+        return (int64_t)((W + CX - 1) / CX) * ((H + CX - 1) / CX) * ((D + cz - 1) / cz) * N * ((nb + nbw - 1) / nbw);
+    };
+    if (!hd.out)
+        while (nbw > 1 && blocks() < CONV_WANTED) nbw >>= 1;
+    if (taps == 27)
+        while (kw < 4 && blocks() < CONV_WANTED) kw <<= 1;
+    ConvTile T;
+    T.ntx = (W + CX - 1) / CX;
+    T.nty = (H + CX - 1) / CX;
+    T.ntz = (D + 4 / kw - 1) / (4 / kw);
+    T.Ds = D;
+    T.nblk = T.ntx * T.nty * T.ntz * N;
     const int lg = cin_p >= 32 ? 2 : cin_p >= 16 ? 1 : 0;
-    size_t lds = (size_t)(T.tx + 2 * R) * (T.ty + 2 * R) * (T.tz + 2 * R) * ((1 << lg) | 1) * 16;
-    const size_t lds_epi = (size_t)4 * (32 * (16 * nbw + 1) + 64) * sizeof(float);
-    if (lds < lds_epi) lds = lds_epi;
+    const size_t lds = (size_t)halo_voxels(R, 4 / kw) * ((1 << lg) | 1) * 16;
     // a multiple of 8 workgroups (the XCD-contiguous tile order; extra ones exit)
     dim3 grid((unsigned)((T.nblk + 7) / 8 * 8), (unsigned)((nb + nbw - 1) / nbw));
-    if (hd.out && (grid.y != 1 || !hd.w || !hd.b)) return SRF_ERR_UNSUPPORTED;   // the head needs every channel
-    auto *ws = (const unsigned short *)w;
-    auto *yb = (unsigned short *)y_bf16;
-    auto st = (hipStream_t)stream;
-#define SRF_CONV(TP, NBW) \
-    hipLaunchKernelGGL((k_conv<TP, NBW>), grid, dim3(256), lds, st, in, ws, bias, d, T, yb, y_f32, hd)
+#define SRF_CONV(TP, NBW, KW) \
+    hipLaunchKernelGGL((k_conv<TP, NBW, KW>), grid, dim3(256), lds, st, in, ws, d, T, o)
     if (taps == 27) {
-        if (nbw == 4) SRF_CONV(27, 4);
-        else if (nbw == 2) SRF_CONV(27, 2);
-        else SRF_CONV(27, 1);
+        if (kw == 1) {
+            if (nbw == 4) SRF_CONV(27, 4, 1);
+            else if (nbw == 2) SRF_CONV(27, 2, 1);
+            else SRF_CONV(27, 1, 1);
+        } else if (kw == 2) {
+            if (nbw == 4) SRF_CONV(27, 4, 2);
+            else if (nbw == 2) SRF_CONV(27, 2, 2);
+            else SRF_CONV(27, 1, 2);
+        } else {
+            if (nbw == 4) SRF_CONV(27, 4, 4);
+            else if (nbw == 2) SRF_CONV(27, 2, 4);
+            else SRF_CONV(27, 1, 4);
+        }
     } else {
-        if (nbw == 4) SRF_CONV(1, 4);
-        else if (nbw == 2) SRF_CONV(1, 2);
-        else SRF_CONV(1, 1);
+        if (nbw == 4) SRF_CONV(1, 4, 1);
+        else if (nbw == 2) SRF_CONV(1, 2, 1);
+        else SRF_CONV(1, 1, 1);
     }
 #undef SRF_CONV
     return launch_status();

@@ -116,9 +116,7 @@ class UNet:
                 for l in self.layers}
 
     def zero_grad(self):
-        for l in self.layers:
-            l.gw.zero_()
-            l.gb.zero_()
+        torch._foreach_zero_([t for l in self.layers for t in (l.gw, l.gb)])   # one launch for all
 
     def _sync_weights(self):
         s = stream_handle(self.dev)

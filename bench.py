@@ -142,9 +142,10 @@ def measure_traffic(args):
             # the probe's copy (the process's first) moves TRAFFIC_COPY bytes each way
             factor = TRAFFIC_COPY / (copy * 1024.0)   # bytes moved per counted byte
             for part, kname in TRAFFIC_KERNELS.items():
+                # the step's variant comes last (the sensitivity image is backprojected by another)
                 vals = [v for k, v in means.items() if kname in k]
                 if vals:
-                    res.setdefault(part, {})[counter] = vals[0] * 1024.0 * factor
+                    res.setdefault(part, {})[counter] = vals[-1] * 1024.0 * factor
             res.setdefault("factor", {})[counter] = factor
     out = {part: d["FETCH_SIZE"] + d["WRITE_SIZE"] for part, d in res.items()
            if part != "factor" and "FETCH_SIZE" in d and "WRITE_SIZE" in d}

@@ -6,8 +6,9 @@
  *    The caller owns every buffer; the library allocates device memory only in
  *    srf_plan_create[_ex], srf_plan_rebuild and srf_batch_create (freed by the
  *    matching *_destroy) and transient scratch in srf_sinogram_lors,
- *    srf_event_order, the srf_sss_* entry points and, for long lists outside
- *    graph capture, srf_project and srf_backproject[_ratio], which run without it
+ *    srf_event_order, the srf_sss_* entry points and, outside graph capture,
+ *    srf_plan_project_batch, srf_cnn_conv_wgrad[_batch] and, for long lists,
+ *    srf_project and srf_backproject[_ratio]; these four run without it
  *    where it is not to be had.
  *  - LORs are AoS rows of `lor_stride` floats [x1,y1,z1,x2,y2,z2,(tof,...)] in
  *    mm, exactly Lors.data of srfnef/data/lors.py:12-22 (stride 6 or 7).
@@ -18,7 +19,9 @@
  *    (srfnef/cc/siddon/siddon.cu.cc:95), i.e. the tf.transpose(image.data) that
  *    srfnef/functions/project.py:27 hands to the op.
  *  - `stream` is a hipStream_t (NULL = the legacy default stream).  Every call is
- *    asynchronous on that stream and host-validated before any launch.
+ *    host-validated before any launch and asynchronous on that stream, but for
+ *    those that say otherwise (plan creation and rebuild, srf_backproject of long
+ *    lists).
  *  - Return value: SRF_OK (0) or a negative SRF_ERR_* code; srf_strerror()
  *    names it.
  */
@@ -412,7 +415,9 @@ int srf_cnn_conv_head_batch(const void *x, const void *w, const float *bias, int
                             void *y_bf16, const void *head_w, const float *head_b, float *head_out, void *stream);
 /* dw[t][n][c] += sum_v dy[v][n] x[v + o_t][c]   (dy bf16 rows of dy_stride);
  * the _batch form over N stacked samples, and with db != NULL also
- * db[n] += sum_v dy[v][n] (the bias gradient, as srf_cnn_bias_grad). */
+ * db[n] += sum_v dy[v][n] (the bias gradient, as srf_cnn_bias_grad).  Partial sums
+ * lie in transient scratch (up to 64 MiB) where that can be had, not under graph
+ * capture; without it they are added by atomics. */
 int srf_cnn_conv_wgrad(const void *x, const void *dy, int32_t dy_stride, int32_t D, int32_t H, int32_t W,
                        int32_t cin_p, int32_t cout, int32_t cout_p, int32_t taps, float *dw, void *stream);
 int srf_cnn_conv_wgrad_batch(const void *x, const void *dy, int32_t dy_stride, int32_t N, int32_t D, int32_t H,

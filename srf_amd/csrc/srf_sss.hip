@@ -4,9 +4,8 @@
 // Physics of srfnef/corrections/scattering/scatter_fraction/scatter_fraction.py:
 // 70-131 and kn_formula.py:6-46 (per LOR (A,B), a Klein-Nishina weighted sum
 // over scatter points S of the emission and attenuation line integrals from S
-// to both detectors).  The line integrals come from the projector kernels
-// (srf_project / plans) over the (detector, scatter point) LOR set; this file
-// holds
+// to both detectors).  The line integrals come from srf_sss_integrals (srf_project.hip)
+// or the projector over the (detector, scatter point) LOR set; this file holds
 //   k_sss_pairs   per (detector, scatter point): unit vector S->D, the
 //                 obliquity / distance factor g = ((D-S).n_D)/|D-S|^3, and the
 //                 emission and attenuation integrals, in the order the bin sum

@@ -171,7 +171,8 @@ __device__ __forceinline__ void conv_chunk(const u16x8 *halo, int v0, int x0, co
 #pragma unroll
         for (int r = 0; r < RB; ++r) {
             to[r] = p[r * STEP * GP];
-            if (4 * s + 3 >= G && 4 * s + q >= G) to[r] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};   // zeros on both sides past the last tap
+            // zeros on both sides past the last tap
+            if (4 * s + 3 >= G && 4 * s + q >= G) to[r] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
         }
     };
 #pragma unroll
@@ -227,7 +228,8 @@ __device__ __forceinline__ u16x8 halo_fetch(const HaloSrc &s, int gx, int gy, in
     const unsigned at = (unsigned)(((gz >> sh) * (s.H >> sh) + (gy >> sh)) * (s.W >> sh) + (gx >> sh)) *
                             (unsigned)s.stride + 16 * g;
     ok = ok && (unsigned)gx < (unsigned)s.W && (unsigned)gy < (unsigned)s.H && gz >= s.zs0 && gz < s.zs1;
-    return __builtin_bit_cast(u16x8, __builtin_amdgcn_raw_buffer_load_b128(s.p, ok ? (int)at : -1, 0, 0));
+    // 2^32 - 16: past any buffer (rows are of 16 bytes and more), and the 16 bytes do not wrap
+    return __builtin_bit_cast(u16x8, __builtin_amdgcn_raw_buffer_load_b128(s.p, ok ? (int)at : -16, 0, 0));
 }
 
 // A layer's epilogue: bias, activation, stores and the head.
@@ -610,7 +612,8 @@ __device__ __forceinline__ void conv_res_chunk(const u16x8 *halo, const u16x8 *w
                 return;
             }
             a[s & 1][k - 1] = p[(k - 1) * RHX * NG];
-            if (K * s + K > 27 && K * s + tq >= 27) a[s & 1][k - 1] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};   // the weights are zero there too
+            // the weights are zero there too
+            if (K * s + K > 27 && K * s + tq >= 27) a[s & 1][k - 1] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
         };
 #pragma unroll
         for (int i = 0; i < 1 + AHEAD; ++i) read(i);

@@ -94,9 +94,10 @@ int srf_project(const float *lors, int64_t n, int64_t lor_stride,
  * accumulate = 0 zeroes `image` first (the op's cudaMemset, siddon.cc:128);
  * 1 adds into it.  `values` may be NULL, meaning all ones (the sensitivity
  * image, emap_generator.py:169-201).  A long list is binned into image tiles for
- * the call (as a plan does; up to about 4 GB of scratch, and `stream` is
- * synchronised); a short one, and any list under graph capture, goes through
- * float atomics. */
+ * the call (up to about 4 GB of scratch, and `stream` is synchronised) and
+ * summed in float64 tile by tile; a short one, and any list under graph capture,
+ * goes through float atomics.  Either keeps every voxel to float32 rounding of
+ * its own sum, far TOF tails included, and passes on NaN and infinite values. */
 int srf_backproject(const float *lors, int64_t n, int64_t lor_stride,
                     const float *tof_values, int64_t tof_stride,
                     const float *values, srf_grid_t grid, const srf_tof_t *tof,
@@ -261,7 +262,10 @@ int srf_plan_project(srf_plan *plan, const float *image, float *out, void *strea
  * osem_full.py:74-75). */
 int srf_plan_project_ratio(srf_plan *plan, const float *image, const float *y, srf_ratio_kind_t kind,
                            float eps, float *q, void *stream);
-/* image (+)= backprojection (srf_backproject semantics; values NULL = ones). */
+/* image (+)= backprojection (srf_backproject semantics; values NULL = ones).
+ * Summed in 64-bit fixed point, so that repeated calls agree bit for bit; terms
+ * below 2^-50 of the largest that a work item's values and weights allow (a TOF
+ * Gaussian beyond 8.3 sigma of its centre) add nothing. */
 int srf_plan_backproject(srf_plan *plan, const float *values, srf_bp_mode_t mode,
                          int accumulate, float *image, void *stream);
 /* srf_plan_project of n_images images (nvox floats each, one after the other) into

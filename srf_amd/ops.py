@@ -145,6 +145,37 @@ def _(lors, y, p, kind, eps, shape, geom, use_tof, tof_bin, tof_sigma2, mode, to
     return lors.new_empty((nz, ny, nx))
 
 
+# ------------------------------------------------------------ point integrals --
+
+@torch.library.custom_op("srf::point_integrals", mutates_args=())
+def point_integrals(det: Tensor, points: Tensor, image_k: Tensor, shape: List[int], geom: List[float]) -> Tensor:
+    """(n_det, n_points) line integrals of an image from every detector (rows of 4) to
+    every point (rows of 3 and more): srf_sss_integrals.  Not differentiable."""
+    _req(det, "det")
+    _req(points, "points")
+    if det.dim() != 2 or det.shape[1] != 4:
+        raise ValueError(f"det must be (N, 4), got {tuple(det.shape)}")
+    if points.dim() != 2 or points.shape[1] < 3:
+        raise ValueError(f"points must be (N, >=3), got {tuple(points.shape)}")
+    _check_image(image_k, shape)
+    if not det.device == points.device == image_k.device:
+        raise ValueError(f"det, points and image are on {det.device}, {points.device} and {image_k.device}")
+    nd, ns = int(det.shape[0]), int(points.shape[0])
+    out = torch.empty((nd, ns), dtype=torch.float32, device=det.device)
+    if nd == 0 or ns == 0:
+        return out
+    with torch.cuda.device(det.device):
+        rc = lib().srf_sss_integrals(det.data_ptr(), nd, points.data_ptr(), ns, int(points.shape[1]), image_k.data_ptr(),
+                                     _grid(shape, geom), out.data_ptr(), stream_handle(det.device))
+    check(rc, "srf_sss_integrals")
+    return out
+
+
+@point_integrals.register_fake
+def _(det, points, image_k, shape, geom):
+    return det.new_empty((det.shape[0], points.shape[0]))
+
+
 # --------------------------------------------------------------- elementwise --
 
 @torch.library.custom_op("srf::ratio", mutates_args=())
@@ -500,5 +531,5 @@ def _(handle, y, p, kind, eps, n, shape, mode):
 # gradients of srf::project / srf::plan_project (adjoint-mode backprojector)
 from . import autograd as _autograd  # noqa: E402,F401
 
-__all__ = ["Plan", "plan_project", "plan_project_batch", "plan_backproject_batch", "plan_backproject", "plan_backproject_ratio", "project", "backproject", "backproject_ratio", "ratio", "em_update", "lor_digest",
+__all__ = ["Plan", "plan_project", "plan_project_batch", "plan_backproject_batch", "plan_backproject", "plan_backproject_ratio", "project", "backproject", "backproject_ratio", "point_integrals", "ratio", "em_update", "lor_digest",
            "to_kernel_layout", "from_kernel_layout", "_lib"]

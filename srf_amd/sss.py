@@ -236,17 +236,10 @@ class SingleScatterSimulation:
         img_k = ops.to_kernel_layout(img_xyz.to(self.dev, torch.float32).contiguous())
         if pts is None and self.plan is not None:
             return (self.plan.project(img_k) * self.to_integral).reshape(self.nd, -1)
-        ops._check_image(img_k, self.shape)
-        xyz = (self.pts_xyz if pts is None else pts).contiguous()
-        ns = int(xyz.shape[0])
-        out = torch.empty((self.nd, ns), dtype=torch.float32, device=self.dev)
-        if ns == 0:
-            return out
-        with torch.cuda.device(self.dev):
-            check(lib().srf_sss_integrals(self.det.data_ptr(), self.nd, xyz.data_ptr(), ns, int(xyz.shape[1]),
-                                          img_k.data_ptr(), ops._grid(self.shape, self.geom), out.data_ptr(),
-                                          stream_handle(self.dev)), "srf_sss_integrals")
-        return out
+        xyz = self.pts_xyz if pts is None else pts
+        if torch.promote_types(xyz.dtype, torch.float32) == torch.float32:
+            xyz = xyz.to(torch.float32)      # integers and half precision; the op refuses the others
+        return ops.point_integrals(self.det, xyz.contiguous(), img_k, self.shape, self.geom)
 
     def points(self, mu_xyz):
         mu = mu_xyz.detach().to(self.dev, torch.float32).reshape(-1)[self.pts_flat]

@@ -351,15 +351,24 @@ int srf_batch_em_step(srf_batch *batch, srf_ratio_kind_t kind, float eps, float 
  *   bins    (n_bins, 2)  detector pairs; out (n_bins)
  *   tables  543 floats: 511/E', window efficiency, KN/sigma_KN per integer
  *           scattering angle 0..180 degrees.
- * Each bin's sum over points is split over wavefronts and, where there are few
- * bins, over workgroups (then through transient scratch, outside graph capture),
- * and combined in a fixed order. */
+ * srf_sss_prepare and srf_sss_sinogram take bins in any order (16 or 64 lanes a bin).
+ * The _ordered forms give the same sums, faster for a large sinogram whose
+ * neighbouring bins lie on neighbouring detectors (one bin a lane; the sum over
+ * points split over workgroups where there are few bins, then through transient
+ * scratch, outside graph capture); rows prepared by one form are read by the same
+ * form only.  Sums are combined in a fixed order. */
 size_t srf_sss_rows_bytes(int32_t n_det, int32_t n_points);
 int srf_sss_prepare(const float *det, int32_t n_det, const float *points, int32_t n_points,
                     const float *em_int, const float *mu_int, void *rows, size_t rows_bytes, void *stream);
 int srf_sss_sinogram(const void *rows, int32_t n_det, const float *points, int32_t n_points,
                      const int32_t *bins, int32_t n_bins, const float *tables, float scale, float *out,
                      void *stream);
+
+int srf_sss_prepare_ordered(const float *det, int32_t n_det, const float *points, int32_t n_points,
+                            const float *em_int, const float *mu_int, void *rows, size_t rows_bytes, void *stream);
+int srf_sss_sinogram_ordered(const void *rows, int32_t n_det, const float *points, int32_t n_points,
+                             const int32_t *bins, int32_t n_bins, const float *tables, float scale, float *out,
+                             void *stream);
 
 /* out[d * n_points + s] = line integral of `image` (kernel layout, per mm) from
  * detector d (rows of 4 floats, as srf_sss_prepare) to point s (rows of

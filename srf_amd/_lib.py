@@ -123,7 +123,9 @@ SIGNATURES = [
     ("srf_sss_rows_bytes", ctypes.c_size_t, [_I32, _I32]),
     ("srf_sss_integrals", ctypes.c_int, [_P, _I32, _P, _I32, _I32, _P, SrfGrid, _P, _P]),
     ("srf_sss_prepare", ctypes.c_int, [_P, _I32, _P, _I32, _P, _P, _P, ctypes.c_size_t, _P]),
+    ("srf_sss_prepare_ordered", ctypes.c_int, [_P, _I32, _P, _I32, _P, _P, _P, ctypes.c_size_t, _P]),
     ("srf_sss_sinogram", ctypes.c_int, [_P, _I32, _P, _I32, _P, _I32, _P, _F, _P, _P]),
+    ("srf_sss_sinogram_ordered", ctypes.c_int, [_P, _I32, _P, _I32, _P, _I32, _P, _F, _P, _P]),
     ("srf_scatter_correct", ctypes.c_int, [_P, _P, _P, _P, _I64, _I64, _F, _P, _P, _P]),
     ("srf_cnn_conv", ctypes.c_int, [_P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _F, _P, _P,
                                     _P]),

@@ -340,13 +340,13 @@ def _main(argv=None):
             t = tick("sss: emission line integrals", t)
             rows = s._rows_for(pts.shape[0])
             st = stream_handle(dev)
-            check(lib().srf_sss_prepare(s.det.data_ptr(), s.nd, pts.data_ptr(), pts.shape[0], em.data_ptr(),
-                                        mu.data_ptr(), rows.data_ptr(), rows.numel() * 4, st), "srf_sss_prepare")
+            prepare, sinogram = s._kernels(pts.shape[0])
+            check(prepare(s.det.data_ptr(), s.nd, pts.data_ptr(), pts.shape[0], em.data_ptr(), mu.data_ptr(),
+                          rows.data_ptr(), rows.numel() * 4, st), "srf_sss_prepare")
             t = tick("sss: srf_sss_prepare (k_sss_pairs)", t)
             out = torch.zeros(s.bins.shape[0], device=dev)
-            check(lib().srf_sss_sinogram(rows.data_ptr(), s.nd, pts.data_ptr(), pts.shape[0], s.bins.data_ptr(),
-                                         s.bins.shape[0], s.tables.data_ptr(), float(s.scale), out.data_ptr(), st),
-                  "srf_sss_sinogram")
+            check(sinogram(rows.data_ptr(), s.nd, pts.data_ptr(), pts.shape[0], s.bins.data_ptr(), s.bins.shape[0],
+                           s.tables.data_ptr(), float(s.scale), out.data_ptr(), st), "srf_sss_sinogram")
             t = tick("sss: srf_sss_sinogram (k_sss_bins)", t)
         torch.cuda.synchronize()
         t = time.time()

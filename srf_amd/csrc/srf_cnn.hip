@@ -765,7 +765,7 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(const unsigned short *__rest
 // the 28th place sums the bias gradient, against ones) or takes every fourth K step
 // (1 tap).  Bound by the LDS reads (2 per SB x tap x K step, 8 cycles of the CU's LDS).
 // A workgroup writes its sums to `part`, which k_wgrad_sum adds up in order; without
-// scratch (part null) it adds them to dW with atomics.
+// scratch (part null: small layers, capture) it adds them to dW with atomics.
 // The 15 layers of the 16-32-64-128 network on four 32 x 64 x 64 samples: 241 us and 123
 // for the sums (1507 with a transposed copy of the tile in LDS, 32 x 32 channel blocks
 // and atomics; 1150 with this kernel and atomics).
@@ -777,7 +777,17 @@ static_assert(2 * (2 * wg_plane(1) + 2 * wg_plane(0)) <= 65536, "static LDS");
 // Workgroups of a launch.  The same layers, kernel and sums: 256 432 us, 512 364 us,
 // 1024 397 us (more parts to add up).
 constexpr int64_t WG_WANTED = 512;
+// One tap (four parts a workgroup): two tiles a workgroup or more, beyond this many workgroups
+// (16 -> 1 channels on 32 x 64 x 64, 512 workgroups or 256: 23, 17 us).
+constexpr int64_t WG_ONE_TAP = 128;
 constexpr size_t WG_SCRATCH = 64u << 20;   // bytes of partial sums at most
+// Small layers add to dW by atomics: up to 64 additions per element, 2^23 in all, or 2^18 in
+// all, cost less than the second launch and its pass over the parts.  us, atomics / parts:
+// 128 -> 128 channels on 8 x 16 x 16 voxels 14 / 32 (the copied tiles of before: 17), 96 -> 32
+// on 16 x 32 x 32 14 / 28, 16 -> 1, one tap, on 16 x 32 x 32 7 / 12; 16 -> 16 on 32 x 64 x 64
+// (512 additions per element) 33 / 22.
+constexpr int WG_ATOMIC_PARTS = 64;
+constexpr int64_t WG_ATOMIC_ADDS = 1 << 23, WG_ATOMIC_FEW = 1 << 18;
 
 struct WgCfg {
     int ntx, nty, ntz;   // tiles of a sample
@@ -1469,8 +1479,10 @@ int srf_cnn_conv_wgrad_batch(const void *x, const void *dy, int32_t dy_stride, i
         WgCfg c;
         c.swap = ny < nx ? 1 : 0;
         const int nf = c.swap ? nx : ny, ns = c.swap ? ny : nx;
-        const int SB = taps == 1 || ns < 2 ? 1 : 2;
-        const int FB = taps == 1 || nf < 2 ? 1 : nf % 3 == 0 && SB == 1 ? 3 : 2;   // (3, 2) would spill
+        // one tap: two blocks of each or one of each (32 -> 64 channels on 64 x 128 x 128 59 us,
+        // one of each 107: both operands are read once per block of the other)
+        const int SB = ns < 2 ? 1 : 2;
+        const int FB = nf < 2 || (taps == 1 && SB == 1) ? 1 : nf % 3 == 0 && SB == 1 ? 3 : 2;   // (3, 2) would spill
         const int gf = (nf + FB - 1) / FB, gs = (ns + SB - 1) / SB;
         c.NF = gf * FB * 16;
         c.NS = gs * SB * 16;
@@ -1484,19 +1496,25 @@ int srf_cnn_conv_wgrad_batch(const void *x, const void *dy, int32_t dy_stride, i
         const size_t per = (size_t)(taps + 1) * c.NF * c.NS * sizeof(float) * (taps == 1 ? 4 : 1);
         // WG_WANTED workgroups, and at most WG_SCRATCH of partial sums
         int64_t parts = WG_WANTED / ((int64_t)gf * gs);
+        const int64_t one = c.ntiles / 2 > WG_ONE_TAP ? c.ntiles / 2 : WG_ONE_TAP;
+        if (taps == 1 && parts > one) parts = one;
         parts = parts < (int64_t)(WG_SCRATCH / per) ? parts : (int64_t)(WG_SCRATCH / per);
         parts = parts < 1 ? 1 : parts;
         c.run = (int)((c.ntiles + parts - 1) / parts);
         dim3 grid((unsigned)((c.ntiles + c.run - 1) / c.run), (unsigned)gf, (unsigned)gs);
         const int nparts = (int)grid.x * (taps == 1 ? 4 : 1);
-        // no scratch under capture, nor where every element has one writer
+        // no scratch under capture, where every element has one writer, nor for few additions
+        // (WG_ATOMIC_*)
+        const int64_t adds = (int64_t)(per / sizeof(float)) * grid.x;
+        const bool few = (nparts <= WG_ATOMIC_PARTS && adds <= WG_ATOMIC_ADDS) || adds <= WG_ATOMIC_FEW;
         float *part = nullptr;
-        if (!capturing(st) && nparts > 1 && per * grid.x <= WG_SCRATCH)
+        if (!few && !capturing(st) && nparts > 1 && per * grid.x <= WG_SCRATCH)
             part = static_cast<float *>(pool_get(per * grid.x, st));
         auto *S = (const unsigned short *)(c.swap ? dy : x), *F = (const unsigned short *)(c.swap ? x : dy);
 #define SRF_WGRAD(TP, FBK, SBK) \
     hipLaunchKernelGGL((k_conv_wgrad_tr<TP, FBK, SBK>), grid, dim3(256), 0, st, S, F, d, c, part, dw, db)
-        if (taps == 1) SRF_WGRAD(1, 1, 1);
+        if (taps == 1 && SB == 2) SRF_WGRAD(1, 2, 2);
+        else if (taps == 1) SRF_WGRAD(1, 1, 1);
         else if (SB == 2) SRF_WGRAD(27, 2, 2);
         else if (FB == 3) SRF_WGRAD(27, 3, 1);
         else if (FB == 2) SRF_WGRAD(27, 2, 1);

@@ -517,13 +517,15 @@ static int check_events(const float *lors, int64_t n, int64_t stride, const floa
 static inline unsigned blocks_for(int64_t n) { return (unsigned)((n + 255) / 256); }
 
 // Lists of at least BUNDLE_SLABS slabs (events times the longer transaxial side of
-// the image; twice that where the image fits an XCD's 4 MiB L2) are bundled,
+// the image; three times that where the image fits an XCD's 4 MiB L2) are bundled,
 // BUNDLE_CHUNK events at a time (the scratch of a chunk is about 20 bytes per event
 // plus the two copies).  Images that fit L2 several times over never are.  Measured,
 // us, bundled / one event per lane:
 //   256 x 256 x 128   65536 events 148 / 126, 98304 188 / 230, 2^18 317 / 548, 2^20 780 / 2838
 //   181 x 217 x 91    65536 109 / 97, 98304 141 / 167, 2^18 245 / 346, 2^20 630 / 1567
-//   128 x 128 x 64    2^17 110 / 90, 2^18 183 / 174, 2^19 272 / 340, 2^20 442 / 672
+//   128 x 128 x 64    2^17 110 / 90, 2^18 183 / 174, 2^19 272 / 340, 2^20 442 / 672;
+//                     random pairs of ends, many of which miss the image: 4e5 235 / 144,
+//                     9e5 328 / 246, 1.4e6 345 / 367
 //   48 x 48 x 24      2^20 275 / 189
 // 5e6 TOF events on 256 x 256 x 128: 2.49 ms against 21.3 ms (each term a line of its
 // own from beyond L2).  Now VALU bound: about 75 instructions per slab.
@@ -557,7 +559,7 @@ static bool project_bundled(const float *lors, int64_t n, int stride, const floa
                             hipStream_t s, int &rc)
 {
     const int64_t bytes = (int64_t)G.nx * G.ny * G.nz * 4, slabs = n * (G.nx > G.ny ? G.nx : G.ny);
-    if (bytes < BUNDLE_IMAGE_MIN || slabs < (bytes > BUNDLE_IMAGE_L2 + (BUNDLE_IMAGE_L2 >> 2) ? 1 : 2) * BUNDLE_SLABS) return false;
+    if (bytes < BUNDLE_IMAGE_MIN || slabs < (bytes > BUNDLE_IMAGE_L2 + (BUNDLE_IMAGE_L2 >> 2) ? 1 : 3) * BUNDLE_SLABS) return false;
     if (!border_fits(G) || capturing(s)) return false;
     const int64_t chunk = n < BUNDLE_CHUNK ? n : BUNDLE_CHUNK;
     size_t sort_bytes = 0;

@@ -42,7 +42,8 @@ struct VoxelIndex {
 // float32 rounds the same way over whole binades (4 times the error at 200 slabs).
 constexpr int SUM_RUN = 16;
 
-// The three loads of a slab are issued together: terms that do not apply read
+// The weight goes into every slab's sum, so that an image of values near float32's largest
+// overflows only where its projection does.  The three loads of a slab are issued together: terms that do not apply read
 // voxel 0 and are replaced by zero.
 struct GatherAct {
     const float *__restrict__ img;
@@ -64,13 +65,13 @@ struct GatherAct {
         g1 = t.v1 ? g1 : 0.0f;
         g2 = t.v2 ? g2 : 0.0f;
         g3 = t.v3 ? g3 : 0.0f;
-        part = fmaf(fmaf(g1, c.r1, fmaf(g2, c.r2, g3 * c.r3)), e, part);
+        part = fmaf(fmaf(g1, c.r1, fmaf(g2, c.r2, g3 * c.r3)), e * W, part);
         if ((ip & (SUM_RUN - 1)) == SUM_RUN - 1) {
             sum += part;
             part = 0.0f;
         }
     }
-    __device__ __forceinline__ void nan_event() { sum = __builtin_nanf(""); W = 1.0f; }
+    __device__ __forceinline__ void nan_event() { sum = __builtin_nanf(""); }
     const LaunchGeom *G;
 };
 
@@ -144,7 +145,7 @@ __global__ __launch_bounds__(256) void k_gather(const float *__restrict__ lors, 
     act.sum = act.part = act.W = 0.0f;
     act.G = &G;
     if (on) march_event<TOF, VAR, DS, DZ>(lors + e * stride, TOF ? tofv[e * tof_stride] : 0.0f, G, part, parts, act);
-    float s = (act.sum + act.part) * act.W;
+    float s = act.sum + act.part;
     for (int k = parts >> 1; k > 0; k >>= 1) s += __shfl_xor(s, k);
     if (on && part == 0) out[e] = s;
 }
@@ -240,11 +241,11 @@ __device__ __forceinline__ int wave_max(int v)
     return __builtin_amdgcn_readfirstlane(v);
 }
 
-// Sum over the slabs [a, b) of every lane's ray (a >= b: none), the wavefront in
+// Weighted sum over the slabs [a, b) of every lane's ray (a >= b: none), the wavefront in
 // step through the planes of a bordered copy of pl floats per plane; of `parts`
 // wavefronts with the same rays, number `part` takes its share of the planes.
 template <bool TOF, bool DS, bool DZ>
-__device__ __forceinline__ float bundle_sum(const Branch &B, float z1, const LaunchGeom &G, int a, int b, float tA,
+__device__ __forceinline__ float bundle_sum(const Branch &B, float W, float z1, const LaunchGeom &G, int a, int b, float tA,
                                             float tB, const float *__restrict__ copy, int64_t pl, int pz, int part, int parts)
 {
     const bool on = a < b;
@@ -294,7 +295,7 @@ __device__ __forceinline__ float bundle_sum(const Branch &B, float z1, const Lau
                 e = __builtin_amdgcn_exp2f(-(dd * dd));
             }
             const float s = fmaf(g1, c.r1, fmaf(g2, c.r2, g3 * c.r3));
-            acc = TOF ? fmaf(s, e, acc) : acc + s;
+            acc = fmaf(s, TOF ? e * W : W, acc);
         }
         if ((ip & (SUM_RUN - 1)) == SUM_RUN - 1) {   // a scalar test: the wavefront is in step
             sum += acc;
@@ -347,10 +348,10 @@ __global__ __launch_bounds__(256) void k_bundle(const float *__restrict__ lors, 
     float s = 0.0f;
     // a wavefront holds one branch, but for the one where the sorted list changes over
     if (__any(a < b && B.xdom))
-        s = bundle_sum<TOF, DS, DZ>(B, r.z1, G, a, B.xdom ? b : a, tA, tB, zx, (int64_t)(G.ny + 2) * pz, pz,
+        s = bundle_sum<TOF, DS, DZ>(B, W, r.z1, G, a, B.xdom ? b : a, tA, tB, zx, (int64_t)(G.ny + 2) * pz, pz,
                                     part, parts);
     if (__any(a < b && !B.xdom)) {
-        const float t = bundle_sum<TOF, DS, DZ>(B, r.z1, G, a, B.xdom ? a : b, tA, tB, zy, (int64_t)(G.nx + 2) * pz, pz,
+        const float t = bundle_sum<TOF, DS, DZ>(B, W, r.z1, G, a, B.xdom ? a : b, tA, tB, zy, (int64_t)(G.nx + 2) * pz, pz,
                                                   part, parts);
         s = B.xdom ? s : t;
     }
@@ -360,7 +361,7 @@ __global__ __launch_bounds__(256) void k_bundle(const float *__restrict__ lors, 
         if (part != 0) return;
         for (int k = 1; k < parts; ++k) s += part_sum[threadIdx.x + 64 * k];
     }
-    if (in) out[e] = r.nan ? __builtin_nanf("") : (a < b ? s * W : 0.0f);
+    if (in) out[e] = r.nan ? __builtin_nanf("") : (a < b ? s : 0.0f);
 }
 
 // values == nullptr: all ones.  y/p != nullptr: value = ratio(y, p).
@@ -429,13 +430,14 @@ __global__ __launch_bounds__(256) void k_point_integrals(const float *__restrict
     int a, b;
     event_slabs<false, V_FP>(r, G, B, a, b);
     if (!in || r.nan) a = b = 0;
+    const float W = B.sq * G.dx_;
     float sum = 0.0f;
     if (BORDER) {
         const int pz = G.nz + 2;
         if (__any(a < b && B.xdom))
-            sum = bundle_sum<false, DS, DZ>(B, r.z1, G, a, B.xdom ? b : a, 0.0f, 0.0f, zx, (int64_t)(G.ny + 2) * pz, pz, 0, 1);
+            sum = bundle_sum<false, DS, DZ>(B, W, r.z1, G, a, B.xdom ? b : a, 0.0f, 0.0f, zx, (int64_t)(G.ny + 2) * pz, pz, 0, 1);
         if (__any(a < b && !B.xdom)) {
-            const float t = bundle_sum<false, DS, DZ>(B, r.z1, G, a, B.xdom ? a : b, 0.0f, 0.0f, zy,
+            const float t = bundle_sum<false, DS, DZ>(B, W, r.z1, G, a, B.xdom ? a : b, 0.0f, 0.0f, zy,
                                                       (int64_t)(G.nx + 2) * pz, pz, 0, 1);
             sum = B.xdom ? sum : t;
         }
@@ -444,11 +446,11 @@ __global__ __launch_bounds__(256) void k_point_integrals(const float *__restrict
         act.img = img;
         act.sum = act.part = 0.0f;
         act.G = &G;
-        act.begin(B, 1.0f);
+        act.begin(B, W);
         march_slabs<false, DS, DZ>(B, r.z1, G, a, b, 0.0f, 0.0f, act);
         sum = act.sum + act.part;
     }
-    if (in) out[(int64_t)d * ns + s] = r.nan ? __builtin_nanf("") : (a < b ? sum * (B.sq * G.dx_) : 0.0f);
+    if (in) out[(int64_t)d * ns + s] = r.nan ? __builtin_nanf("") : (a < b ? sum : 0.0f);
 }
 
 // ----------------------------------------------------------------- host side --

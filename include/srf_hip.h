@@ -185,9 +185,11 @@ int srf_image_from_kernel_layout(const float *src_kernel, float *dst_xyz, int32_
  * bin into at most 2^31 - 1 segments, and a plan's grid may have at most 32767
  * cells along x and along y (SRF_ERR_UNSUPPORTED beyond: split the list into
  * several plans, as OSEM subsets are).  The memory comes from a pool per
- * device that keeps up to 16 GiB of freed plan memory for the next plans, in
- * order between streams by events (srf_plan_pool_trim releases it);
- * srf_plan_destroy first waits for the device, as hipFree does. */
+ * device that keeps up to 16 GiB of freed memory for the next plans, of it up to
+ * 6 GiB that was scratch of other calls (srf_project, srf_backproject and the
+ * others named at the top take theirs from it), in order between streams by
+ * events (srf_plan_pool_trim releases it); srf_plan_destroy first waits for the
+ * device, as hipFree does. */
 typedef struct srf_plan srf_plan;
 
 int srf_plan_create(const float *lors, int64_t n, int64_t lor_stride,
@@ -229,9 +231,9 @@ int srf_plan_rebuild(srf_plan *plan, const float *lors, int64_t n, int64_t lor_s
                      const float *tof_values, int64_t tof_stride, srf_grid_t grid, const srf_tof_t *tof,
                      const srf_plan_opts_t *opts, void *stream);
 int srf_plan_destroy(srf_plan *plan);
-/* Returns the current device's pooled plan memory above keep_bytes to the
- * system (hipFree after draining the device), so that other HIP users
- * of the process (torch's caching allocator) can have it; 0 releases all
+/* Returns the current device's pooled memory (of plans and of the scratch of
+ * other calls) above keep_bytes to the system (hipFree after draining the
+ * device), so that other HIP users of the process (torch's caching allocator) can have it; 0 releases all
  * memory no live plan holds.  No reference counterpart (the plan pool is this
  * library's). */
 int srf_plan_pool_trim(size_t keep_bytes);

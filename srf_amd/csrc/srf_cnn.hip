@@ -1528,7 +1528,7 @@ int srf_cnn_conv_wgrad_batch(const void *x, const void *dy, int32_t dy_stride, i
                                    c, dw, db);
                 rc = launch_status();
             }
-            pool_put(part, st);
+            pool_put(part, st, false, true);
         }
         return rc;
     }

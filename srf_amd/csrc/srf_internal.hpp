@@ -22,9 +22,10 @@ int fill_f32(float *dst, float v, int64_t n, hipStream_t s);
 // Device memory for plans and scratch (srf_pool.hip).  pool_get: at least `bytes`
 // on the current device, for use in stream order on s (nullptr: none left).
 // pool_put: given back once the work queued on s so far is done (idle: nothing
-// uses it any more).  Not for a stream that is being captured.
+// uses it any more; scratch: not a plan's, of which the pool keeps less).  Not for
+// a stream that is being captured.  Neither throws.
 void *pool_get(size_t bytes, hipStream_t s);
-void pool_put(void *p, hipStream_t s, bool idle = false);
+void pool_put(void *p, hipStream_t s, bool idle = false, bool scratch = false);
 
 // True on a stream that is being captured (no scratch can be taken for it then),
 // or whose state cannot be told.

@@ -2,7 +2,8 @@
 // pool_get / pool_put), and srf_plan_pool_trim.
 //
 // Blocks are hipMalloc'd in rounded sizes and kept when they are given back: at
-// most POOL_KEEP bytes per device, the oldest ones going to the system first.
+// most POOL_KEEP bytes per device, and SCRATCH_KEEP of them from the scratch of calls
+// that keep no plan, the oldest ones going to the system first.
 // A block given back on a stream carries an event recorded there; whoever takes
 // it next, on any stream or host thread, first lets its stream wait for that
 // event.  The stream-ordered pool of the HIP runtime served this before: it
@@ -21,6 +22,7 @@
 namespace {
 
 constexpr uint64_t POOL_KEEP = 16ull << 30;
+constexpr uint64_t SCRATCH_KEEP = 6ull << 30;   // one long backprojection takes up to about 4 GB
 constexpr int POOL_DEVICES = 64;
 
 struct Block {
@@ -29,6 +31,7 @@ struct Block {
     int dev;
     hipEvent_t ev;     // recorded when the block was given back
     bool wait;         // the next user waits for ev
+    bool scratch;      // given back by a call that keeps no plan
 };
 
 std::mutex mu;
@@ -42,7 +45,7 @@ std::list<Block> &kept(int dev)             // blocks given back, oldest first
     static auto *l = new std::list<Block>[POOL_DEVICES];
     return l[dev];
 }
-uint64_t kept_bytes[POOL_DEVICES];
+uint64_t kept_bytes[POOL_DEVICES], kept_scratch[POOL_DEVICES];
 
 int current_device()
 {
@@ -70,16 +73,39 @@ void release(Block &b)
     if (b.ev) (void)hipEventDestroy(b.ev);
 }
 
-// Releases kept blocks of the device, oldest first, down to keep bytes.
-void trim_locked(int dev, uint64_t keep)
+// Takes a kept block out of its list.
+Block take(std::list<Block>::iterator it, int dev)
+{
+    const Block b = *it;
+    kept(dev).erase(it);
+    kept_bytes[dev] -= b.bytes;
+    if (b.scratch) kept_scratch[dev] -= b.bytes;
+    return b;
+}
+
+// Releases kept blocks of the device, oldest first, down to keep bytes and scratch bytes.
+void trim_locked(int dev, uint64_t keep, uint64_t scratch)
 {
     auto &l = kept(dev);
-    while (kept_bytes[dev] > keep && !l.empty()) {
-        Block b = l.front();
-        l.pop_front();
-        kept_bytes[dev] -= b.bytes;
+    for (auto it = l.begin(); it != l.end() && (kept_bytes[dev] > keep || kept_scratch[dev] > scratch);) {
+        const auto here = it++;
+        if (kept_bytes[dev] <= keep && !here->scratch) continue;
+        Block b = take(here, dev);
         release(b);
     }
+}
+
+// A new block of `want` bytes, or of `least` where the card has no more.
+void *allocate(size_t want, size_t least, int dev, size_t &got)
+{
+    void *p = nullptr;
+    for (int tries = 0; tries < 3; ++tries) {
+        got = tries < 2 ? want : least;
+        if (hipMalloc(&p, got) == hipSuccess) return p;
+        (void)hipGetLastError();
+        if (tries == 0) trim_locked(dev, 0, 0);
+    }
+    return nullptr;
 }
 
 }  // namespace
@@ -92,37 +118,33 @@ void *pool_get(size_t bytes, hipStream_t s)
     if (dev < 0) return nullptr;
     const size_t want = rounded(bytes ? bytes : 1);
     std::lock_guard<std::mutex> lock(mu);
-    auto &l = kept(dev);
-    // the smallest kept block that fits without wasting more than a quarter;
-    // among equals the one given back last
-    auto best = l.end();
-    for (auto it = l.begin(); it != l.end(); ++it)
-        if (it->bytes >= want && it->bytes - want <= want / 4 && (best == l.end() || it->bytes <= best->bytes)) best = it;
-    Block b{nullptr, 0, dev, nullptr, false};
-    if (best != l.end()) {
-        b = *best;
-        if (b.wait && hipStreamWaitEvent(s, b.ev, 0) != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
-        l.erase(best);
-        kept_bytes[dev] -= b.bytes;
-    } else {
-        if (hipMalloc(&b.p, want) != hipSuccess) {
-            (void)hipGetLastError();
-            trim_locked(dev, 0);
-            if (hipMalloc(&b.p, want) != hipSuccess) {
+    Block b{nullptr, 0, dev, nullptr, false, false};
+    try {
+        auto &l = kept(dev);
+        // the smallest kept block that fits without wasting more than a quarter;
+        // among equals the one given back last
+        auto best = l.end();
+        for (auto it = l.begin(); it != l.end(); ++it)
+            if (it->bytes >= want && it->bytes - want <= want / 4 && (best == l.end() || it->bytes <= best->bytes)) best = it;
+        if (best != l.end()) {
+            if (best->wait && hipStreamWaitEvent(s, best->ev, 0) != hipSuccess) {
                 (void)hipGetLastError();
                 return nullptr;
             }
+            b = take(best, dev);
+        } else {
+            b.p = allocate(want, bytes ? bytes : 1, dev, b.bytes);
+            if (!b.p) return nullptr;
         }
-        b.bytes = want;
+        live()[b.p] = b;
+        return b.p;
+    } catch (...) {   // no host memory for the pool's own lists
+        if (b.p) release(b);
+        return nullptr;
     }
-    live()[b.p] = b;
-    return b.p;
 }
 
-void pool_put(void *p, hipStream_t s, bool idle)
+void pool_put(void *p, hipStream_t s, bool idle, bool scratch)
 {
     if (!p) return;
     std::lock_guard<std::mutex> lock(mu);
@@ -131,6 +153,7 @@ void pool_put(void *p, hipStream_t s, bool idle)
     Block b = it->second;
     live().erase(it);
     b.wait = false;
+    b.scratch = scratch;
     if (!idle) {
         if ((b.ev || hipEventCreateWithFlags(&b.ev, hipEventDisableTiming) == hipSuccess) &&
             hipEventRecord(b.ev, s) == hipSuccess) {
@@ -141,9 +164,15 @@ void pool_put(void *p, hipStream_t s, bool idle)
             return;
         }
     }
-    kept(b.dev).push_back(b);
+    try {
+        kept(b.dev).push_back(b);
+    } catch (...) {
+        release(b);
+        return;
+    }
     kept_bytes[b.dev] += b.bytes;
-    trim_locked(b.dev, POOL_KEEP);
+    if (scratch) kept_scratch[b.dev] += b.bytes;
+    trim_locked(b.dev, POOL_KEEP, SCRATCH_KEEP);
 }
 
 }  // namespace srf
@@ -157,6 +186,6 @@ extern "C" int srf_plan_pool_trim(size_t keep_bytes)
         return SRF_ERR_LAUNCH;
     }
     std::lock_guard<std::mutex> lock(mu);
-    trim_locked(dev, keep_bytes);
+    trim_locked(dev, keep_bytes, keep_bytes);
     return SRF_OK;
 }

@@ -614,7 +614,7 @@ static bool project_bundled(const float *lors, int64_t n, int stride, const floa
 #undef SRF_BUNDLE
         rc = launch_status();
     }
-    pool_put(w, s);
+    pool_put(w, s, false, true);
     return true;
 }
 
@@ -674,7 +674,7 @@ int srf_sss_integrals(const float *det, int32_t n_det, const float *points, int3
         if (zx) {
             zy = zx + nx;
             if ((rc = border_image(image, G, zx, zy, s))) {
-                pool_put(zx, s);
+                pool_put(zx, s, false, true);
                 return rc;
             }
         }
@@ -691,7 +691,7 @@ int srf_sss_integrals(const float *det, int32_t n_det, const float *points, int3
     }
 #undef SRF_POINTS
     rc = launch_status();
-    pool_put(zx, s);
+    pool_put(zx, s, false, true);
     return rc;
 }
 

@@ -424,7 +424,7 @@ static int sum_bins(const void *rows, int32_t n_det, const float *points, int32_
                                scale, out);
             rc = launch_status();
         }
-        pool_put(part, s);
+        pool_put(part, s, false, true);
     }
     return rc;
 }

@@ -34,6 +34,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <new>
 #include <vector>
 
 #include "marcher.hpp"
@@ -1535,11 +1536,11 @@ int dmalloc(T **p, size_t count, size_t &total)
 }
 
 // Given back to the pool (srf_pool.hip): `idle` once nothing uses the buffer any
-// more, else in stream order on s.
+// more, else in stream order on s; `scratch`: of a call that keeps no plan.
 template <class T>
-void dfree(DevBuf<T> &b, hipStream_t s, bool idle = false)
+void dfree(DevBuf<T> &b, hipStream_t s, bool idle = false, bool scratch = false)
 {
-    pool_put(b.p, s, idle);
+    pool_put(b.p, s, idle, scratch);
     b.p = nullptr;
     b.cap = 0;
 }
@@ -1566,31 +1567,29 @@ int ensure(DevBuf<T> &b, size_t count, hipStream_t s)
     return SRF_OK;
 }
 
-// (after the stream has been synchronised)
-void free_scratch(srf_plan *P)
+void free_scratch(srf_plan *P, hipStream_t s, bool idle, bool scratch)
 {
-    const hipStream_t s = nullptr;
-    dfree(P->ev_cnt, s, true);
-    dfree(P->key_count, s, true);
-    dfree(P->scan_tmp, s, true);
-    dfree(P->sort_tmp, s, true);
-    dfree(P->sk, s, true);
-    dfree(P->sk2, s, true);
-    dfree(P->sg, s, true);
-    dfree(P->sg2, s, true);
-    dfree(P->wpair, s, true);
-    dfree(P->ev_cut, s, true);
+    dfree(P->ev_cnt, s, idle, scratch);
+    dfree(P->key_count, s, idle, scratch);
+    dfree(P->scan_tmp, s, idle, scratch);
+    dfree(P->sort_tmp, s, idle, scratch);
+    dfree(P->sk, s, idle, scratch);
+    dfree(P->sk2, s, idle, scratch);
+    dfree(P->sg, s, idle, scratch);
+    dfree(P->sg2, s, idle, scratch);
+    dfree(P->wpair, s, idle, scratch);
+    dfree(P->ev_cut, s, idle, scratch);
 }
 
-void plan_release(srf_plan *P, hipStream_t s, bool idle)
+void plan_release(srf_plan *P, hipStream_t s, bool idle, bool scratch)
 {
-    dfree(P->recs, s, idle);
-    dfree(P->rec_ev, s, idle);
-    dfree(P->tables, s, idle);
-    dfree(P->ev_off, s, idle);
-    dfree(P->ev_flag, s, idle);
-    dfree(P->partial, s, idle);
-    dfree(P->tile_buf, s, idle);
+    dfree(P->recs, s, idle, scratch);
+    dfree(P->rec_ev, s, idle, scratch);
+    dfree(P->tables, s, idle, scratch);
+    dfree(P->ev_off, s, idle, scratch);
+    dfree(P->ev_flag, s, idle, scratch);
+    dfree(P->partial, s, idle, scratch);
+    dfree(P->tile_buf, s, idle, scratch);
 }
 
 // Destroy: the plan may have been used on any stream, so the device is
@@ -1599,8 +1598,8 @@ void plan_free(srf_plan *P)
 {
     if (!P) return;
     (void)hipDeviceSynchronize();
-    plan_release(P, nullptr, true);
-    free_scratch(P);
+    plan_release(P, nullptr, true, false);
+    free_scratch(P, nullptr, true, false);
     delete P;
 }
 
@@ -1845,6 +1844,26 @@ int plan_build(srf_plan *P, const float *lors, int64_t n, int64_t lor_stride, co
     return SRF_OK;
 }
 
+// plan_build without an exception for its host tables' memory, and whether the stream was
+// left without work that uses P's buffers.
+int try_plan_build(srf_plan *P, const float *lors, int64_t n, int64_t lor_stride, const float *tof_values,
+                   int64_t tof_stride, srf_grid_t grid, const srf_tof_t *tof, const srf_plan_opts_t *opts,
+                   hipStream_t s, bool &idle)
+{
+    int rc;
+    try {
+        rc = plan_build(P, lors, n, lor_stride, tof_values, tof_stride, grid, tof, opts, s);
+    } catch (...) {
+        rc = SRF_ERR_LAUNCH;
+    }
+    idle = true;
+    if (rc) {
+        idle = hipStreamSynchronize(s) == hipSuccess;
+        (void)hipGetLastError();
+    }
+    return rc;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1861,15 +1880,16 @@ int srf_plan_create_ex(const float *lors, int64_t n, int64_t lor_stride, const f
 {
     if (!out) return SRF_ERR_INVALID_ARG;
     *out = nullptr;
-    srf_plan *P = new srf_plan();
-    const int rc = plan_build(P, lors, n, lor_stride, tof_values, tof_stride, grid, tof, opts, (hipStream_t)stream);
+    srf_plan *P = new (std::nothrow) srf_plan();
+    if (!P) return SRF_ERR_LAUNCH;
+    bool idle;
+    const int rc = try_plan_build(P, lors, n, lor_stride, tof_values, tof_stride, grid, tof, opts, (hipStream_t)stream,
+                                  idle);
     if (rc) {
-        (void)hipStreamSynchronize((hipStream_t)stream);
-        (void)hipGetLastError();
         plan_free(P);
         return rc;
     }
-    free_scratch(P);
+    free_scratch(P, nullptr, true, false);   // plan_build has synchronised the stream
     *out = P;
     return SRF_OK;
 }
@@ -1879,11 +1899,10 @@ int srf_plan_rebuild(srf_plan *plan, const float *lors, int64_t n, int64_t lor_s
                      void *stream)
 {
     if (!plan) return SRF_ERR_INVALID_ARG;
-    const int rc = plan_build(plan, lors, n, lor_stride, tof_values, tof_stride, grid, tof, opts,
-                              (hipStream_t)stream);
+    bool idle;
+    const int rc = try_plan_build(plan, lors, n, lor_stride, tof_values, tof_stride, grid, tof, opts,
+                                  (hipStream_t)stream, idle);
     if (rc) {
-        (void)hipStreamSynchronize((hipStream_t)stream);
-        (void)hipGetLastError();
         // plan_build committed nothing: the plan keeps its previous grid and
         // holds an empty list (projections write nothing, backprojections
         // zeros); it cannot join a batch until a rebuild succeeds
@@ -1915,10 +1934,10 @@ int srf_event_order(const float *lors, int64_t n_lors, int64_t lor_stride, const
     DevBuf<unsigned char> tmp;
     DevBuf<int> bad;
     auto cleanup = [&]() {
-        dfree(key, s);
-        dfree(key2, s);
-        dfree(tmp, s);
-        dfree(bad, s);
+        dfree(key, s, false, true);
+        dfree(key2, s, false, true);
+        dfree(tmp, s, false, true);
+        dfree(bad, s, false, true);
     };
     SRF_TRY(ensure(key, (size_t)n, s));
     SRF_TRY(ensure(key2, (size_t)n, s));
@@ -2059,11 +2078,12 @@ int backproject_binned(const float *lors, int64_t n, int64_t lor_stride, const f
                        const srf_tof_t *tof, srf_bp_mode_t mode, int accumulate, float *image, hipStream_t s)
 {
     srf_plan P = {};
-    int rc = plan_build(&P, lors, n, lor_stride, tof_values, tof_stride, grid, tof, nullptr, s);
+    bool idle;
+    int rc = try_plan_build(&P, lors, n, lor_stride, tof_values, tof_stride, grid, tof, nullptr, s, idle);
     if (rc == SRF_OK) rc = plan_bp(&P, values, y, p, kind, eps, mode, accumulate, image, s, true);
-    else (void)hipStreamSynchronize(s);   // what was queued of a build that failed
-    free_scratch(&P);
-    plan_release(&P, s, false);
+    // (a build that succeeded has synchronised the stream: its scratch is idle)
+    free_scratch(&P, s, idle, true);
+    plan_release(&P, s, idle && !P.valid, true);
     return rc;
 }
 
@@ -2126,7 +2146,7 @@ int srf_plan_project_batch(srf_plan *P, const float *images, int32_t n_images, f
         rc = launch_status();
         b += 2;
     }
-    pool_put(more, s);
+    pool_put(more, s, false, true);
     return rc;
 }
 

@@ -44,9 +44,10 @@ struct LaunchGeom;
 int make_geom(const srf_grid_t &g, const srf_tof_t *tof, LaunchGeom &G);
 
 // Backprojection of one list through a plan of its own (srf_tiled.hip); anything but
-// SRF_OK: nothing was added to the image.  Synchronises s.
+// SRF_OK: nothing was added to the image.  SRF_ERR_WORKSPACE: the list has more segments
+// than a call may take scratch for, `fit` of its events would do.  Synchronises s.
 int backproject_binned(const float *lors, int64_t n, int64_t lor_stride, const float *tof_values, int64_t tof_stride,
                        const float *values, const float *y, const float *p, int kind, float eps, srf_grid_t grid,
-                       const srf_tof_t *tof, srf_bp_mode_t mode, int accumulate, float *image, hipStream_t s);
+                       const srf_tof_t *tof, srf_bp_mode_t mode, int accumulate, float *image, hipStream_t s, int64_t &fit);
 
 }  // namespace srf

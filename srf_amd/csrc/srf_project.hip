@@ -720,8 +720,9 @@ static int scatter_events(const float *lors, int64_t n, int64_t lor_stride, cons
 //   181 x 217 x 91    16384 417 / 281, 32768 442 / 525, 2^20 1980 / 15200
 //   128 x 128 x 64    16384 238 / 197, 32768 295 / 358, 2^20 1300 / 10100
 //   48 x 48 x 24      65536 368 / 301, 2^17 421 / 541, 2^20 742 / 3730
-// A part of BINNED_CHUNK events takes about 3.5 GB of scratch (4 times as many: 3%
-// faster at 5e6 events).
+// A part of BINNED_CHUNK events takes about 3.5 GB of scratch on 256 x 256 x 128 (4 times as
+// many: 3% faster at 5e6 events); grids whose events have more segments take smaller parts
+// (ONCE_SEGMENTS, srf_tiled.hip), at most about 4 GB.
 constexpr int64_t BINNED_SLABS = 3500000;
 constexpr int64_t BINNED_TILE_SLABS = 6000;
 constexpr int64_t BINNED_CHUNK = 1 << 21;
@@ -747,16 +748,23 @@ static int backproject_impl(const float *lors, int64_t n, int64_t lor_stride, co
     // a long list is binned into image tiles, in parts of equal size; a part that
     // cannot be (no memory, a grid beyond the plans') is scattered
     if (binned_pays(n, G) && !capturing(s)) {
-        const int64_t parts = (n + BINNED_CHUNK - 1) / BINNED_CHUNK, chunk = (n + parts - 1) / parts;
-        for (int64_t c = 0; c < n; c += chunk) {
+        const int64_t parts = (n + BINNED_CHUNK - 1) / BINNED_CHUNK;
+        int64_t chunk = (n + parts - 1) / parts;
+        for (int64_t c = 0; c < n;) {
             const int64_t m = n - c < chunk ? n - c : chunk;
             const float *L = lors + c * lor_stride, *T = tof ? tof_values + c * tof_stride : nullptr;
             const float *V = values ? values + c : nullptr, *Y = y ? y + c : nullptr, *Q = p ? p + c : nullptr;
+            int64_t fit = m;
             rc = backproject_binned(L, m, lor_stride, T, tof_stride, V, Y, Q, kind, eps, grid, tof, mode,
-                                    accumulate || c > 0, image, s);
+                                    accumulate || c > 0, image, s, fit);
+            if (rc == SRF_ERR_WORKSPACE && fit < m) {   // too many segments for the scratch of a part
+                chunk = fit;
+                continue;
+            }
             if (rc) rc = scatter_events(L, m, lor_stride, T, tof_stride, V, Y, Q, kind, eps, G, tof != nullptr, mode,
                                         accumulate || c > 0 ? 0 : nvox, image, s);
             if (rc) return rc;
+            c += m;
         }
         return SRF_OK;
     }

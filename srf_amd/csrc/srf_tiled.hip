@@ -1657,9 +1657,14 @@ static bool pow2_edge(float v)
     return v != 1.0f && v >= 0x1p-64f && v <= 0x1p64f && frexpf(v, &e) == 0.5f;
 }
 
+// fit: null for a plan.  For a list that is backprojected once (no partial sums): lists of
+// more than ONCE_SEGMENTS segments return SRF_ERR_WORKSPACE before any memory is taken for
+// them, with the number of events that would do in *fit.
+constexpr int64_t ONCE_SEGMENTS = 40000000;   // about 100 bytes each: 4 GB
+
 int plan_build(srf_plan *P, const float *lors, int64_t n, int64_t lor_stride, const float *tof_values,
                int64_t tof_stride, srf_grid_t grid, const srf_tof_t *tof, const srf_plan_opts_t *opts,
-               hipStream_t s)
+               hipStream_t s, int64_t *fit)
 {
     const int32_t item_records = (opts && opts->item_records) ? opts->item_records : ITEM;
     const float twin = opts ? opts->tof_window : 0.0f;
@@ -1723,11 +1728,16 @@ int plan_build(srf_plan *P, const float *lors, int64_t n, int64_t lor_stride, co
     // 32-bit prefix sum above would have wrapped) is refused
     uint64_t kc_sum = 0;
     for (unsigned c : kc) kc_sum += c;
-    if (kc_sum > (uint64_t)INT_MAX) return SRF_ERR_UNSUPPORTED;
+    if (kc_sum > (uint64_t)INT_MAX && !fit) return SRF_ERR_UNSUPPORTED;
     const int64_t nseg = (int64_t)kc_sum;
+    if (fit && nseg > ONCE_SEGMENTS && n > 1) {
+        // a sixteenth less than in proportion: the parts of a list differ
+        *fit = std::max<int64_t>(1, (int64_t)((double)n * 0.9375 * (double)ONCE_SEGMENTS / (double)nseg));
+        return SRF_ERR_WORKSPACE;
+    }
     PB_TRY(ensure(P->recs, (size_t)nseg, s));
     PB_TRY(ensure(P->rec_ev, (size_t)nseg, s));
-    PB_TRY(ensure(P->partial, (size_t)nseg, s));
+    if (!fit) PB_TRY(ensure(P->partial, (size_t)nseg, s));
     // the records are built and sorted on the device while the host lays out the
     // work items below (the items come from the key counts alone)
     if (nseg > 0) {
@@ -1848,11 +1858,11 @@ int plan_build(srf_plan *P, const float *lors, int64_t n, int64_t lor_stride, co
 // left without work that uses P's buffers.
 int try_plan_build(srf_plan *P, const float *lors, int64_t n, int64_t lor_stride, const float *tof_values,
                    int64_t tof_stride, srf_grid_t grid, const srf_tof_t *tof, const srf_plan_opts_t *opts,
-                   hipStream_t s, bool &idle)
+                   hipStream_t s, int64_t *fit, bool &idle)
 {
     int rc;
     try {
-        rc = plan_build(P, lors, n, lor_stride, tof_values, tof_stride, grid, tof, opts, s);
+        rc = plan_build(P, lors, n, lor_stride, tof_values, tof_stride, grid, tof, opts, s, fit);
     } catch (...) {
         rc = SRF_ERR_LAUNCH;
     }
@@ -1884,7 +1894,7 @@ int srf_plan_create_ex(const float *lors, int64_t n, int64_t lor_stride, const f
     if (!P) return SRF_ERR_LAUNCH;
     bool idle;
     const int rc = try_plan_build(P, lors, n, lor_stride, tof_values, tof_stride, grid, tof, opts, (hipStream_t)stream,
-                                  idle);
+                                  nullptr, idle);
     if (rc) {
         plan_free(P);
         return rc;
@@ -1901,7 +1911,7 @@ int srf_plan_rebuild(srf_plan *plan, const float *lors, int64_t n, int64_t lor_s
     if (!plan) return SRF_ERR_INVALID_ARG;
     bool idle;
     const int rc = try_plan_build(plan, lors, n, lor_stride, tof_values, tof_stride, grid, tof, opts,
-                                  (hipStream_t)stream, idle);
+                                  (hipStream_t)stream, nullptr, idle);
     if (rc) {
         // plan_build committed nothing: the plan keeps its previous grid and
         // holds an empty list (projections write nothing, backprojections
@@ -2075,11 +2085,11 @@ namespace srf {
 // tile voxel instead of an atomic per term.
 int backproject_binned(const float *lors, int64_t n, int64_t lor_stride, const float *tof_values, int64_t tof_stride,
                        const float *values, const float *y, const float *p, int kind, float eps, srf_grid_t grid,
-                       const srf_tof_t *tof, srf_bp_mode_t mode, int accumulate, float *image, hipStream_t s)
+                       const srf_tof_t *tof, srf_bp_mode_t mode, int accumulate, float *image, hipStream_t s, int64_t &fit)
 {
     srf_plan P = {};
     bool idle;
-    int rc = try_plan_build(&P, lors, n, lor_stride, tof_values, tof_stride, grid, tof, nullptr, s, idle);
+    int rc = try_plan_build(&P, lors, n, lor_stride, tof_values, tof_stride, grid, tof, nullptr, s, &fit, idle);
     if (rc == SRF_OK) rc = plan_bp(&P, values, y, p, kind, eps, mode, accumulate, image, s, true);
     // (a build that succeeded has synchronised the stream: its scratch is idle)
     free_scratch(&P, s, idle, true);

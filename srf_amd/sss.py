@@ -171,9 +171,9 @@ class SingleScatterSimulation:
     """SSS sinogram of (emission, mu) images on a fixed geometry.
 
     compact=True (default) keeps only the scatter points with mu > 0 for each
-    call (the sum skips the others, so the sinogram is the same) and builds
-    the (detector, point) LORs for those; compact=False projects the full grid
-    and, with tiled=True, bins that fixed LOR set once into a projector plan.
+    call (the sum skips the others, so the sinogram is the same); compact=False
+    takes the full grid and, with tiled=True, bins its (detector, point) LORs
+    once into a projector plan, which line_integrals of the full grid then uses.
     rings: evaluate only the bins of these rings (their detectors only);
     the output is then (len(rings), n_angles, n_radial)."""
 
@@ -206,11 +206,11 @@ class SingleScatterSimulation:
                                                                      physical=physical_grid)
         self.ns = self.pts_xyz.shape[0]
         self.plan = None
-        if not self.compact:
+        if tiled and not self.compact:
             # p1 = detector, p2 = scatter point: the projector's segment cut ends the
             # integral at the point (siddon.cu.cc:56-57; preprocess.py:46-54 order)
             self.lors, self.to_integral = self._lors(self.pts_xyz)
-            self.plan = ops.Plan(self.lors, self.shape, self.geom, False) if tiled else None
+            self.plan = ops.Plan(self.lors, self.shape, self.geom, False)
         self.bins = torch.from_numpy(bins.astype(np.int32)).to(self.dev).contiguous()
         self.tables = torch.from_numpy(energy_tables(geometry.low_energy, geometry.high_energy,
                                                      geometry.resolution, physical_kn)).to(self.dev)

@@ -106,6 +106,13 @@ def _counter_means(csv_path, counter):
     return {k: sum(v) / len(v) for k, v in acc.items()}, first_copy
 
 
+def _step_value(means, kernel):
+    """The mean of the OSEM step's variant of a tiled kernel: TOF, cubic voxels (the sensitivity
+    image is backprojected without TOF).  None unless exactly one kernel name is that variant."""
+    vals = [v for k, v in means.items() if kernel + "<true, false, false>" in k]
+    return vals[0] if len(vals) == 1 else None
+
+
 def measure_traffic(args):
     """HBM bytes per launch of the tiled kernels, measured now: two child runs
     of this script (a 1 GiB device copy, then one OSEM step of the same
@@ -142,10 +149,9 @@ def measure_traffic(args):
             # the probe's copy (the process's first) moves TRAFFIC_COPY bytes each way
             factor = TRAFFIC_COPY / (copy * 1024.0)   # bytes moved per counted byte
             for part, kname in TRAFFIC_KERNELS.items():
-                # the step's variant comes last (the sensitivity image is backprojected by another)
-                vals = [v for k, v in means.items() if kname in k]
-                if vals:
-                    res.setdefault(part, {})[counter] = vals[-1] * 1024.0 * factor
+                value = _step_value(means, kname)
+                if value is not None:
+                    res.setdefault(part, {})[counter] = value * 1024.0 * factor
             res.setdefault("factor", {})[counter] = factor
     out = {part: d["FETCH_SIZE"] + d["WRITE_SIZE"] for part, d in res.items()
            if part != "factor" and "FETCH_SIZE" in d and "WRITE_SIZE" in d}

@@ -424,7 +424,8 @@ def plan_project_batch(handle: int, images_k: Tensor, n: int, shape: List[int]) 
     """Projections of B images at once (srf_plan_project_batch): (B, n)."""
     _req(images_k, "images")
     nx, ny, nz = (int(v) for v in shape)
-    if images_k.dim() != 4 or tuple(images_k.shape[1:]) != (nz, ny, nx):
+    # per image as _check_image: its number of voxels
+    if images_k.dim() != 4 or images_k[:1].numel() not in (0, nx * ny * nz):
         raise ValueError(f"images are {tuple(images_k.shape)}, grid says (B, {nz}, {ny}, {nx})")
     B = int(images_k.shape[0])
     out = torch.empty((B, n), dtype=torch.float32, device=images_k.device)

@@ -423,7 +423,7 @@ int srf_psf_xy(const float *x, int32_t nx, int32_t ny, int32_t nz, const float *
     if (!x || !weights || !out || half < 0 || half > 32 || (adjoint != 0 && adjoint != 1)) return SRF_ERR_INVALID_ARG;
     if (x == out || (d && d == out)) return SRF_ERR_INVALID_ARG;
     const int64_t n = (int64_t)nx * ny * nz;
-    if (half == PSF_H && n < (int64_t)1 << 31) {
+    if (half == PSF_H && n < (int64_t)1 << 31 && nz < 1 << 30) {   // 32-bit byte offsets in a column
         // two slices per lane where that leaves no more idle lanes than one, and
         // as many wavefronts along the slices as divide their chunks
         const int c1 = (nz + 63) / 64, zv = c1 % 2 == 0 ? 2 : 1, cz = c1 / zv;

@@ -82,7 +82,10 @@ int srf_version(void);
 /* Forward projection (Projection / ProjectionTof, siddon.cc:11-21,
  * siddon_tof.cc:11-24; host fn projection(), siddon.cu.cc:706-728 and
  * siddon_tof.cu.cc:761-785).  out[e] = sum_v image[v] * w_ev for every event;
- * events the reference skips get 0.  `out` is fully overwritten. */
+ * events the reference skips get 0.  `out` is fully overwritten.  The order of
+ * an event's sum, and so its last bits, depend on the list: its length picks 1 to
+ * 16 lanes an event, or (long lists, outside graph capture) bundles of
+ * neighbouring lines, in which 1 to 4 wavefronts share the sum. */
 int srf_project(const float *lors, int64_t n, int64_t lor_stride,
                 const float *tof_values, int64_t tof_stride,
                 const float *image, srf_grid_t grid, const srf_tof_t *tof,

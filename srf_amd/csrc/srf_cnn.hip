@@ -1378,7 +1378,6 @@ static int conv_launch(ConvIn in, const void *w, const float *bias, int32_t N, i
         else hipLaunchKernelGGL(k_conv_rows<1>, grid, dim3(256), lds, st, in, ws, d, T, o);
         return launch_status();
     }
-    // CONV_RULE
     int nbw = widest, kw = 1;
     auto blocks = [&] {
         const int cz = 4 / kw;

@@ -3,8 +3,9 @@ same events in short lists (float atomics), summed in float64; and the cutting o
 plan's records into work items.
 
 Non-negative values: a voxel of a short list gets at most a few hundred float
-additions per list, 500 half-ulps = 3e-5 of its sum; a binned term is resolved to 2^-50
-of its item's largest, below 1e-9 of the image's largest voxel."""
+additions per list, 500 half-ulps = 3e-5 of its sum; a plan's term is resolved to 2^-50
+of its item's largest, below 1e-9 of the image's largest voxel (a one-shot call's to
+float64: test_gpu_binned_range.py holds every voxel to its own sum)."""
 import numpy as np
 import pytest
 import torch

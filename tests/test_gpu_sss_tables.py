@@ -1,6 +1,7 @@
-"""The SSS kernels at the edges of their layouts: bins per workgroup (64), points per
-group (1, or 4 above 8192 detectors), points split over workgroups, an index outside
-the table, and the point line integrals over the copies and without them.
+"""The SSS kernels in the layout for bins in any order, at small and odd numbers of
+detectors, points (groups of 16) and bins, an index outside the table, and the point line
+integrals over the copies and without them.  (Both layouts at the edges of their groups,
+workgroups and lanes: test_gpu_sss_orders.py.)
 
 Bin sums against float64 with the whole-degree angle of each pair taken from the
 float32 cosine the path forms (unit vectors and three fused multiply-adds), so that no

@@ -122,8 +122,8 @@ def test_in_loop_model_on_held_out_osem_iterates():
 
 
 def test_ring_subset_sss_matches_full(setup):
-    """SSS on a few rings (4096 bins: one wavefront per bin) equals those rings
-    of the full SSS (131072 bins: one lane per bin) to float rounding."""
+    """SSS on a few rings (12288 bins, the points split over workgroups) equals those
+    rings of the full SSS (131072 bins) to float rounding."""
     import torch
     from srf_amd import phantom
     from srf_amd.sss import SingleScatterSimulation
